@@ -21,6 +21,9 @@ def _say(msg):
     # of the gauge field's two buffers before the second pass
     ((4, 4, 4), (0.05, 1.0, 1.0, 1.0), 16.0, 2, 4, None, False),
     ((3, 4, 5), (0.1, 1.0, 0.8, 1.2), 8.0, 1, 3, 5e-3, True),
+    # less than one block of 64 sites; a last block with 7 sites
+    ((2, 3, 2), (0.05, 1.0, 1.0, 1.0), 16.0, 2, 1, 1e-2, True),
+    ((5, 3, 9), (0.1, 1.0, 0.8, 1.2), 8.0, 1, 2, 2e-2, False),
 ])
 def test_equilibrium_init_matches_oracle(nrq, oracle, lattice, ext, sp, beta, nef, neq, tol, charge):
     _say(f"EquilibriumInit {ext} beta {beta} x{nef}, {neq} steps, tol {tol}, charge {charge}")
@@ -54,3 +57,13 @@ def test_equilibrium_init_rejects_bad_arguments(nrq, lattice):
         g.EquilibriumInit(-1.0, 1, 1)
     with pytest.raises(nrq.NRQError):
         g.EquilibriumInit(16.0, -1, 1)
+
+
+def test_equilibrium_init_without_a_sweep(nrq, lattice):
+    """A tolerance above the starting deviation: no projection, the field as drawn."""
+    lattice((5, 3, 9), (0.05, 1.0, 1.0, 1.0))
+    nrq.random_init(4)
+    g = nrq.GaugeConfiguration()
+    _, dev, nproj = g.EquilibriumInit(16.0, 1, 0, 1e6)
+    assert nproj[0] == 0 and 0 < dev[0] < 1e6
+    assert np.isclose(dev[0], g.GetGaussMax(), rtol=1e-12)
