@@ -28,12 +28,11 @@
 // gaps before), 69 us at 64^3 (54, 40 and 5 us); FP32 at 64^3 50 us (74 us).
 //
 // Sweeps run in batches without host synchronisation.  The maximum of the
-// state before sweep j lies in row j of a table of EQ_SLOTS slots (atomic
-// maxima of non-negative doubles, whose bit patterns order like integers); a
-// sweep that finds its row at or below the tolerance writes nothing, and so
+// state before sweep j lies in row j of a table (nrq_maxrow.h); a sweep that finds its row at or below the tolerance writes nothing, and so
 // leaves the next row at zero, which is below the tolerance too: exactly the
 // reference's number of sweeps changes E.
 #include "nrq_internal.h"
+#include "nrq_maxrow.h"
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -144,7 +143,6 @@ __device__ __forceinline__ void eq_projected(const mat3<double> &u, const mat3<d
 }
 
 constexpr int EQ_SITES = 64; // sites per block, one per lane
-constexpr int EQ_SLOTS = 64; // slots per row of the deviation table
 
 // One projection sweep (PROJ), or G and the deviation of the E field as it is
 // (PROJ = false: ef is read, ef_new and the old G are not used).  A block is
@@ -172,10 +170,7 @@ __global__ __launch_bounds__(6 * EQ_SITES) void k_eq_sweep(const cplx<R> *__rest
         // grid: the sweeps past the last leave here (2.2 us each at 16^3, 9 us
         // at 64^3; a look just before the stores, to hide its latency, saved
         // nothing measurable on a full sweep and cost these 5 and 69 us)
-        double seen = row[lane];
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) seen = fmax(seen, __shfl_xor(seen, off, 64));
-        if (seen <= tol) return;
+        if (row_max(row) <= tol) return;
     }
     double e[8];
     lsite p = {0, 0, 0, 0};
@@ -239,26 +234,21 @@ __global__ __launch_bounds__(6 * EQ_SITES) void k_eq_sweep(const cplx<R> *__rest
 #pragma unroll
         for (int a = 0; a < 8; ++a) dev = fmax(dev, fabs(tr[a]));
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) dev = fmax(dev, __shfl_xor(dev, off, 64));
-    // dev >= 0: its bits order like an unsigned integer
-    if (lane == 0)
-        atomicMax((unsigned long long *)row_new + blockIdx.x % EQ_SLOTS, (unsigned long long)__double_as_longlong(dev));
+    dev = lane_max(dev);
+    if (lane == 0) row_raise(row_new, dev);
 }
 
 // Zeroes rows [first, first + n) of the deviation table (n blocks).
-__global__ __launch_bounds__(EQ_SLOTS) void k_eq_clear(double *__restrict__ table, int first, int rows)
+__global__ __launch_bounds__(MAXROW) void k_eq_clear(double *__restrict__ table, int first, int rows)
 {
-    table[(int64_t)((first + (int)blockIdx.x) % rows) * EQ_SLOTS + threadIdx.x] = 0.0;
+    table[(int64_t)((first + (int)blockIdx.x) % rows) * MAXROW + threadIdx.x] = 0.0;
 }
 
 // out[b] = maximum of row first + b
-__global__ __launch_bounds__(EQ_SLOTS) void k_eq_rows(const double *__restrict__ table, int first, int rows,
+__global__ __launch_bounds__(MAXROW) void k_eq_rows(const double *__restrict__ table, int first, int rows,
                                                      double *__restrict__ out)
 {
-    double v = table[(int64_t)((first + (int)blockIdx.x) % rows) * EQ_SLOTS + threadIdx.x];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
+    const double v = row_max(table + (int64_t)((first + (int)blockIdx.x) % rows) * MAXROW);
     if (threadIdx.x == 0) out[blockIdx.x] = v;
 }
 
@@ -295,7 +285,7 @@ static int equilibrium_t(nrq_gauge *h, double beta, int64_t nefieldinit, int64_t
     const size_t ebytes = sizeof(R) * 24 * (size_t)V;
     if (hipMalloc((void **)&b.gm[0], sizeof(double) * 9 * (size_t)V) != hipSuccess ||
         hipMalloc((void **)&b.gm[1], sizeof(double) * 9 * (size_t)V) != hipSuccess ||
-        hipMalloc((void **)&b.table, sizeof(double) * EQ_ROWS * EQ_SLOTS) != hipSuccess ||
+        hipMalloc((void **)&b.table, sizeof(double) * EQ_ROWS * MAXROW) != hipSuccess ||
         hipMalloc((void **)&b.dev, sizeof(double) * 2 * EQ_BATCH) != hipSuccess || hipMalloc(&b.ealt, ebytes) != hipSuccess ||
         (rho_host && hipMalloc((void **)&b.rho, sizeof(double) * 3 * (size_t)V) != hipSuccess) ||
         hipHostMalloc((void **)&b.hdev, sizeof(double) * 2 * EQ_BATCH, hipHostMallocDefault) != hipSuccess) {
@@ -306,15 +296,15 @@ static int equilibrium_t(nrq_gauge *h, double beta, int64_t nefieldinit, int64_t
     if (rho_host) NRQ_HIP(hipMemcpyAsync(b.rho, rho_host, sizeof(double) * 3 * (size_t)V, hipMemcpyHostToDevice, stream()));
     if (int r = nrq_gauge_cold(h)) return r;
     R *ebuf[2] = {(R *)h->e, (R *)b.ealt};
-    auto row = [&](int64_t j) { return b.table + (j % EQ_ROWS) * EQ_SLOTS; };
+    auto row = [&](int64_t j) { return b.table + (j % EQ_ROWS) * MAXROW; };
     // G (buffer 0) and deviation of the configuration in h->e (row 0); the
     // links are looked up at every use, since the leapfrog swaps their buffers
     auto start = [&](double *dev) -> int {
-        hipLaunchKernelGGL(k_eq_clear, dim3(1), dim3(EQ_SLOTS), 0, stream(), b.table, 0, EQ_ROWS);
+        hipLaunchKernelGGL(k_eq_clear, dim3(1), dim3(MAXROW), 0, stream(), b.table, 0, EQ_ROWS);
         hipLaunchKernelGGL((k_eq_sweep<R, false>), dim3(nb), dim3(6 * EQ_SITES), 0, stream(), (const cplx<R> *)gauge_links(h),
                            (const R *)h->e, (const double *)nullptr, b.rho, g, 0.0, (R *)nullptr, b.gm[0], tol,
                            (const double *)nullptr, row(0));
-        hipLaunchKernelGGL(k_eq_rows, dim3(1), dim3(EQ_SLOTS), 0, stream(), b.table, 0, EQ_ROWS, b.dev);
+        hipLaunchKernelGGL(k_eq_rows, dim3(1), dim3(MAXROW), 0, stream(), b.table, 0, EQ_ROWS, b.dev);
         NRQ_HIP(hipGetLastError());
         NRQ_HIP(hipMemcpyAsync(b.hdev, b.dev, sizeof(double), hipMemcpyDeviceToHost, stream()));
         NRQ_HIP(hipStreamSynchronize(stream()));
@@ -347,7 +337,7 @@ static int equilibrium_t(nrq_gauge *h, double beta, int64_t nefieldinit, int64_t
         auto issue = [&]() -> int {
             const int64_t first = launched;
             const int half = (int)(first / EQ_BATCH & 1);
-            hipLaunchKernelGGL(k_eq_clear, dim3(EQ_BATCH), dim3(EQ_SLOTS), 0, stream(), b.table,
+            hipLaunchKernelGGL(k_eq_clear, dim3(EQ_BATCH), dim3(MAXROW), 0, stream(), b.table,
                                (int)((first + 1) % EQ_ROWS), EQ_ROWS);
             for (; launched < first + EQ_BATCH; ++launched) {
                 const int64_t j = launched;
@@ -355,7 +345,7 @@ static int equilibrium_t(nrq_gauge *h, double beta, int64_t nefieldinit, int64_t
                                    (const R *)ebuf[j & 1], (const double *)b.gm[j & 1], b.rho, g, EQ_KAPPA * a0,
                                    ebuf[(j + 1) & 1], b.gm[(j + 1) & 1], tol, (const double *)row(j), row(j + 1));
             }
-            hipLaunchKernelGGL(k_eq_rows, dim3(EQ_BATCH), dim3(EQ_SLOTS), 0, stream(), b.table,
+            hipLaunchKernelGGL(k_eq_rows, dim3(EQ_BATCH), dim3(MAXROW), 0, stream(), b.table,
                                (int)((first + 1) % EQ_ROWS), EQ_ROWS, b.dev + half * EQ_BATCH);
             NRQ_HIP(hipGetLastError());
             NRQ_HIP(hipMemcpyAsync(b.hdev + half * EQ_BATCH, b.dev + half * EQ_BATCH, sizeof(double) * EQ_BATCH,

@@ -35,6 +35,8 @@
 // eigen-decomposition in nrq_grouplog.h.
 #include "nrq_internal.h"
 #include "nrq_grouplog.h"
+#include "nrq_map.h"
+#include "nrq_maxrow.h"
 #include <hipfft/hipfft.h>
 #include <algorithm>
 #include <cmath>
@@ -86,13 +88,16 @@ __device__ __forceinline__ double lattice_momentum(const geom &g, int64_t s, cpl
 // gauge fixing
 // ---------------------------------------------------------------------------
 
-// -i Delta(x) into GF_PLANES complex planes; per-block max of ||Delta||_F / 9.
+// -i Delta(x) into GF_PLANES complex planes; the maximum of ||Delta||_F / 9
+// raises `row`.  Bound by its link reads; each XCD walks one contiguous eighth
+// of the lattice, so that U_i(x - i) is found in its L2 (with k_gf_apply in the
+// same order, 100 iterations at 64^3: 17.3 -> 15.8 ms).
 template <typename R>
 __global__ __launch_bounds__(GF_THREADS) void k_gf_divergence(const cplx<R> *__restrict__ u, geom g,
-                                                             cplx<double> *__restrict__ div, double *__restrict__ partial)
+                                                             cplx<double> *__restrict__ div, double *__restrict__ row)
 {
     __shared__ double sh[GF_THREADS / 64];
-    const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t s = (int64_t)xcd_block(gridDim.x, 8) * blockDim.x + threadIdx.x;
     double dev = 0;
     if (s < g.vol) {
         const lsite p = make_site(g, s);
@@ -124,32 +129,32 @@ __global__ __launch_bounds__(GF_THREADS) void k_gf_divergence(const cplx<R> *__r
         for (int e = 0; e < 9; ++e) f += d.m[e].re * d.m[e].re + d.m[e].im * d.m[e].im;
         dev = sqrt(f) / 9.0;
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) dev = fmax(dev, __shfl_down(dev, off, 64));
+    dev = lane_max(dev);
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = dev;
     __syncthreads();
     if (threadIdx.x == 0) {
         double m = 0;
         for (int k = 0; k < GF_THREADS / 64; ++k) m = fmax(m, sh[k]);
-        partial[blockIdx.x] = m;
+        row_raise(row, m);
     }
 }
 
-// max of n partials (one block)
-__global__ __launch_bounds__(GF_THREADS) void k_gf_fold_max(const double *__restrict__ partial, int64_t n,
-                                                           double *__restrict__ out)
+// The maximum of `row` to *out (pinned host memory); `next` starts at zero.
+__global__ __launch_bounds__(MAXROW) void k_gf_fold_max(const double *__restrict__ row, double *__restrict__ next,
+                                                       double *__restrict__ out)
 {
-    __shared__ double sh[GF_THREADS / 64];
-    double m = 0;
-    for (int64_t k = threadIdx.x; k < n; k += blockDim.x) m = fmax(m, partial[k]);
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_down(m, off, 64));
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = m;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int k = 0; k < GF_THREADS / 64; ++k) m = fmax(m, sh[k]);
-        *out = m;
-    }
+    const double m = row_max(row);
+    next[threadIdx.x] = 0.0;
+    if (threadIdx.x == 0) *out = m;
+}
+
+// Whether the transformation of the iteration whose divergence maximum is in
+// `row` is made: not once it is at or below the tolerance (or infinite, which
+// the host reports).
+__device__ __forceinline__ bool gf_goes_on(const double *__restrict__ row, double tol)
+{
+    const double m = row_max(row);
+    return m > tol && m < INFINITY;
 }
 
 // Momentum-space step: scale = fwd * bwd * alpha, times (p_max/|p|)^2 where |p| > tol.
@@ -201,12 +206,14 @@ __device__ __forceinline__ mat3<double> gf_group(const cplx<double> *__restrict_
 // U_i(x) <- g(x) U_i(x) g(x + i)^+ for the three directions at x, with
 // g = exp(Delta) formed here from Delta (gf_group) for x and its three
 // forward neighbours, so no separate pass writes g: the exponentials are
-// FP64 arithmetic inside a memory-bound kernel.
+// FP64 arithmetic inside a memory-bound kernel (46 us at 64^3 for 226 MB of
+// links).  Blocks in the order of k_gf_divergence.
 template <typename R>
 __global__ __launch_bounds__(GF_THREADS) void k_gf_apply(cplx<R> *__restrict__ u, const cplx<double> *__restrict__ delta,
-                                                         geom g)
+                                                         geom g, const double *__restrict__ row, double tol)
 {
-    const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (!gf_goes_on(row, tol)) return;
+    const int64_t s = (int64_t)xcd_block(gridDim.x, 8) * blockDim.x + threadIdx.x;
     if (s >= g.vol) return;
     const lsite p = make_site(g, s);
     const mat3<double> gx = gf_group(delta, g.vol, s);
@@ -352,13 +359,16 @@ static double max_momentum(const geom &g)
 // Device buffers of one call, freed on every exit path.
 struct gf_buffers {
     cplx<double> *fld = nullptr;
-    double *partial = nullptr, *dmax = nullptr, *hmax = nullptr;
+    double *partial = nullptr, *rows = nullptr, *hmax = nullptr;
+    hipEvent_t ev[2] = {nullptr, nullptr};
     ~gf_buffers()
     {
         if (fld) (void)hipFree(fld);
         if (partial) (void)hipFree(partial);
-        if (dmax) (void)hipFree(dmax);
+        if (rows) (void)hipFree(rows);
         if (hmax) (void)hipHostFree(hmax);
+        for (hipEvent_t e : ev)
+            if (e) (void)hipEventDestroy(e);
     }
 };
 
@@ -400,39 +410,57 @@ static int gaugefix_t(nrq_gauge *h, double tol, double alpha, int64_t maxit, int
     const unsigned nblk = (unsigned)((v + GF_THREADS - 1) / GF_THREADS);
     gf_buffers b;
     if (hipMalloc((void **)&b.fld, sizeof(cplx<double>) * GF_PLANES * (size_t)v) != hipSuccess ||
-        hipMalloc((void **)&b.partial, sizeof(double) * nblk) != hipSuccess ||
-        hipMalloc((void **)&b.dmax, sizeof(double)) != hipSuccess ||
-        hipHostMalloc((void **)&b.hmax, sizeof(double), hipHostMallocDefault) != hipSuccess) {
+        hipMalloc((void **)&b.rows, sizeof(double) * 3 * MAXROW) != hipSuccess ||
+        hipHostMalloc((void **)&b.hmax, sizeof(double) * 2, hipHostMallocDefault) != hipSuccess) {
         (void)hipGetLastError();
         return fail(NRQ_ERR_ALLOC, "gauge fixing: device allocation failed (V=%lld)", (long long)v);
     }
+    for (hipEvent_t &e : b.ev) NRQ_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     hipfftHandle plan = 0;
     if (int e = gf_plan(g, GF_PLANES, &plan)) return e;
     cplx<R> *u = (cplx<R> *)gauge_links_mut(h);
     const double fwd = g.a[1] * g.a[2] * g.a[3];
     const double bwd = 1.0 / ((double)g.n0 * g.a[1] * (double)g.n1 * g.a[2] * (double)g.n2 * g.a[3]);
     const double pmax = max_momentum(g);
-    int64_t done = 0;
+    // row n % 3 holds the divergence maximum before transformation n; the fold
+    // of row n clears that of n + 1, last read by transformation n - 2
+    auto row = [&](int64_t n) { return b.rows + (n % 3) * MAXROW; };
+    NRQ_HIP(hipMemsetAsync(b.rows, 0, sizeof(double) * 3 * MAXROW, stream()));
+    auto measure = [&](int64_t n) -> int {
+        hipLaunchKernelGGL(k_gf_divergence<R>, dim3(nblk), dim3(GF_THREADS), 0, stream(), u, g, b.fld, row(n));
+        hipLaunchKernelGGL(k_gf_fold_max, dim3(1), dim3(MAXROW), 0, stream(), row(n), row(n + 1), b.hmax + (n & 1));
+        NRQ_HIP(hipGetLastError());
+        NRQ_HIP(hipEventRecord(b.ev[n & 1], stream()));
+        return NRQ_OK;
+    };
+    // transformation n: made by k_gf_apply if the maximum before it asks for
+    // it.  The next one is enqueued before the host looks at this one's
+    // maximum, so the GPU never waits for the host; one transform pair too many
+    // runs at the end.
+    if (int e = measure(0)) return e;
+    int64_t enqueued = 0;
     double dev = 0;
-    for (;;) {
-        hipLaunchKernelGGL(k_gf_divergence<R>, dim3(nblk), dim3(GF_THREADS), 0, stream(), u, g, b.fld, b.partial);
-        hipLaunchKernelGGL(k_gf_fold_max, dim3(1), dim3(GF_THREADS), 0, stream(), b.partial, (int64_t)nblk, b.dmax);
-        NRQ_HIP(hipGetLastError());
-        NRQ_HIP(hipMemcpyAsync(b.hmax, b.dmax, sizeof(double), hipMemcpyDeviceToHost, stream()));
-        NRQ_HIP(hipStreamSynchronize(stream()));
-        dev = *b.hmax;
+    for (int64_t done = 0;; ++done) {
+        while (enqueued < maxit && enqueued <= done) {
+            const int64_t n = enqueued;
+            hipfftResult fr = hipfftExecZ2Z(plan, (hipfftDoubleComplex *)b.fld, (hipfftDoubleComplex *)b.fld, HIPFFT_FORWARD);
+            if (fr != HIPFFT_SUCCESS) return gf_fft_fail(fr, "exec (forward)");
+            hipLaunchKernelGGL(k_gf_accelerate, dim3(nblk), dim3(GF_THREADS), 0, stream(), b.fld, g, pmax, fwd * bwd * alpha);
+            fr = hipfftExecZ2Z(plan, (hipfftDoubleComplex *)b.fld, (hipfftDoubleComplex *)b.fld, HIPFFT_BACKWARD);
+            if (fr != HIPFFT_SUCCESS) return gf_fft_fail(fr, "exec (backward)");
+            hipLaunchKernelGGL(k_gf_apply<R>, dim3(nblk), dim3(GF_THREADS), 0, stream(), u, b.fld, g, row(n), tol);
+            // n + 1 uses the event and host slot of n - 1, which the host has read
+            if (int e = measure(n + 1)) return e;
+            ++enqueued;
+        }
+        NRQ_HIP(hipEventSynchronize(b.ev[done & 1]));
+        dev = *(volatile double *)(b.hmax + (done & 1));
         if (!std::isfinite(dev)) return fail(NRQ_ERR_NOCONV, "gauge fixing: non-finite divergence");
-        if (dev <= tol || done >= maxit) break;
-        hipfftResult fr = hipfftExecZ2Z(plan, (hipfftDoubleComplex *)b.fld, (hipfftDoubleComplex *)b.fld, HIPFFT_FORWARD);
-        if (fr != HIPFFT_SUCCESS) return gf_fft_fail(fr, "exec (forward)");
-        hipLaunchKernelGGL(k_gf_accelerate, dim3(nblk), dim3(GF_THREADS), 0, stream(), b.fld, g, pmax, fwd * bwd * alpha);
-        fr = hipfftExecZ2Z(plan, (hipfftDoubleComplex *)b.fld, (hipfftDoubleComplex *)b.fld, HIPFFT_BACKWARD);
-        if (fr != HIPFFT_SUCCESS) return gf_fft_fail(fr, "exec (backward)");
-        hipLaunchKernelGGL(k_gf_apply<R>, dim3(nblk), dim3(GF_THREADS), 0, stream(), u, b.fld, g);
-        NRQ_HIP(hipGetLastError());
-        ++done;
+        if (dev <= tol || done >= maxit) {
+            if (iterations) *iterations = done;
+            break;
+        }
     }
-    if (iterations) *iterations = done;
     if (final_dev) *final_dev = dev;
     return NRQ_OK;
 }
