@@ -40,7 +40,7 @@ namespace nrq {
 const void *gauge_links(const nrq_gauge *h);
 
 constexpr int CHEB_MAX = 64;  // Chebyshev steps per coefficient table
-constexpr int VBLOCKS = 256;  // blocks per slot in the vector kernels
+constexpr int VBLOCKS = 256;  // most blocks per slot in the vector kernels
 constexpr int VTHREADS = 256;
 constexpr int SBS = 256;      // threads per block in the stencil kernels (site-block maps)
 constexpr int SBS_WAVE = 512; // at most, with one work item per wavefront (wave-item map)
@@ -340,12 +340,14 @@ __global__ __launch_bounds__(SBS_WAVE, CN_WAVES) void k_cn_rhs(const cplx<RL> *_
     chunk_partials<NC>(nrm, r0, nf, t, mp.nsb, partial, mp.mode >= 3);
 }
 
-// FP64 true residual r_r = y_r - (1 + beta_r K) x_r, stored to res as type
-// TR when WRITE_RES; partial ||r_r||^2 per site block.
-template <int NC, typename RL, typename TR, bool WRITE_RES>
-__global__ __launch_bounds__(SBS_WAVE, CN_WAVES) void k_cn_resid(const cplx<RL> *__restrict__ u, slots<double> x, slots<double> y,
-                                                  slots<TR> res, const cplx<double> *__restrict__ beta, int nf, geom g,
-                                                  lf_map mp, double *__restrict__ partial)
+// True residual r_r = y_r - (1 + beta_r K) x_r in the arithmetic type T for the
+// active slots (all when active is null), stored to res as type TR when
+// WRITE_RES; partial ||r_r||^2 per site block.
+template <int NC, typename RL, typename T, typename TR, bool WRITE_RES>
+__global__ __launch_bounds__(SBS_WAVE, CN_WAVES) void k_cn_resid(const cplx<RL> *__restrict__ u, slots<T> x, slots<T> y,
+                                                  slots<TR> res, const cplx<double> *__restrict__ beta,
+                                                  const int *__restrict__ active, int nf, geom g, lf_map mp,
+                                                  double *__restrict__ partial)
 {
     lsite p = {0, 0, 0, 0};
     int64_t t = 0;
@@ -356,28 +358,28 @@ __global__ __launch_bounds__(SBS_WAVE, CN_WAVES) void k_cn_resid(const cplx<RL> 
     double nrm[NC] = {};
     bool on[NC];
     int rs[NC];
-    if (valid && chunk_slots<NC>(r0, nf, nullptr, on, rs)) {
-        ld_fields<NC, double, double> ld;
-        ld_fields<NC, double, double, true> ly;
+    if (valid && chunk_slots<NC>(r0, nf, active, on, rs)) {
+        ld_fields<NC, T, T> ld;
+        ld_fields<NC, T, T, true> ly;
 #pragma unroll
         for (int q = 0; q < NC; ++q) {
             ld.f[q] = x.p[rs[q]];
             ly.f[q] = y.p[rs[q]];
         }
-        cplx<double> hop[NC][3];
-        hop_chunk<NC, double>(u, ld, p, g, hop);
-        cplx<double> v0[NC][3], yv[NC][3];
-        own_chunk<NC, double>(ld, s, g.vol, v0);
-        own_chunk<NC, double>(ly, s, g.vol, yv);
-        const double dsum = g_dsum(g);
+        cplx<T> hop[NC][3];
+        hop_chunk<NC, T>(u, ld, p, g, hop);
+        cplx<T> v0[NC][3], yv[NC][3];
+        own_chunk<NC, T>(ld, s, g.vol, v0);
+        own_chunk<NC, T>(ly, s, g.vol, yv);
+        const T dsum = T(g_dsum(g));
 #pragma unroll
         for (int q = 0; q < NC; ++q) {
             if (!on[q]) continue;
             const int r = r0 + q;
-            const cplx<double> bt = beta[r];
+            const cplx<T> bt = to<T>(beta[r]);
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
-                const cplx<double> rr = yv[q][c] - (v0[q][c] + bt * (dsum * v0[q][c] - 0.5 * hop[q][c]));
+                const cplx<T> rr = yv[q][c] - (v0[q][c] + bt * (dsum * v0[q][c] - T(0.5) * hop[q][c]));
                 if (WRITE_RES) store_nt(at32(res.p[r] + (int64_t)c * g.vol, (uint32_t)s), cplx<TR>{(TR)rr.re, (TR)rr.im});
                 nrm[q] += nrm2(rr);
             }
@@ -467,15 +469,74 @@ __global__ __launch_bounds__(SBS_WAVE, CN_WAVES) void k_cheb(const cplx<RL> *__r
 // vector kernels (grid: VBLOCKS x slots)
 // ---------------------------------------------------------------------------
 
-// partial[r][i][blk] = this block's share of <V_i,r, w_r>, i < nv (FP64 sums).
+// Krylov basis of one GMRES cycle.  The vectors are kept as the orthogonal-
+// isation left them, W_i, with their scale factors 1 / ||W_i|| beside them
+// (gm_state::sc): the unit vectors are v_i = sc_i W_i, and no pass over memory
+// normalises them (at 64^3 with 12 columns that pass took 45 us of the 455 us
+// of an iteration).  W_0, the residual the cycle starts from, stays where it
+// is.
+template <typename T> struct gm_basis {
+    const cplx<T> *w0; // W_0, slot-major
+    cplx<T> *w;        // W_i, i >= 1, at w + i * nf * n
+    __device__ __host__ __forceinline__ const cplx<T> *at(int i, int r, int nf, int64_t n) const
+    {
+        return i == 0 ? w0 + (int64_t)r * n : w + ((int64_t)i * nf + r) * n;
+    }
+};
+
+// Per-slot GMRES scalars on the device (allocated for restart m): the
+// Hessenberg columns and rotations live where the sums are made, so that a
+// step's kernels follow each other without the host.
+struct gm_state {
+    cplx<double> *H;    // [slot][column j][row i], (m + 1) x m per slot, rotated in place
+    cplx<double> *sn;   // [slot][m] rotations
+    cplx<double> *g;    // [slot][m + 1] rotated right-hand side
+    cplx<double> *coef; // [slot][m + 1] coefficients of the next combination of W_i
+    double *cs;         // [slot][m]
+    double *sc;         // [slot][m + 1] 1 / ||W_i||
+    double *stop;       // [slot] |g_{j+1}| at or below this ends the slot's cycle
+    int *left;          // [slot] steps the iteration cap still allows
+    int *used;          // [slot] columns of the cycle
+    int *fallen;        // [slot] the network's direction was not finite
+    int *cyc;           // [slot] the slot's cycle goes on
+    int *act;           // [slot] the slot is part of this cycle
+    int m;
+};
+
+// What the host gives a cycle, passed by value.
+struct gm_start {
+    double rn[NSLOTS], stop[NSLOTS];
+    int left[NSLOTS];
+    unsigned long long act;
+};
+
+__global__ __launch_bounds__(64) void k_gm_begin(gm_state st, gm_start in)
+{
+    const int r = threadIdx.x;
+    if (r >= NSLOTS) return;
+    const int on = (int)(in.act >> r & 1ull);
+    st.cyc[r] = st.act[r] = on;
+    st.used[r] = st.fallen[r] = 0;
+    st.stop[r] = in.stop[r];
+    st.left[r] = in.left[r];
+    st.g[(int64_t)r * (st.m + 1)] = {in.rn[r], 0.0};
+    st.sc[(int64_t)r * (st.m + 1)] = in.rn[r] > 0 ? 1.0 / in.rn[r] : 0.0;
+}
+
+// active[r] = bit r of mask
+__global__ __launch_bounds__(64) void k_set_mask(int *__restrict__ active, unsigned long long mask)
+{
+    if (threadIdx.x < NSLOTS) active[threadIdx.x] = (int)(mask >> threadIdx.x & 1ull);
+}
+
+// partial[r][i][blk] = this block's share of <W_i,r, w_r>, i < nv (FP64 sums).
 // The basis vectors go in groups of MDOT_G, each group in one pass that reads
 // w_r once (PETSc's VecMDot); per thread and per block the sums run in the
 // same order for every grouping.
 constexpr int MDOT_G = 8;
 template <typename T>
-__global__ __launch_bounds__(VTHREADS) void k_mdot(const cplx<T> *__restrict__ basis, int nv, const cplx<T> *__restrict__ w,
-                                                   int64_t n, int nf, const int *__restrict__ active,
-                                                   cplx<double> *__restrict__ partial)
+__global__ __launch_bounds__(VTHREADS) void k_mdot(gm_basis<T> basis, int nv, const cplx<T> *__restrict__ w, int64_t n, int nf,
+                                                   const int *__restrict__ active, cplx<double> *__restrict__ partial)
 {
     const int r = blockIdx.y;
     if (!active[r]) return;
@@ -485,16 +546,20 @@ __global__ __launch_bounds__(VTHREADS) void k_mdot(const cplx<T> *__restrict__ b
     for (int i0 = 0; i0 < nv; i0 += MDOT_G) {
         const int gn = nv - i0 < MDOT_G ? nv - i0 : MDOT_G;
         double re[MDOT_G], im[MDOT_G];
+        const cplx<T> *b[MDOT_G];
 #pragma unroll
-        for (int j = 0; j < MDOT_G; ++j) re[j] = im[j] = 0;
+        for (int j = 0; j < MDOT_G; ++j) {
+            re[j] = im[j] = 0;
+            b[j] = basis.at(j < gn ? i0 + j : i0, r, nf, n);
+        }
         for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (int64_t)gridDim.x * blockDim.x) {
-            const cplx<T> b = wr[k];
+            const cplx<T> x = wr[k];
 #pragma unroll
             for (int j = 0; j < MDOT_G; ++j) {
                 if (j >= gn) break;
-                const cplx<T> a = basis[((int64_t)(i0 + j) * nf + r) * n + k];
-                re[j] += (double)a.re * b.re + (double)a.im * b.im;
-                im[j] += (double)a.re * b.im - (double)a.im * b.re;
+                const cplx<T> a = b[j][k];
+                re[j] += (double)a.re * x.re + (double)a.im * x.im;
+                im[j] += (double)a.re * x.im - (double)a.im * x.re;
             }
         }
         __syncthreads(); // sh is free (previous group read)
@@ -517,15 +582,16 @@ __global__ __launch_bounds__(VTHREADS) void k_mdot(const cplx<T> *__restrict__ b
     }
 }
 
-// out[t] = sum over the nblk block partials of t = r * count + i, one
-// wavefront per t (lane l sums partials l, l + 64, ..., then the wavefront
-// sum): a fixed order, and 64 loads in flight instead of one.
-__global__ __launch_bounds__(256) void k_fold_c(const cplx<double> *__restrict__ partial, int nblk, int count, int nf,
-                                                const int *__restrict__ active, cplx<double> *__restrict__ out)
+// h_i = <v_i, A v_j> of step j from the partials of <W_i, A W_j>, one wavefront
+// per (slot, i) (lane l sums partials l, l + 64, ..., then the wavefront sum: a
+// fixed order, and 64 loads in flight instead of one); and the coefficient
+// sc_i h_i with which W_i enters the Gram-Schmidt update.
+__global__ __launch_bounds__(256) void k_gm_dots(const cplx<double> *__restrict__ partial, int nblk, int nv, int nf, gm_state st)
 {
     const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (t >= count * nf) return;
-    if (!active[t / count]) return;
+    if (t >= nv * nf) return;
+    const int r = t / nv, i = t - r * nv;
+    if (!st.cyc[r]) return;
     double re = 0, im = 0;
     for (int b = lane; b < nblk; b += 64) {
         const cplx<double> v = partial[(int64_t)t * nblk + b];
@@ -534,16 +600,24 @@ __global__ __launch_bounds__(256) void k_fold_c(const cplx<double> *__restrict__
     }
     re = wsum(re);
     im = wsum(im);
-    if (lane == 0) out[t] = {re, im};
+    if (lane == 0) {
+        const double *sc = st.sc + (int64_t)r * (st.m + 1);
+        const double f = sc[i] * sc[nv - 1];
+        const cplx<double> h = {f * re, f * im};
+        st.H[((int64_t)r * st.m + nv - 1) * (st.m + 1) + i] = h;
+        st.coef[(int64_t)r * (st.m + 1) + i] = sc[i] * h;
+    }
 }
 
 // out[r] = sum_b partial[r * nblk + b] for the slot r = blockIdx.x if
 // active[r] (active may be null); fixed summation order.  FOLD_THREADS
 // threads with four independent sums each keep enough loads in flight for
-// the V / 64 partials of the wave-item map.
+// the V / 64 partials of the wave-item map.  host (pinned, may be null)
+// receives the sums as well.
 constexpr int FOLD_THREADS = 1024;
 __global__ __launch_bounds__(FOLD_THREADS) void k_fold_slots(const double *__restrict__ partial, int64_t nblk,
-                                                             const int *__restrict__ active, double *__restrict__ out)
+                                                             const int *__restrict__ active, double *__restrict__ out,
+                                                             double *__restrict__ host)
 {
     const int r = blockIdx.x;
     if (active && !active[r]) return;
@@ -558,85 +632,153 @@ __global__ __launch_bounds__(FOLD_THREADS) void k_fold_slots(const double *__res
         if (b + 3 * FOLD_THREADS < nblk) s3 += p[b + 3 * FOLD_THREADS];
     }
     double s = block_sum((s0 + s1) + (s2 + s3), sh);
-    if (threadIdx.x == 0) out[r] = s;
+    if (threadIdx.x == 0) {
+        out[r] = s;
+        if (host) host[r] = s;
+    }
 }
 
-// CGS update w_r -= sum_i h[r][i] V_i,r and partial ||w_r||^2
+// Gram-Schmidt update W_nv = sc_j (A W_j) - sum_{i < nv} coef_i W_i (j = nv - 1,
+// A W_j in w, in place) and partial ||W_nv||^2
 template <typename T>
-__global__ __launch_bounds__(VTHREADS) void k_cgs_update(const cplx<T> *__restrict__ basis, int nv, cplx<T> *__restrict__ w,
-                                                         int64_t n, int nf, const int *__restrict__ active,
-                                                         const cplx<double> *__restrict__ h, double *__restrict__ partial)
+__global__ __launch_bounds__(VTHREADS) void k_cgs_update(gm_basis<T> basis, int nv, cplx<T> *__restrict__ w, int64_t n, int nf,
+                                                         gm_state st, double *__restrict__ partial)
 {
     const int r = blockIdx.y;
-    if (!active[r]) return;
+    if (!st.cyc[r]) return;
     __shared__ double sh[8];
     cplx<T> *wr = w + (int64_t)r * n;
+    const double scj = st.sc[(int64_t)r * (st.m + 1) + nv - 1];
+    const cplx<double> *h = st.coef + (int64_t)r * (st.m + 1);
     double nrm = 0;
     for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (int64_t)gridDim.x * blockDim.x) {
         const cplx<T> w0 = wr[k];
-        cplx<double> a = {(double)w0.re, (double)w0.im};
+        cplx<double> a = {scj * (double)w0.re, scj * (double)w0.im};
         for (int i = 0; i < nv; ++i) {
-            const cplx<T> v = basis[((int64_t)i * nf + r) * n + k];
-            a = a - h[(int64_t)r * nv + i] * cplx<double>{(double)v.re, (double)v.im};
+            const cplx<T> v = basis.at(i, r, nf, n)[k];
+            a = a - h[i] * cplx<double>{(double)v.re, (double)v.im};
         }
-        const cplx<T> st = {(T)a.re, (T)a.im};
-        wr[k] = st;
-        nrm += nrm2(st);
+        const cplx<T> o = {(T)a.re, (T)a.im};
+        wr[k] = o;
+        nrm += nrm2(o);
     }
     nrm = block_sum(nrm, sh);
     if (threadIdx.x == 0) partial[(int64_t)r * gridDim.x + blockIdx.x] = nrm;
 }
 
-// dst_r = src_r / sqrt(nrm2[r]) (zero norm leaves zeros)
-template <typename T>
-__global__ void k_scale(const cplx<T> *__restrict__ src, cplx<T> *__restrict__ dst, int64_t n,
-                        const double *__restrict__ nrm2v, const int *__restrict__ active)
+// End of Arnoldi step j of slot r = blockIdx.x: ||W_{j+1}|| from its partials,
+// the Givens rotation of column j and the residual estimate; the slot's cycle
+// ends at `stop`, at its iteration cap, or (net) when a coefficient is not
+// finite, which leaves the columns before j.  Whether it goes on is also
+// written to *host_cyc (pinned).
+__global__ __launch_bounds__(VTHREADS) void k_gm_step(const double *__restrict__ partial, int nblk, int j, int net, gm_state st,
+                                                      int *__restrict__ host_cyc)
 {
-    const int r = blockIdx.y;
-    if (!active[r]) return;
-    const double nn = nrm2v[r];
-    const T inv = (T)(nn > 0 ? 1.0 / sqrt(nn) : 0.0);
-    for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (int64_t)gridDim.x * blockDim.x)
-        dst[(int64_t)r * n + k] = inv * src[(int64_t)r * n + k];
-}
-
-// x_r += sum_i y[r][i] V_i,r
-template <typename T>
-__global__ void k_xupdate(cplx<T> *__restrict__ x, const cplx<T> *__restrict__ basis, int nf, int64_t n,
-                          const cplx<double> *__restrict__ y, int ystride, const int *__restrict__ nused,
-                          const int *__restrict__ active)
-{
-    const int r = blockIdx.y;
-    if (!active[r]) return;
-    const int nv = nused[r];
-    for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (int64_t)gridDim.x * blockDim.x) {
-        const cplx<T> x0 = x[(int64_t)r * n + k];
-        cplx<double> a = {(double)x0.re, (double)x0.im};
-        for (int i = 0; i < nv; ++i) {
-            const cplx<T> v = basis[((int64_t)i * nf + r) * n + k];
-            a = a + y[(int64_t)r * ystride + i] * cplx<double>{(double)v.re, (double)v.im};
+    const int r = blockIdx.x;
+    if (!st.cyc[r]) {
+        if (threadIdx.x == 0) host_cyc[r] = 0;
+        return;
+    }
+    __shared__ double sh[VTHREADS / 64];
+    double v = 0;
+    for (int b = threadIdx.x; b < nblk; b += blockDim.x) v += partial[(int64_t)r * nblk + b];
+    v = block_sum(v, sh);
+    if (threadIdx.x != 0) return;
+    const int m = st.m;
+    cplx<double> *H = st.H + ((int64_t)r * m + j) * (m + 1), *g = st.g + (int64_t)r * (m + 1), *sn = st.sn + (int64_t)r * m;
+    double *cs = st.cs + (int64_t)r * m;
+    if (net) {
+        bool fin = isfinite(v);
+        for (int i = 0; i <= j; ++i) fin = fin && isfinite(H[i].re) && isfinite(H[i].im);
+        if (!fin) {
+            st.cyc[r] = 0;
+            st.fallen[r] = 1;
+            host_cyc[r] = 0;
+            return;
         }
-        x[(int64_t)r * n + k] = {(T)a.re, (T)a.im};
     }
+    const double hn = sqrt(fmax(v, 0.0));
+    st.sc[(int64_t)r * (m + 1) + j + 1] = hn > 0 ? 1.0 / hn : 0.0;
+    cplx<double> a = H[0];
+    for (int i = 0; i < j; ++i) {
+        const cplx<double> c = H[i + 1];
+        H[i] = cs[i] * a + sn[i] * c;
+        a = cs[i] * c - cmul(sn[i], a); // -conj(sn) a + cs c
+    }
+    const double na = sqrt(a.re * a.re + a.im * a.im), den = sqrt(a.re * a.re + a.im * a.im + hn * hn);
+    double c = 1;
+    cplx<double> sj = {0.0, 0.0};
+    if (den > 0) {
+        c = na / den;
+        sj = na > 0 ? (hn / den / na) * a : cplx<double>{1.0, 0.0};
+    }
+    cs[j] = c;
+    sn[j] = sj;
+    H[j] = c * a + hn * sj;
+    const cplx<double> gj = g[j];
+    const cplx<double> gn = cmul(sj, gj);
+    g[j + 1] = {-gn.re, -gn.im};
+    g[j] = c * gj;
+    st.used[r] = j + 1;
+    const bool end = sqrt(gn.re * gn.re + gn.im * gn.im) <= st.stop[r] || j + 1 >= st.left[r];
+    if (end) st.cyc[r] = 0;
+    host_cyc[r] = end ? 0 : 1;
 }
 
-// res_r = b_r - t_r and partial ||res_r||^2
+// End of a cycle: back substitution H y = g of slot r = blockIdx.x, with the
+// scale factors of the basis folded into coef; used and fallen go to the
+// pinned host arrays.  A solution that is not finite (net) keeps x (used = 0
+// in *st.used, with fallen set).
+__global__ __launch_bounds__(64) void k_gm_solve(gm_state st, int net, int *__restrict__ host_used, int *__restrict__ host_fallen)
+{
+    const int r = blockIdx.x;
+    if (threadIdx.x != 0) return;
+    const int m = st.m, n = st.act[r] ? st.used[r] : 0;
+    cplx<double> *y = st.coef + (int64_t)r * (m + 1);
+    const cplx<double> *g = st.g + (int64_t)r * (m + 1);
+    const double *sc = st.sc + (int64_t)r * (m + 1);
+    host_used[r] = n;
+    bool fin = true;
+    for (int i = n - 1; i >= 0; --i) {
+        cplx<double> s = g[i];
+        for (int k = i + 1; k < n; ++k) s = s - st.H[((int64_t)r * m + k) * (m + 1) + i] * y[k];
+        const cplx<double> d = st.H[((int64_t)r * m + i) * (m + 1) + i];
+        // s / d with d scaled by its larger part first
+        const double big = fmax(fabs(d.re), fabs(d.im));
+        const cplx<double> q = {d.re / big, d.im / big};
+        const double q2 = (q.re * q.re + q.im * q.im) * big;
+        const cplx<double> t = cmul(q, s);
+        y[i] = {t.re / q2, t.im / q2};
+        fin = fin && isfinite(y[i].re) && isfinite(y[i].im);
+    }
+    for (int i = 0; i < n; ++i) y[i] = sc[i] * y[i];
+    if (net && !fin) st.fallen[r] = 1;
+    st.used[r] = net && !fin ? 0 : n;
+    host_fallen[r] = st.fallen[r];
+}
+
+// x_r = (zero ? 0 : x_r) + sum_{i < used_r} coef_i V_i,r with V the basis (or
+// the preconditioned directions).  Slots without columns keep x, or get 0.
 template <typename T>
-__global__ __launch_bounds__(VTHREADS) void k_residual(const cplx<T> *__restrict__ b, const cplx<T> *__restrict__ t,
-                                                       cplx<T> *__restrict__ res, int64_t n, const int *__restrict__ active,
-                                                       double *__restrict__ partial)
+__global__ __launch_bounds__(VTHREADS) void k_xupdate(slots<T> x, gm_basis<T> basis, int nf, int64_t n, gm_state st, int zero)
 {
     const int r = blockIdx.y;
-    if (!active[r]) return;
-    __shared__ double sh[8];
-    double nrm = 0;
+    const int nv = st.used[r];
+    if (nv == 0 && !zero) return;
+    cplx<T> *xr = x.p[r];
+    const cplx<double> *y = st.coef + (int64_t)r * (st.m + 1);
     for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (int64_t)gridDim.x * blockDim.x) {
-        const cplx<T> a = b[(int64_t)r * n + k] - t[(int64_t)r * n + k];
-        res[(int64_t)r * n + k] = a;
-        nrm += nrm2(a);
+        cplx<double> a = {0.0, 0.0};
+        if (!zero) {
+            const cplx<T> x0 = xr[k];
+            a = {(double)x0.re, (double)x0.im};
+        }
+        for (int i = 0; i < nv; ++i) {
+            const cplx<T> v = basis.at(i, r, nf, n)[k];
+            a = a + y[i] * cplx<double>{(double)v.re, (double)v.im};
+        }
+        xr[k] = {(T)a.re, (T)a.im};
     }
-    nrm = block_sum(nrm, sh);
-    if (threadIdx.x == 0) partial[(int64_t)r * gridDim.x + blockIdx.x] = nrm;
 }
 
 template <typename T>
@@ -712,29 +854,36 @@ struct workspace {
     cplx<double> *y = nullptr, *x = nullptr, *t = nullptr, *res = nullptr;
     cplx<float> *y32 = nullptr, *x32 = nullptr, *t32 = nullptr, *res32 = nullptr;
     cplx<float> *links32 = nullptr;    // FP32 copy of the links for the inner solves
-    cplx<double> *beta = nullptr, *cpar = nullptr, *hdev = nullptr, *ydev = nullptr, *cpart = nullptr;
+    cplx<double> *beta = nullptr, *cpar = nullptr, *cpart = nullptr;
+    gm_state gm = {};                  // GMRES scalars, in the buffers gmz, gmd, gmi
+    cplx<double> *gmz = nullptr;
+    double *gmd = nullptr;
+    int *gmi = nullptr;
     cplx<double> *negone = nullptr;    // -1 per slot: k_stencil with it as gco gives beta K in
     cplx<double> *cheb = nullptr;      // Chebyshev coefficients [iteration][slot][2]
     double *rpart = nullptr, *spart = nullptr, *nrm = nullptr;
-    int *active = nullptr, *nused = nullptr;
+    int *active = nullptr;
     cplx<double> *fptr[NSLOTS] = {};   // heavy field of each slot in the current CN step
     cplx<double> *zbasis = nullptr;    // FGMRES: preconditioned directions, m x rcap x 3V
     int zm = 0;
-    cplx<double> *hbuf = nullptr;      // pinned host
+    int *ibuf = nullptr;               // pinned host, NSLOTS each: cycle flags of even and odd steps, used, fallen
     double *nbuf = nullptr;            // pinned host (NRM doubles)
+    hipEvent_t ev[2] = {nullptr, nullptr}; // end of even and odd GMRES steps
 
-    // nrm layout, NSLOTS each: working norms, ||y||^2, saved refinement
-    // ||r||^2, GMRES restart norms
-    static constexpr int NRM_Y = NSLOTS, NRM_SAVED = 2 * NSLOTS, NRM_RESTART = 3 * NSLOTS, NRM = 4 * NSLOTS;
+    // layout of nrm and nbuf, NSLOTS each: working norms, ||y||^2, saved refinement ||r||^2
+    static constexpr int NRM_Y = NSLOTS, NRM_SAVED = 2 * NSLOTS, NRM = 3 * NSLOTS;
+    static constexpr int I_USED = 2 * NSLOTS, I_FALLEN = 3 * NSLOTS, I_ALL = 4 * NSLOTS;
 
     void release()
     {
-        void *dev[] = {basis, y, x, t, res, y32, x32, t32, res32, links32, beta, cpar, hdev, ydev, cpart,
-                       rpart, spart, nrm, active, nused, cheb, negone};
+        void *dev[] = {basis, y, x, t, res, y32, x32, t32, res32, links32, beta, cpar, gmz, gmd, gmi, cpart,
+                       rpart, spart, nrm, active, cheb, negone};
         for (void *q : dev)
             if (q) (void)hipFree(q);
-        if (hbuf) (void)hipHostFree(hbuf);
+        if (ibuf) (void)hipHostFree(ibuf);
         if (nbuf) (void)hipHostFree(nbuf);
+        for (hipEvent_t e : ev)
+            if (e) (void)hipEventDestroy(e);
         if (zbasis) (void)hipFree(zbasis);
         *this = workspace();
     }
@@ -762,14 +911,17 @@ struct workspace {
                   dm((void **)&beta, sizeof(cplx<double>) * NSLOTS) && dm((void **)&cpar, sizeof(cplx<double>) * 2 * NSLOTS) &&
                   dm((void **)&negone, sizeof(cplx<double>) * NSLOTS) &&
                   dm((void **)&cheb, sizeof(cplx<double>) * 2 * NSLOTS * CHEB_MAX) &&
-                  dm((void **)&hdev, sizeof(cplx<double>) * NSLOTS * (mm + 1)) &&
-                  dm((void **)&ydev, sizeof(cplx<double>) * NSLOTS * (mm + 1)) &&
+                  dm((void **)&gmz, sizeof(cplx<double>) * NSLOTS * ((size_t)(mm + 1) * mm + mm + 2 * (mm + 1))) &&
+                  dm((void **)&gmd, sizeof(double) * NSLOTS * (mm + (mm + 1) + 1)) &&
+                  dm((void **)&gmi, sizeof(int) * NSLOTS * 5) &&
                   dm((void **)&cpart, sizeof(cplx<double>) * NSLOTS * (mm + 1) * VBLOCKS) &&
                   dm((void **)&rpart, sizeof(double) * std::max(KRYLOV_REDUCE_DOUBLES, (size_t)NSLOTS * VBLOCKS * 8)) &&
                   dm((void **)&spart, sizeof(double) * NSLOTS * (size_t)sb) && dm((void **)&nrm, sizeof(double) * NRM) &&
-                  dm((void **)&active, sizeof(int) * NSLOTS) && dm((void **)&nused, sizeof(int) * NSLOTS) &&
-                  hipHostMalloc((void **)&hbuf, sizeof(cplx<double>) * NSLOTS * (mm + 1), hipHostMallocDefault) == hipSuccess &&
-                  hipHostMalloc((void **)&nbuf, sizeof(double) * NRM, hipHostMallocDefault) == hipSuccess;
+                  dm((void **)&active, sizeof(int) * NSLOTS) &&
+                  hipHostMalloc((void **)&ibuf, sizeof(int) * I_ALL, hipHostMallocDefault) == hipSuccess &&
+                  hipHostMalloc((void **)&nbuf, sizeof(double) * NRM, hipHostMallocDefault) == hipSuccess &&
+                  hipEventCreateWithFlags(&ev[0], hipEventDisableTiming) == hipSuccess &&
+                  hipEventCreateWithFlags(&ev[1], hipEventDisableTiming) == hipSuccess;
         if (!ok) {
             (void)hipGetLastError();
             release();
@@ -783,6 +935,20 @@ struct workspace {
                 return fail(NRQ_ERR_HIP, "CN: workspace initialisation failed");
             }
         }
+        const size_t nh = (size_t)NSLOTS * (mm + 1) * mm;
+        gm.m = mm;
+        gm.H = gmz;
+        gm.sn = gmz + nh;
+        gm.g = gm.sn + (size_t)NSLOTS * mm;
+        gm.coef = gm.g + (size_t)NSLOTS * (mm + 1);
+        gm.cs = gmd;
+        gm.sc = gm.cs + (size_t)NSLOTS * mm;
+        gm.stop = gm.sc + (size_t)NSLOTS * (mm + 1);
+        gm.left = gmi;
+        gm.used = gmi + NSLOTS;
+        gm.fallen = gmi + 2 * NSLOTS;
+        gm.cyc = gmi + 3 * NSLOTS;
+        gm.act = gmi + 4 * NSLOTS;
         vol = v;
         m = mm;
         rcap = rc;
@@ -815,12 +981,31 @@ void krylov_release() { g_ws.release(); }
 double *krylov_reduce_scratch() { return g_ws.rpart; }
 double *krylov_host_scratch() { return g_ws.nbuf; }
 
-static int upload_ints(int *dev, const std::vector<int> &v)
+// The slots with act[r] != 0 as a bit mask.
+static unsigned long long mask_of(const std::vector<int> &act)
 {
-    NRQ_HIP(hipMemcpyAsync(dev, v.data(), sizeof(int) * v.size(), hipMemcpyHostToDevice, stream()));
+    unsigned long long b = 0;
+    for (size_t r = 0; r < act.size(); ++r) b |= (unsigned long long)(act[r] != 0) << r;
+    return b;
+}
+
+// Slot mask of the next launches (a kernel argument: a copy from pageable host
+// memory would hold the queue and the host for longer).
+static int upload_active(const std::vector<int> &act)
+{
+    hipLaunchKernelGGL(k_set_mask, dim3(1), dim3(64), 0, stream(), g_ws.active, mask_of(act));
+    NRQ_HIP(hipGetLastError());
     return NRQ_OK;
 }
-static int upload_active(const std::vector<int> &act) { return upload_ints(g_ws.active, act); }
+
+// Blocks per slot of the vector kernels: four elements per thread up to
+// VBLOCKS blocks.  Fewer elements per thread cost more in partial sums than
+// they gain (16^3, 12 columns: k_mdot with 256 blocks of 48 elements took
+// 29 us, with 12 blocks of 1,024 7 us).
+static unsigned vblocks(int64_t n)
+{
+    return (unsigned)std::min<int64_t>(VBLOCKS, std::max<int64_t>(1, (n + 4 * VTHREADS - 1) / (4 * VTHREADS)));
+}
 
 // Launch shape of the stencil kernels: slots per thread (NC, sharing each
 // link load) for FP64 and for FP32 arithmetic, and the site-block mapping of
@@ -896,18 +1081,18 @@ static slots<double> psi_slots(int R)
     return t;
 }
 
-// out[r] = sum of the nblk partials of slot r (r < nf; active may be null)
-static int fold_slots(const double *partial, int64_t nblk, int nf, const int *active, double *out)
+// out[r] = sum of the nblk partials of slot r (r < nf; active may be null),
+// also to the pinned host (may be null)
+static int fold_slots(const double *partial, int64_t nblk, int nf, const int *active, double *out, double *host)
 {
-    hipLaunchKernelGGL(k_fold_slots, dim3(nf), dim3(FOLD_THREADS), 0, stream(), partial, nblk, active, out);
+    hipLaunchKernelGGL(k_fold_slots, dim3(nf), dim3(FOLD_THREADS), 0, stream(), partial, nblk, active, out, host);
     NRQ_HIP(hipGetLastError());
     return NRQ_OK;
 }
 
-// g_ws.nrm to the pinned host buffer g_ws.nbuf; waits for the stream
-static int nrm_to_host()
+// Waits for the stream: the sums folded so far are in g_ws.nbuf.
+static int wait_sums()
 {
-    NRQ_HIP(hipMemcpyAsync(g_ws.nbuf, g_ws.nrm, sizeof(double) * workspace::NRM, hipMemcpyDeviceToHost, stream()));
     NRQ_HIP(hipStreamSynchronize(stream()));
     return NRQ_OK;
 }
@@ -915,12 +1100,12 @@ static int nrm_to_host()
 // out_r = in_r + beta_r K in_r for the active slots
 template <typename RL, typename T>
 static void launch_stencil(const cplx<RL> *u, const slots<T> &in, const slots<T> &out, int nf,
-                           const cplx<double> *gco = nullptr)
+                           const int *active, const cplx<double> *gco = nullptr)
 {
     const int nc = nc_of<T>();
     const lf_map mp = cn_map(nf, nc);
     NC_DISPATCH(nc, hipLaunchKernelGGL((k_stencil<NCV, RL, T>), dim3(grid_of(mp)), dim3(mp.bs), 0, stream(), u, in, out,
-                                       g_ws.beta, g_ws.active, nf, lat().g, mp, gco));
+                                       g_ws.beta, active, nf, lat().g, mp, gco));
 }
 
 // One Chebyshev step (k_cheb) for the active slots of R
@@ -934,16 +1119,17 @@ static void launch_cheb(const cplx<RL> *links, const slots<T> &xk, const slots<T
                                        xnext, b, g_ws.beta, cf, g_ws.active, R, lat().g, mp, mode, fin, fi, fo));
 }
 
-// FP64 true residual r = y - A x of the R slots x (r stored as TR when
-// WRITE); partial ||r||^2 to g_ws.spart.  Returns the partials per slot.
-template <typename RL, typename TR, bool WRITE>
-static int64_t launch_resid(const cplx<RL> *u, int R, const slots<double> &x, const slots<TR> &res)
+// True residual r = y - A x of the R slots x (the active ones; all when active
+// is null) in the arithmetic type T (r stored as TR when WRITE); partial
+// ||r||^2 to g_ws.spart.  Returns the partials per slot.
+template <typename RL, typename T, typename TR, bool WRITE>
+static int64_t launch_resid(const cplx<RL> *u, int R, const slots<T> &x, const slots<T> &y, const slots<TR> &res,
+                            const int *active)
 {
-    const slots<double> ty = ws_slots(g_ws.y, R);
-    const int nc = shape().nc64;
+    const int nc = nc_of<T>();
     const lf_map mp = cn_map(R, nc);
-    NC_DISPATCH(nc, hipLaunchKernelGGL((k_cn_resid<NCV, RL, TR, WRITE>), dim3(grid_of(mp)), dim3(mp.bs), 0, stream(), u, x, ty,
-                                       res, g_ws.beta, R, lat().g, mp, g_ws.spart));
+    NC_DISPATCH(nc, hipLaunchKernelGGL((k_cn_resid<NCV, RL, T, TR, WRITE>), dim3(grid_of(mp)), dim3(mp.bs), 0, stream(), u, x,
+                                       y, res, g_ws.beta, active, R, lat().g, mp, g_ws.spart));
     return mp.nsb;
 }
 
@@ -960,33 +1146,26 @@ static int64_t launch_rhs(const cplx<RL> *u, int R, const slots<double> &psi, co
     return mp.nsb;
 }
 
-template <typename RL, typename T>
-static int apply_t(const cplx<RL> *u, const cplx<T> *in, cplx<T> *out, int nf)
-{
-    launch_stencil<RL, T>(u, ws_slots(in, nf), ws_slots(out, nf), nf);
-    NRQ_HIP(hipGetLastError());
-    return NRQ_OK;
-}
-
 int krylov_norms2(const cplx<double> *x, int nf, double *out)
 {
     std::vector<int> all(nf, 1);
     if (int e = upload_active(all)) return e;
     const int64_t n = 3 * g_ws.vol;
-    hipLaunchKernelGGL(k_norm2<double>, dim3(VBLOCKS, nf), dim3(VTHREADS), 0, stream(), x, n, g_ws.active, g_ws.rpart);
+    const unsigned nb = vblocks(n);
+    hipLaunchKernelGGL(k_norm2<double>, dim3(nb, nf), dim3(VTHREADS), 0, stream(), x, n, g_ws.active, g_ws.rpart);
     NRQ_HIP(hipGetLastError());
-    if (int e = fold_slots(g_ws.rpart, VBLOCKS, nf, g_ws.active, g_ws.nrm)) return e;
-    if (int e = nrm_to_host()) return e;
+    if (int e = fold_slots(g_ws.rpart, nb, nf, g_ws.active, g_ws.nrm, g_ws.nbuf)) return e;
+    if (int e = wait_sums()) return e;
     memcpy(out, g_ws.nbuf, sizeof(double) * nf);
     return NRQ_OK;
 }
 
 // f1_r = beta_r K in_r, f2_r = beta_r K f1_r for the active slots of R
 template <typename RL, typename T>
-static int bk_features(const cplx<RL> *u, const slots<T> &in, const slots<T> &f1, const slots<T> &f2, int R)
+static int bk_features(const cplx<RL> *u, const slots<T> &in, const slots<T> &f1, const slots<T> &f2, int R, const int *active)
 {
-    launch_stencil<RL, T>(u, in, f1, R, g_ws.negone);
-    launch_stencil<RL, T>(u, f1, f2, R, g_ws.negone);
+    launch_stencil<RL, T>(u, in, f1, R, active, g_ws.negone);
+    launch_stencil<RL, T>(u, f1, f2, R, active, g_ws.negone);
     NRQ_HIP(hipGetLastError());
     return NRQ_OK;
 }
@@ -997,8 +1176,8 @@ int krylov_rhs_features(const nrq_gauge *gf, int R, const cplx<double> **f1, con
     std::vector<int> all(R, 1);
     if (int e = upload_active(all)) return e;
     const slots<double> y = ws_slots(g_ws.y, R), a = ws_slots(g_ws.t, R), b = ws_slots(g_ws.res, R);
-    const int e = gf->precision == 64 ? bk_features<double, double>((const cplx<double> *)gauge_links(gf), y, a, b, R)
-                                      : bk_features<float, double>((const cplx<float> *)gauge_links(gf), y, a, b, R);
+    const int e = gf->precision == 64 ? bk_features<double, double>((const cplx<double> *)gauge_links(gf), y, a, b, R, g_ws.active)
+                                      : bk_features<float, double>((const cplx<float> *)gauge_links(gf), y, a, b, R, g_ws.active);
     if (e) return e;
     *f1 = g_ws.t;
     *f2 = g_ws.res;
@@ -1013,12 +1192,21 @@ static cplx<double> g_beta_host[NSLOTS];
 
 // ---------------------------------------------------------------------------
 // GMRES(m) core: solves (1 + beta_r K) x_r = b_r for the slots with act[r],
-// from the current x (x = 0 when zero_guess), until the T-precision true
+// from the current x (x = 0 when zero_guess: x is then only written, and
+// becomes 0 for the slots that need no step), until the T-precision true
 // residual satisfies ||b - A x|| <= tol ||b|| or its[r] reaches maxit.
 // rel_out[r] receives the last true relative residual.  beta must already be
-// on the device.
+// on the device; res is scratch, and may hold b.
+//
+// A step is five launches (operator, dot products, their fold, Gram-Schmidt
+// update, rotation) that need nothing from the host: the rotations and the
+// decision whether a slot goes on are made on the device (k_gm_step), which
+// every kernel of the next step looks at.  The host enqueues step j + 2 once it
+// has seen step j end, so the queue does not run empty; the one step enqueued
+// too many leaves at its first instruction.
 // ---------------------------------------------------------------------------
-// With net (FGMRES): z_j = M(v_j), w = A z_j, x += Z y.  A slot
+// With net (FGMRES): z_j = M(W_j), A z_j in place of A W_j, x from the z_j (M
+// is positively homogeneous, so z_j carries the scale factor of W_j).  A slot
 // whose network output makes the Arnoldi step non-finite, whose cycle reduces
 // its residual by less than FGMRES_STALL, or that has not converged after
 // FGMRES_CYCLES cycles leaves the solve with x intact and fallen[r] = 1, for
@@ -1026,26 +1214,31 @@ static cplx<double> g_beta_host[NSLOTS];
 constexpr double FGMRES_STALL = 0.1;
 constexpr int FGMRES_CYCLES = 4;
 template <typename T, typename RL>
-static int gmres_core(const cplx<RL> *links, int R, const cplx<T> *b, cplx<T> *x, cplx<T> *basis, cplx<T> *t,
+static int gmres_core(const cplx<RL> *links, int R, const cplx<T> *b, const slots<T> &x, cplx<T> *basis, cplx<T> *t,
                       cplx<T> *res, bool zero_guess, const double *bnorm, std::vector<int> act, double tol, int m,
                       int64_t maxit, std::vector<int64_t> &its, double *rel_out, int64_t &cycles,
                       nrq_cnn *net = nullptr, cplx<T> *zbasis = nullptr, std::vector<int> *fallen = nullptr)
 {
-    typedef std::complex<double> zc;
     const int64_t n = 3 * g_ws.vol;
-    const size_t fbytes = sizeof(cplx<T>) * (size_t)n;
+    const unsigned nb = vblocks(n);
+    const gm_state gm = g_ws.gm;
+    const slots<T> bs = ws_slots(b, R), rs = ws_slots(res, R);
     std::vector<double> rn(R, 0.0);
-    if (int e = upload_active(act)) return e;
     const cplx<T> *r0 = res; // residual the next cycle starts from
+    // ||b - A x||^2 of the slots in `on` (device mask) to g_ws.nbuf; WRITE: and the residual to res
+    auto residual = [&](bool write, const int *on) -> int {
+        const int64_t nsb = write ? launch_resid<RL, T, T, true>(links, R, x, bs, rs, on)
+                                  : launch_resid<RL, T, T, false>(links, R, x, bs, rs, on);
+        NRQ_HIP(hipGetLastError());
+        return fold_slots(g_ws.spart, nsb, R, on, g_ws.nrm, g_ws.nbuf);
+    };
     if (zero_guess) {
-        NRQ_HIP(hipMemsetAsync(x, 0, fbytes * R, stream()));
         r0 = b;
         for (int r = 0; r < R; ++r) rn[r] = bnorm[r];
     } else {
-        if (int e = apply_t<RL, T>(links, x, t, R)) return e;
-        hipLaunchKernelGGL(k_residual<T>, dim3(VBLOCKS, R), dim3(VTHREADS), 0, stream(), b, t, res, n, g_ws.active, g_ws.rpart);
-        if (int e = fold_slots(g_ws.rpart, VBLOCKS, R, g_ws.active, g_ws.nrm)) return e;
-        if (int e = nrm_to_host()) return e;
+        if (int e = upload_active(act)) return e;
+        if (int e = residual(true, g_ws.active)) return e;
+        if (int e = wait_sums()) return e;
         for (int r = 0; r < R; ++r) rn[r] = act[r] ? std::sqrt(std::max(g_ws.nbuf[r], 0.0)) : 0.0;
     }
     for (int r = 0; r < R; ++r) {
@@ -1053,156 +1246,110 @@ static int gmres_core(const cplx<RL> *links, int R, const cplx<T> *b, cplx<T> *x
         rel_out[r] = bnorm[r] > 0 ? rn[r] / bnorm[r] : 0.0;
         if (rn[r] <= tol * bnorm[r]) act[r] = 0;
     }
-    std::vector<std::vector<zc>> H(R, std::vector<zc>((size_t)(m + 1) * m)), G(R, std::vector<zc>(m + 1)),
-        SN(R, std::vector<zc>(m)), Y(R, std::vector<zc>(m));
-    std::vector<std::vector<double>> CS(R, std::vector<double>(m));
-    std::vector<int> jused(R, 0), cycle(R), ncycles(R, 0);
+    std::vector<int> ncycles(R, 0);
     std::vector<double> rn_start(R, 0.0);
-    double *restart_n2 = g_ws.nrm + workspace::NRM_RESTART;
+    bool first = true;
     while (true) {
         bool any = false;
         for (int r = 0; r < R; ++r) any = any || act[r];
-        if (!any) break;
+        if (!any) {
+            if (first && zero_guess) {
+                // no slot needs a step: x = 0
+                for (int r = 0; r < R; ++r) NRQ_HIP(hipMemsetAsync(x.p[r], 0, sizeof(cplx<T>) * (size_t)n, stream()));
+            }
+            break;
+        }
         ++cycles;
         rn_start = rn;
-        std::vector<double> rn2(R);
+        gm_start in = {};
         for (int r = 0; r < R; ++r) {
-            rn2[r] = act[r] ? rn[r] * rn[r] : 0.0;
-            std::fill(G[r].begin(), G[r].end(), zc(0));
-            G[r][0] = rn[r];
-            jused[r] = 0;
+            in.rn[r] = rn[r];
+            in.stop[r] = tol * bnorm[r];
+            in.left[r] = (int)std::min<int64_t>(m, std::max<int64_t>(1, maxit - its[r]));
         }
-        NRQ_HIP(hipMemcpyAsync(restart_n2, rn2.data(), sizeof(double) * R, hipMemcpyHostToDevice, stream()));
-        if (int e = upload_active(act)) return e;
-        hipLaunchKernelGGL(k_scale<T>, dim3(VBLOCKS, R), dim3(VTHREADS), 0, stream(), r0, basis, n, (const double *)restart_n2,
-                           g_ws.active);
-        cycle = act;
+        in.act = mask_of(act);
+        hipLaunchKernelGGL(k_gm_begin, dim3(1), dim3(64), 0, stream(), gm, in);
+        if (net && r0 == res) {
+            // res holds features below: the starting residual moves to the basis
+            NRQ_HIP(hipMemcpyAsync(basis, res, sizeof(cplx<T>) * (size_t)n * R, hipMemcpyDeviceToDevice, stream()));
+            r0 = basis;
+        }
+        const gm_basis<T> W = {r0, basis};
+        std::vector<int> cycle = act;
         for (int j = 0; j < m; ++j) {
-            bool busy = false;
-            for (int r = 0; r < R; ++r) busy = busy || cycle[r];
-            if (!busy) break;
-            if (int e = upload_active(cycle)) return e;
-            cplx<T> *vj = basis + (size_t)j * R * n;
+            // with a network the host needs the slots that are left
+            const int seen = net ? j - 1 : j - 2;
+            if (seen >= 0) {
+                NRQ_HIP(hipEventSynchronize(g_ws.ev[seen & 1]));
+                bool busy = false;
+                for (int r = 0; r < R; ++r) {
+                    cycle[r] = *(volatile int *)(g_ws.ibuf + (seen & 1) * NSLOTS + r);
+                    busy = busy || cycle[r];
+                }
+                if (!busy) break;
+            }
             cplx<T> *w = basis + (size_t)(j + 1) * R * n;
+            const slots<T> vj = ws_slots(W.at(j, 0, R, n), R);
             if (net) {
-                // z_j = M(v_j) from v_j and its features beta K v_j (in t) and
-                // (beta K)^2 v_j (in res; the next cycle's residual is
+                // z_j = M(W_j) from W_j and its features beta K W_j (in t) and
+                // (beta K)^2 W_j (in res; the next cycle's residual is
                 // recomputed after this loop)
                 cplx<T> *zj = zbasis + (size_t)j * R * n;
-                if (int e = bk_features<RL, T>(links, ws_slots(vj, R), ws_slots(t, R), ws_slots(res, R), R)) return e;
+                if (int e = bk_features<RL, T>(links, vj, ws_slots(t, R), rs, R, gm.cyc)) return e;
                 const cplx<T> *vp[NSLOTS], *f1p[NSLOTS], *f2p[NSLOTS];
                 cplx<T> *zp[NSLOTS];
                 for (int r = 0; r < R; ++r) {
-                    vp[r] = vj + (size_t)r * n;
+                    vp[r] = vj.p[r];
                     f1p[r] = t + (size_t)r * n;
                     f2p[r] = res + (size_t)r * n;
                     zp[r] = zj + (size_t)r * n;
                 }
                 if (int e = cnn_precondition<T>(net, vp, f1p, f2p, zp, R, cycle.data(), g_beta_host)) return e;
-                if (int e = apply_t<RL, T>(links, zj, w, R)) return e;
-            } else if (int e = apply_t<RL, T>(links, vj, w, R)) {
-                return e;
+                launch_stencil<RL, T>(links, ws_slots(zj, R), ws_slots(w, R), R, gm.cyc);
+            } else {
+                launch_stencil<RL, T>(links, vj, ws_slots(w, R), R, gm.cyc);
             }
             const int nv = j + 1;
-            hipLaunchKernelGGL(k_mdot<T>, dim3(VBLOCKS, R), dim3(VTHREADS), 0, stream(), (const cplx<T> *)basis, nv,
-                               (const cplx<T> *)w, n, R, g_ws.active, g_ws.cpart);
-            hipLaunchKernelGGL(k_fold_c, dim3((nv * R + 3) / 4), dim3(256), 0, stream(), g_ws.cpart, VBLOCKS, nv, R, g_ws.active,
-                               g_ws.hdev);
-            hipLaunchKernelGGL(k_cgs_update<T>, dim3(VBLOCKS, R), dim3(VTHREADS), 0, stream(), (const cplx<T> *)basis, nv, w, n, R,
-                               g_ws.active, g_ws.hdev, g_ws.rpart);
-            if (int e = fold_slots(g_ws.rpart, VBLOCKS, R, g_ws.active, g_ws.nrm)) return e;
-            hipLaunchKernelGGL(k_scale<T>, dim3(VBLOCKS, R), dim3(VTHREADS), 0, stream(), (const cplx<T> *)w, w, n,
-                               (const double *)g_ws.nrm, g_ws.active);
+            hipLaunchKernelGGL(k_mdot<T>, dim3(nb, R), dim3(VTHREADS), 0, stream(), W, nv, (const cplx<T> *)w, n, R,
+                               (const int *)gm.cyc, g_ws.cpart);
+            hipLaunchKernelGGL(k_gm_dots, dim3((nv * R + 3) / 4), dim3(256), 0, stream(), g_ws.cpart, (int)nb, nv, R, gm);
+            hipLaunchKernelGGL(k_cgs_update<T>, dim3(nb, R), dim3(VTHREADS), 0, stream(), W, nv, w, n, R, gm, g_ws.rpart);
+            hipLaunchKernelGGL(k_gm_step, dim3(R), dim3(VTHREADS), 0, stream(), g_ws.rpart, (int)nb, j, net ? 1 : 0, gm,
+                               g_ws.ibuf + (j & 1) * NSLOTS);
             NRQ_HIP(hipGetLastError());
-            NRQ_HIP(hipMemcpyAsync(g_ws.hbuf, g_ws.hdev, sizeof(cplx<double>) * nv * R, hipMemcpyDeviceToHost, stream()));
-            if (int e = nrm_to_host()) return e;
-            for (int r = 0; r < R; ++r) {
-                if (!cycle[r]) continue;
-                if (net) {
-                    // the network's direction broke the Arnoldi step: end the
-                    // slot's cycle before column j (x keeps columns < j)
-                    bool fin = std::isfinite(g_ws.nbuf[r]);
-                    for (int i = 0; i < nv && fin; ++i)
-                        fin = std::isfinite(g_ws.hbuf[r * nv + i].re) && std::isfinite(g_ws.hbuf[r * nv + i].im);
-                    if (!fin) {
-                        cycle[r] = 0;
-                        (*fallen)[r] = 1;
-                        continue;
-                    }
-                }
-                ++its[r];
-                zc *Hc = H[r].data() + (size_t)(m + 1) * j;
-                for (int i = 0; i < nv; ++i) Hc[i] = zc(g_ws.hbuf[r * nv + i].re, g_ws.hbuf[r * nv + i].im);
-                const double hn = std::sqrt(std::max(g_ws.nbuf[r], 0.0));
-                for (int i = 0; i < j; ++i) {
-                    const zc a = Hc[i], c = Hc[i + 1];
-                    Hc[i] = CS[r][i] * a + SN[r][i] * c;
-                    Hc[i + 1] = -std::conj(SN[r][i]) * a + CS[r][i] * c;
-                }
-                const zc a = Hc[j];
-                const double den = std::sqrt(std::norm(a) + hn * hn);
-                if (den == 0) {
-                    CS[r][j] = 1;
-                    SN[r][j] = 0;
-                } else if (std::abs(a) == 0) {
-                    CS[r][j] = 0;
-                    SN[r][j] = 1;
-                } else {
-                    CS[r][j] = std::abs(a) / den;
-                    SN[r][j] = (a / std::abs(a)) * (hn / den);
-                }
-                Hc[j] = CS[r][j] * a + SN[r][j] * hn;
-                G[r][j + 1] = -std::conj(SN[r][j]) * G[r][j];
-                G[r][j] = CS[r][j] * G[r][j];
-                jused[r] = j + 1;
-                if (std::abs(G[r][j + 1]) <= tol * bnorm[r] || its[r] >= maxit) cycle[r] = 0;
-            }
+            NRQ_HIP(hipEventRecord(g_ws.ev[j & 1], stream()));
         }
-        // y = H^-1 g per slot, x += V y
-        std::vector<int> nu(R, 0);
-        for (int r = 0; r < R; ++r) {
-            if (!act[r]) continue;
-            const int jj = jused[r];
-            nu[r] = jj;
-            for (int i = jj - 1; i >= 0; --i) {
-                zc sacc = G[r][i];
-                for (int k = i + 1; k < jj; ++k) sacc -= H[r][(size_t)(m + 1) * k + i] * Y[r][k];
-                Y[r][i] = sacc / H[r][(size_t)(m + 1) * i + i];
-            }
-            if (net) {
-                bool fin = true;
-                for (int i = 0; i < jj && fin; ++i) fin = std::isfinite(Y[r][i].real()) && std::isfinite(Y[r][i].imag());
-                if (!fin) {
-                    nu[r] = 0; // keep x
-                    (*fallen)[r] = 1;
-                }
-            }
-            for (int i = 0; i < nu[r]; ++i) g_ws.hbuf[r * (m + 1) + i] = {Y[r][i].real(), Y[r][i].imag()};
-        }
-        if (int e = upload_active(act)) return e;
-        NRQ_HIP(hipMemcpyAsync(g_ws.ydev, g_ws.hbuf, sizeof(cplx<double>) * R * (m + 1), hipMemcpyHostToDevice, stream()));
-        if (int e = upload_ints(g_ws.nused, nu)) return e;
-        hipLaunchKernelGGL(k_xupdate<T>, dim3(VBLOCKS, R), dim3(VTHREADS), 0, stream(), x,
-                           (const cplx<T> *)(net ? zbasis : basis), R, n, g_ws.ydev, m + 1, g_ws.nused, g_ws.active);
+        hipLaunchKernelGGL(k_gm_solve, dim3(R), dim3(64), 0, stream(), gm, net ? 1 : 0, g_ws.ibuf + workspace::I_USED,
+                           g_ws.ibuf + workspace::I_FALLEN);
+        const gm_basis<T> X = net ? gm_basis<T>{zbasis, zbasis} : W;
+        hipLaunchKernelGGL(k_xupdate<T>, dim3(nb, R), dim3(VTHREADS), 0, stream(), x, X, R, n, gm, first && zero_guess ? 1 : 0);
         // true residual in precision T
-        if (int e = apply_t<RL, T>(links, x, t, R)) return e;
-        hipLaunchKernelGGL(k_residual<T>, dim3(VBLOCKS, R), dim3(VTHREADS), 0, stream(), b, (const cplx<T> *)t, res, n,
-                           g_ws.active, g_ws.rpart);
-        r0 = res;
-        if (int e = fold_slots(g_ws.rpart, VBLOCKS, R, g_ws.active, g_ws.nrm)) return e;
-        if (int e = nrm_to_host()) return e;
+        if (int e = residual(false, gm.act)) return e;
+        if (int e = wait_sums()) return e;
+        first = false;
+        bool again = false;
         for (int r = 0; r < R; ++r) {
             if (!act[r]) continue;
+            its[r] += g_ws.ibuf[workspace::I_USED + r];
+            const bool fell = net && g_ws.ibuf[workspace::I_FALLEN + r];
+            if (fell) (*fallen)[r] = 1;
             rn[r] = std::sqrt(std::max(g_ws.nbuf[r], 0.0));
             rel_out[r] = bnorm[r] > 0 ? rn[r] / bnorm[r] : 0.0;
             if (rn[r] <= tol * bnorm[r] || its[r] >= maxit) {
                 act[r] = 0;
                 continue;
             }
-            if (net && ((*fallen)[r] || !(rn[r] <= FGMRES_STALL * rn_start[r]) || ++ncycles[r] >= FGMRES_CYCLES)) {
+            if (net && (fell || !(rn[r] <= FGMRES_STALL * rn_start[r]) || ++ncycles[r] >= FGMRES_CYCLES)) {
                 act[r] = 0;
                 (*fallen)[r] = 1;
             }
+            again = again || act[r];
+        }
+        if (again) {
+            // another cycle starts from the residual: one more pass stores it
+            if (int e = upload_active(act)) return e;
+            if (int e = residual(true, g_ws.active)) return e;
+            r0 = res;
         }
     }
     return NRQ_OK;
@@ -1311,13 +1458,14 @@ static int cheb_run(const cplx<RL> *links, int R, const cplx<T> *b, cplx<T> *x, 
 template <typename RL>
 static int cn_resid(const cplx<RL> *u, int R, const slots<double> &x, cplx<float> *res32)
 {
+    const slots<double> y = ws_slots(g_ws.y, R);
     int64_t nsb;
     if (res32)
-        nsb = launch_resid<RL, float, true>(u, R, x, ws_slots(res32, R));
+        nsb = launch_resid<RL, double, float, true>(u, R, x, y, ws_slots(res32, R), nullptr);
     else
-        nsb = launch_resid<RL, float, false>(u, R, x, slots<float>{});
+        nsb = launch_resid<RL, double, float, false>(u, R, x, y, slots<float>{}, nullptr);
     NRQ_HIP(hipGetLastError());
-    return fold_slots(g_ws.spart, nsb, R, nullptr, g_ws.nrm);
+    return fold_slots(g_ws.spart, nsb, R, nullptr, g_ws.nrm, g_ws.nbuf);
 }
 
 // Per-slot convergence check of the residual norms in g_ws.nbuf; returns
@@ -1380,7 +1528,7 @@ static int cheb_solve(const cplx<RL> *u, int R, const std::vector<zc> &alpha, co
             x = xk;
             for (int r = 0; r < R; ++r) its[r] += act[r] ? k : 0;
             if (int e = cn_resid<RL>(u, R, ws_slots(x, R), nullptr)) return e;
-            if (int e = nrm_to_host()) return e;
+            if (int e = wait_sums()) return e;
             if (round == 0) bn_from_host();
             if (!check_slots(R, bn, p.tol, act, rel, need)) break;
             if (int e = upload_active(act)) return e;
@@ -1406,7 +1554,7 @@ static int cheb_solve(const cplx<RL> *u, int R, const std::vector<zc> &alpha, co
         // FP64 residual pass; the FP64 true residual after the correction
         // still decides
         launch_stencil<float, float>(l32, ws_slots((const cplx<float> *)g_ws.t32, R), ws_slots(g_ws.y32, R), R,
-                                     g_ws.cpar + NSLOTS);
+                                     g_ws.active, g_ws.cpar + NSLOTS);
         NRQ_HIP(hipGetLastError());
     } else if (int e = cn_resid<RL>(u, R, tx, g_ws.y32)) {
         return e;
@@ -1436,11 +1584,11 @@ static int cheb_solve(const cplx<RL> *u, int R, const std::vector<zc> &alpha, co
             bnd[r] *= cheb_bound(sig[r], k) + FP32_CORR_ERR;
         }
     }
-    if (int e = nrm_to_host()) return e;
+    if (int e = wait_sums()) return e;
     bn_from_host();
     if (!*in_psi) {
         // no correction was needed: the guess goes to the heavy field
-        hipLaunchKernelGGL(k_copy_slots, dim3(VBLOCKS, R), dim3(VTHREADS), 0, stream(), tx, tpsi, 3 * g_ws.vol);
+        hipLaunchKernelGGL(k_copy_slots, dim3(vblocks(3 * g_ws.vol), R), dim3(VTHREADS), 0, stream(), tx, tpsi, 3 * g_ws.vol);
         NRQ_HIP(hipGetLastError());
         *in_psi = true;
     }
@@ -1452,7 +1600,7 @@ static int cheb_solve(const cplx<RL> *u, int R, const std::vector<zc> &alpha, co
         ++cycles;
         if (int e = correct(k)) return e;
         for (int r = 0; r < R; ++r) its[r] += act[r] ? k : 0;
-        if (int e = nrm_to_host()) return e;
+        if (int e = wait_sums()) return e;
     }
     return NRQ_OK;
 }
@@ -1477,10 +1625,10 @@ static int gmres_mixed(const cplx<RL> *u, int R, std::vector<double> &bn, const 
     const slots<double> tx = ws_slots(g_ws.x, R), tres = ws_slots(g_ws.res, R);
     for (int outer = 0; outer < 40; ++outer) {
         // FP64 true residual r = y - A x
-        const int64_t nsb = launch_resid<RL, double, true>(u, R, tx, tres);
+        const int64_t nsb = launch_resid<RL, double, double, true>(u, R, tx, ws_slots(g_ws.y, R), tres, nullptr);
         NRQ_HIP(hipGetLastError());
-        if (int e = fold_slots(g_ws.spart, nsb, R, nullptr, g_ws.nrm)) return e;
-        if (int e = nrm_to_host()) return e;
+        if (int e = fold_slots(g_ws.spart, nsb, R, nullptr, g_ws.nrm, g_ws.nbuf)) return e;
+        if (int e = wait_sums()) return e;
         bool any = false;
         for (int r = 0; r < R; ++r) {
             if (!act[r]) continue;
@@ -1496,13 +1644,13 @@ static int gmres_mixed(const cplx<RL> *u, int R, std::vector<double> &bn, const 
         NRQ_HIP(hipMemcpyAsync(rnorm2, g_ws.nrm, sizeof(double) * R, hipMemcpyDeviceToDevice, stream()));
         // normalised FP32 correction problem A d = r / ||r||
         if (int e = upload_active(act)) return e;
-        hipLaunchKernelGGL(k_demote, dim3(VBLOCKS, R), dim3(VTHREADS), 0, stream(), (const cplx<double> *)g_ws.res, g_ws.y32, n,
+        hipLaunchKernelGGL(k_demote, dim3(vblocks(n), R), dim3(VTHREADS), 0, stream(), (const cplx<double> *)g_ws.res, g_ws.y32, n,
                            (const double *)rnorm2, g_ws.active);
         std::vector<double> inner_rel(R, 0.0);
         int64_t inner_cycles = 0;
         const double itol = std::max(p.inner_tol, std::max(p.tol / 1e-3, 2e-7));
         std::vector<int> fallen(R, 0);
-        if (int e = gmres_core<float, float>(l32, R, g_ws.y32, g_ws.x32, (cplx<float> *)g_ws.basis, g_ws.t32, g_ws.res32, true,
+        if (int e = gmres_core<float, float>(l32, R, g_ws.y32, ws_slots(g_ws.x32, R), (cplx<float> *)g_ws.basis, g_ws.t32, g_ws.res32, true,
                                              one.data(), act, itol, p.restart, p.maxit, its, inner_rel.data(), inner_cycles,
                                              net, (cplx<float> *)g_ws.zbasis, net ? &fallen : nullptr))
             return e;
@@ -1510,7 +1658,7 @@ static int gmres_mixed(const cplx<RL> *u, int R, std::vector<double> &bn, const 
         for (int f : fallen) nfall += f;
         if (nfall) {
             g_fallbacks += nfall;
-            if (int e = gmres_core<float, float>(l32, R, g_ws.y32, g_ws.x32, (cplx<float> *)g_ws.basis, g_ws.t32, g_ws.res32,
+            if (int e = gmres_core<float, float>(l32, R, g_ws.y32, ws_slots(g_ws.x32, R), (cplx<float> *)g_ws.basis, g_ws.t32, g_ws.res32,
                                                  false, one.data(), fallen, itol, p.restart, p.maxit, its, inner_rel.data(),
                                                  inner_cycles))
                 return e;
@@ -1518,7 +1666,7 @@ static int gmres_mixed(const cplx<RL> *u, int R, std::vector<double> &bn, const 
         // gmres_core left the slot masks of the inner solve on the device;
         // the refinement updates every slot that is still active here
         if (int e = upload_active(act)) return e;
-        hipLaunchKernelGGL(k_promote_add, dim3(VBLOCKS, R), dim3(VTHREADS), 0, stream(), g_ws.x, (const cplx<float> *)g_ws.x32, n,
+        hipLaunchKernelGGL(k_promote_add, dim3(vblocks(n), R), dim3(VTHREADS), 0, stream(), g_ws.x, (const cplx<float> *)g_ws.x32, n,
                            (const double *)rnorm2, g_ws.active);
         NRQ_HIP(hipGetLastError());
     }
@@ -1541,7 +1689,7 @@ static int cn_step_t(const cplx<RL> *u, int R, const std::vector<zc> &alpha, con
     const int wk = guess && p.kind == KRYLOV_CHEB_MIXED ? 1 : 0;
     const int64_t nsb = launch_rhs<RL>(u, R, tpsi, ty, tx, guess ? 1 : 0, ws_slots(g_ws.t32, R), wk);
     NRQ_HIP(hipGetLastError());
-    if (int e = fold_slots(g_ws.spart, nsb, R, nullptr, g_ws.nrm + workspace::NRM_Y)) return e;
+    if (int e = fold_slots(g_ws.spart, nsb, R, nullptr, g_ws.nrm + workspace::NRM_Y, g_ws.nbuf + workspace::NRM_Y)) return e;
     cplx<double> *xsol = g_ws.x;
     bool in_psi = false;
     int status = NRQ_OK;
@@ -1552,28 +1700,30 @@ static int cn_step_t(const cplx<RL> *u, int R, const std::vector<zc> &alpha, con
         if (left) {
             // spectrum bound violated (e.g. links far from unitary): GMRES from here
             if (in_psi) {
-                hipLaunchKernelGGL(k_copy_slots, dim3(VBLOCKS, R), dim3(VTHREADS), 0, stream(), tpsi, tx, n);
+                hipLaunchKernelGGL(k_copy_slots, dim3(vblocks(n), R), dim3(VTHREADS), 0, stream(), tpsi, tx, n);
                 NRQ_HIP(hipGetLastError());
                 in_psi = false;
             } else if (xsol != g_ws.x) {
                 NRQ_HIP(hipMemcpyAsync(g_ws.x, xsol, sizeof(cplx<double>) * (size_t)n * R, hipMemcpyDeviceToDevice, stream()));
             }
             xsol = g_ws.x;
-            status = gmres_core<double, RL>(u, R, g_ws.y, g_ws.x, (cplx<double> *)g_ws.basis, g_ws.t, g_ws.res, false,
+            status = gmres_core<double, RL>(u, R, g_ws.y, tx, (cplx<double> *)g_ws.basis, g_ws.t, g_ws.res, false,
                                             bn.data(), act, p.tol, p.restart, p.maxit, its, rel.data(), cycles);
         }
     } else {
-        if (int e = nrm_to_host()) return e;
+        if (int e = wait_sums()) return e;
         for (int r = 0; r < R; ++r) bn[r] = std::sqrt(std::max(g_ws.nbuf[workspace::NRM_Y + r], 0.0));
-        if (p.kind == KRYLOV_GMRES_FP64)
-            status = gmres_core<double, RL>(u, R, g_ws.y, g_ws.x, (cplx<double> *)g_ws.basis, g_ws.t, g_ws.res, true,
+        if (p.kind == KRYLOV_GMRES_FP64) {
+            // from a zero guess, straight into the heavy field
+            status = gmres_core<double, RL>(u, R, g_ws.y, tpsi, (cplx<double> *)g_ws.basis, g_ws.t, g_ws.res, true,
                                             bn.data(), act, p.tol, p.restart, p.maxit, its, rel.data(), cycles);
-        else if (p.kind == KRYLOV_FGMRES_CNN) {
+            in_psi = true;
+        } else if (p.kind == KRYLOV_FGMRES_CNN) {
             nrq_cnn *net = cn_preconditioner();
             if (!net) return fail(NRQ_ERR_STATE, "CN: FGMRES needs a network (nrq_cn_set_preconditioner)");
             if (int e = reserve_zbasis()) return e;
             std::vector<int> fallen(R, 0);
-            status = gmres_core<double, RL>(u, R, g_ws.y, g_ws.x, (cplx<double> *)g_ws.basis, g_ws.t, g_ws.res,
+            status = gmres_core<double, RL>(u, R, g_ws.y, tx, (cplx<double> *)g_ws.basis, g_ws.t, g_ws.res,
                                             !p.extrapolate, bn.data(), act, p.tol, p.restart, p.maxit, its, rel.data(),
                                             cycles, net, g_ws.zbasis, &fallen);
             int nfall = 0;
@@ -1583,7 +1733,7 @@ static int cn_step_t(const cplx<RL> *u, int R, const std::vector<zc> &alpha, con
                 // operator's diagonal is constant, so Jacobi scaling leaves
                 // GMRES unchanged) from the iterate reached so far
                 g_fallbacks += nfall;
-                status = gmres_core<double, RL>(u, R, g_ws.y, g_ws.x, (cplx<double> *)g_ws.basis, g_ws.t, g_ws.res,
+                status = gmres_core<double, RL>(u, R, g_ws.y, tx, (cplx<double> *)g_ws.basis, g_ws.t, g_ws.res,
                                                 false, bn.data(), fallen, p.tol, p.restart, p.maxit, its, rel.data(),
                                                 cycles);
             }
@@ -1598,7 +1748,7 @@ static int cn_step_t(const cplx<RL> *u, int R, const std::vector<zc> &alpha, con
     if (status) return status;
     if (!in_psi) {
         // psi_f = x for every slot
-        hipLaunchKernelGGL(k_copy_slots, dim3(VBLOCKS, R), dim3(VTHREADS), 0, stream(), ws_slots(xsol, R), tpsi, n);
+        hipLaunchKernelGGL(k_copy_slots, dim3(vblocks(n), R), dim3(VTHREADS), 0, stream(), ws_slots(xsol, R), tpsi, n);
         NRQ_HIP(hipGetLastError());
     }
     double worst = 0;
