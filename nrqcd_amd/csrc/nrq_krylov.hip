@@ -27,6 +27,7 @@
 // convergence: precision and solver change the work, never the answer.
 #include "nrq_krylov.h"
 #include "nrq_cnn.h"
+#include "nrq_hop_tile.h"
 #include "nrq_map.h"
 #include <algorithm>
 #include <cmath>
@@ -466,6 +467,154 @@ __global__ __launch_bounds__(SBS_WAVE, CN_WAVES) void k_cheb(const cplx<RL> *__r
 }
 
 // ---------------------------------------------------------------------------
+// the same four kernels through LDS tiles (k_hop_tile of nrq_hop_tile.h): what
+// each does at a site of slot r once it has the hop
+// ---------------------------------------------------------------------------
+
+// k_stencil
+template <typename T> struct tile_stencil {
+    static constexpr bool NORM = false;
+    struct pre {};
+    slots<T> src, out;
+    const cplx<double> *beta, *gco;
+    const int *active;
+    __device__ __forceinline__ bool on(int r) const { return !active || active[r]; }
+    __device__ __forceinline__ const cplx<T> *in(int r) const { return src.p[r]; }
+    __device__ __forceinline__ void load(int, int64_t, uint32_t, pre &) const {}
+    __device__ __forceinline__ void use(int r, int64_t vol, uint32_t s, const pre &, const cplx<T> (&f)[3],
+                                        const cplx<T> (&hop)[3], T dsum, double &) const
+    {
+        cplx<double> b = beta[r];
+        if (gco) {
+            const cplx<double> gc = gco[r];
+            b = {-(b.re * gc.re - b.im * gc.im), -(b.re * gc.im + b.im * gc.re)};
+        }
+        const cplx<T> cf = to<T>(b);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const cplx<T> kf = dsum * f[c] - T(0.5) * hop[c];
+            store_nt(at32(out.p[r] + (int64_t)c * vol, s), gco ? cf * kf : f[c] + cf * kf);
+        }
+    }
+    __device__ __forceinline__ void sum(int, unsigned, double) const {}
+};
+
+// k_cn_rhs
+struct tile_rhs {
+    static constexpr bool NORM = true;
+    struct pre {};
+    slots<double> psi, y, x;
+    slots<float> kout;
+    const cplx<double> *alpha, *gco;
+    double *partial;
+    int64_t nsb;
+    int guess, wk;
+    __device__ __forceinline__ bool on(int) const { return true; }
+    __device__ __forceinline__ const cplx<double> *in(int r) const { return psi.p[r]; }
+    __device__ __forceinline__ void load(int, int64_t, uint32_t, pre &) const {}
+    __device__ __forceinline__ void use(int r, int64_t vol, uint32_t s, const pre &, const cplx<double> (&f)[3],
+                                        const cplx<double> (&hop)[3], double dsum, double &nrm) const
+    {
+        const cplx<double> a = alpha[r], gc = gco[r];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const int64_t cv = (int64_t)c * vol;
+            const cplx<double> kf = dsum * f[c] - 0.5 * hop[c];
+            const cplx<double> yv = f[c] + a * kf;
+            store_nt(at32(y.p[r] + cv, s), yv);
+            if (x.p[r]) store_nt(at32(x.p[r] + cv, s), guess ? f[c] + gc * kf : cplx<double>{0.0, 0.0});
+            if (wk) store_nt(at32(kout.p[r] + cv, s), cplx<float>{(float)kf.re, (float)kf.im});
+            nrm += nrm2(yv);
+        }
+    }
+    __device__ __forceinline__ void sum(int r, unsigned i, double v) const { partial[(int64_t)r * nsb + i] = v; }
+};
+
+// k_cn_resid
+template <typename T, typename TR, bool WRITE_RES> struct tile_resid {
+    static constexpr bool NORM = true;
+    struct pre {
+        cplx<T> y[3];
+    };
+    slots<T> x, y;
+    slots<TR> res;
+    const cplx<double> *beta;
+    const int *active;
+    double *partial;
+    int64_t nsb;
+    __device__ __forceinline__ bool on(int r) const { return !active || active[r]; }
+    __device__ __forceinline__ const cplx<T> *in(int r) const { return x.p[r]; }
+    __device__ __forceinline__ void load(int r, int64_t vol, uint32_t s, pre &v) const
+    {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) v.y[c] = load_nt(at32((const cplx<T> *)y.p[r] + (int64_t)c * vol, s));
+    }
+    __device__ __forceinline__ void use(int r, int64_t vol, uint32_t s, const pre &v, const cplx<T> (&f)[3],
+                                        const cplx<T> (&hop)[3], T dsum, double &nrm) const
+    {
+        const cplx<T> bt = to<T>(beta[r]);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const cplx<T> rr = v.y[c] - (f[c] + bt * (dsum * f[c] - T(0.5) * hop[c]));
+            if (WRITE_RES) store_nt(at32(res.p[r] + (int64_t)c * vol, s), cplx<TR>{(TR)rr.re, (TR)rr.im});
+            nrm += nrm2(rr);
+        }
+    }
+    __device__ __forceinline__ void sum(int r, unsigned i, double v) const { partial[(int64_t)r * nsb + i] = v; }
+};
+
+// k_cheb; FIN: with the FP64 iterate (fin)
+template <typename T, bool FIN> struct tile_cheb {
+    static constexpr bool NORM = false;
+    struct pre {
+        cplx<T> b[3], xp[3];
+        cplx<double> xo[FIN ? 3 : 1];
+    };
+    slots<T> xk, xprev, xnext, b;
+    slots<double> fin_in, fin_out;
+    const cplx<double> *beta, *coef;
+    const int *active;
+    int mode;
+    __device__ __forceinline__ bool on(int r) const { return !active || active[r]; }
+    __device__ __forceinline__ const cplx<T> *in(int r) const { return xk.p[r]; }
+    __device__ __forceinline__ void load(int r, int64_t vol, uint32_t s, pre &v) const
+    {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const int64_t cv = (int64_t)c * vol;
+            if (mode != 2) v.b[c] = load_nt(at32((const cplx<T> *)b.p[r] + cv, s));
+            if (mode == 0) v.xp[c] = load_nt(at32((const cplx<T> *)xprev.p[r] + cv, s));
+            if (FIN) v.xo[c] = load_nt(at32((const cplx<double> *)fin_in.p[r] + cv, s));
+        }
+    }
+    __device__ __forceinline__ void use(int r, int64_t vol, uint32_t s, const pre &v, const cplx<T> (&f)[3],
+                                        const cplx<T> (&hop)[3], T, double &) const
+    {
+        // c_r = 1 + beta_r dsum, so x_k's own value cancels in
+        // x_k + (b - x_k - beta_r (dsum x_k - hop / 2)) / c_r = (b + beta_r hop / 2) / c_r
+        const cplx<double> bd = beta[r], icd = coef[2 * r], rd = coef[2 * r + 1];
+        const cplx<T> ra = to<T>(rd * icd); // rho / c_r
+        const cplx<double> half = {0.5 * bd.re, 0.5 * bd.im}, om = {1.0 - rd.re, -rd.im};
+        const cplx<T> hb = to<T>(mode == 2 ? half * icd : half), pb = to<T>(mode == 3 ? om * icd : om);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const int64_t cv = (int64_t)c * vol;
+            const cplx<T> bq = mode == 2 ? f[c] : v.b[c];
+            cplx<T> t = bq, nx = {T(0), T(0)};
+            mac(t, hb, hop[c]);
+            mac(nx, ra, t);
+            if (mode == 3) mac(nx, pb, bq);
+            else if (mode == 0) mac(nx, pb, v.xp[c]);
+            if (FIN)
+                store_nt(at32(fin_out.p[r] + cv, s), cplx<double>{v.xo[c].re + (double)nx.re, v.xo[c].im + (double)nx.im});
+            else
+                store_nt(at32(xnext.p[r] + cv, s), nx);
+        }
+    }
+    __device__ __forceinline__ void sum(int, unsigned, double) const {}
+};
+
+// ---------------------------------------------------------------------------
 // vector kernels (grid: VBLOCKS x slots)
 // ---------------------------------------------------------------------------
 
@@ -903,6 +1052,8 @@ struct workspace {
         const size_t f32 = f64 / 2;
         int64_t sb = 0;
         for (int md = 0; md <= 4; ++md) sb = std::max(sb, make_lf_map(lg, md >= 3 ? SBS_WAVE : SBS, 8, md, 1).nsb);
+        const hop_tiles tl = hop_tiles_for(lg, 1); // fewer groups, more runs
+        sb = std::max(sb, (int64_t)tl.ntx * tl.nty * tl.nzr);
         auto dm = [](void **p, size_t b) { return hipMalloc(p, b) == hipSuccess; };
         bool ok = dm(&basis, f64 * (size_t)(mm + 1)) && dm((void **)&y, f64) && dm((void **)&x, f64) &&
                   dm((void **)&t, f64) && dm((void **)&res, f64) && dm((void **)&y32, f32) &&
@@ -1046,6 +1197,16 @@ static lf_map cn_map(int nf, int nc)
     return make_lf_map(lat().g, shape().mode >= 3 ? SBS_WAVE : SBS, shape().xcd, shape().mode, (nf + nc - 1) / nc);
 }
 
+// Whether a launch of nf slots goes through the LDS tiles: where they pay
+// (hop_tiles_for) and no other shape than the default was chosen.
+static bool use_tiles(int nf, hop_tiles *t)
+{
+    if (shape().mode != 4 || shape().xcd != 8) return false;
+    *t = hop_tiles_for(lat().g, nf);
+    return t->groups > 0;
+}
+static dim3 tile_grid(const hop_tiles &t) { return dim3(hop_grid(t)); }
+
 // Runs the statements after `nc` with the compile-time chunk width NCV equal
 // to nc (1, 2 or 4).
 #define NC_DISPATCH(nc, ...)                                                                                             \
@@ -1102,6 +1263,13 @@ template <typename RL, typename T>
 static void launch_stencil(const cplx<RL> *u, const slots<T> &in, const slots<T> &out, int nf,
                            const int *active, const cplx<double> *gco = nullptr)
 {
+    hop_tiles tl;
+    if (use_tiles(nf, &tl)) {
+        const tile_stencil<T> op = {in, out, g_ws.beta, gco, active};
+        hipLaunchKernelGGL((k_hop_tile<RL, T, tile_stencil<T>>), tile_grid(tl), dim3(HT_THREADS), 0, stream(), u, op, nf,
+                           lat().g, tl);
+        return;
+    }
     const int nc = nc_of<T>();
     const lf_map mp = cn_map(nf, nc);
     NC_DISPATCH(nc, hipLaunchKernelGGL((k_stencil<NCV, RL, T>), dim3(grid_of(mp)), dim3(mp.bs), 0, stream(), u, in, out,
@@ -1113,6 +1281,19 @@ template <typename RL, typename T>
 static void launch_cheb(const cplx<RL> *links, const slots<T> &xk, const slots<T> &xnext, const slots<T> &b,
                         const cplx<double> *cf, int R, int mode, int fin, const slots<double> &fi, const slots<double> &fo)
 {
+    hop_tiles tl;
+    if (use_tiles(R, &tl)) {
+        if (fin) {
+            const tile_cheb<T, true> op = {xk, xnext, xnext, b, fi, fo, g_ws.beta, cf, g_ws.active, mode};
+            hipLaunchKernelGGL((k_hop_tile<RL, T, tile_cheb<T, true>>), tile_grid(tl), dim3(HT_THREADS), 0, stream(), links,
+                               op, R, lat().g, tl);
+        } else {
+            const tile_cheb<T, false> op = {xk, xnext, xnext, b, fi, fo, g_ws.beta, cf, g_ws.active, mode};
+            hipLaunchKernelGGL((k_hop_tile<RL, T, tile_cheb<T, false>>), tile_grid(tl), dim3(HT_THREADS), 0, stream(), links,
+                               op, R, lat().g, tl);
+        }
+        return;
+    }
     const int nc = nc_of<T>();
     const lf_map mp = cn_map(R, nc);
     NC_DISPATCH(nc, hipLaunchKernelGGL((k_cheb<NCV, RL, T>), dim3(grid_of(mp)), dim3(mp.bs), 0, stream(), links, xk, xnext,
@@ -1126,6 +1307,14 @@ template <typename RL, typename T, typename TR, bool WRITE>
 static int64_t launch_resid(const cplx<RL> *u, int R, const slots<T> &x, const slots<T> &y, const slots<TR> &res,
                             const int *active)
 {
+    hop_tiles tl;
+    if (use_tiles(R, &tl)) {
+        const int64_t nsb = (int64_t)tl.ntx * tl.nty * tl.nzr;
+        const tile_resid<T, TR, WRITE> op = {x, y, res, g_ws.beta, active, g_ws.spart, nsb};
+        hipLaunchKernelGGL((k_hop_tile<RL, T, tile_resid<T, TR, WRITE>>), tile_grid(tl), dim3(HT_THREADS), 0, stream(), u, op,
+                           R, lat().g, tl);
+        return nsb;
+    }
     const int nc = nc_of<T>();
     const lf_map mp = cn_map(R, nc);
     NC_DISPATCH(nc, hipLaunchKernelGGL((k_cn_resid<NCV, RL, T, TR, WRITE>), dim3(grid_of(mp)), dim3(mp.bs), 0, stream(), u, x,
@@ -1139,6 +1328,14 @@ template <typename RL>
 static int64_t launch_rhs(const cplx<RL> *u, int R, const slots<double> &psi, const slots<double> &y,
                           const slots<double> &x, int guess, const slots<float> &kout, int wk)
 {
+    hop_tiles tl;
+    if (use_tiles(R, &tl)) {
+        const int64_t nsb = (int64_t)tl.ntx * tl.nty * tl.nzr;
+        const tile_rhs op = {psi, y, x, kout, g_ws.cpar, g_ws.cpar + NSLOTS, g_ws.spart, nsb, guess, wk};
+        hipLaunchKernelGGL((k_hop_tile<RL, double, tile_rhs>), tile_grid(tl), dim3(HT_THREADS), 0, stream(), u, op, R,
+                           lat().g, tl);
+        return nsb;
+    }
     const int nc = shape().nc64;
     const lf_map mp = cn_map(R, nc);
     NC_DISPATCH(nc, hipLaunchKernelGGL((k_cn_rhs<NCV, RL>), dim3(grid_of(mp)), dim3(mp.bs), 0, stream(), u, psi, y, x,

@@ -153,6 +153,44 @@ def test_every_cn_shape_matches_oracle(nrq, oracle, lattice):
         nrq.nrqcd_finalize()
 
 
+@pytest.mark.parametrize("ext,prec", [
+    ((17, 17, 64), 64),  # a last tile of one column and of one row
+    ((48, 6, 61), 32),   # whole tiles along x, half tiles along y, a last run of fewer planes
+    ((18, 13, 41), 64),
+    ((64, 4, 65), 32),   # one row of tiles: a tile is its own y neighbour
+])
+def test_lds_tiles_match_wave_items(nrq, lattice, ext, prec):
+    """Lattices that the CN kernels take through LDS tiles: random propagators
+    (24 fields) with every solver equal the wave items' result (both solve to
+    true relative residual 1e-12, so 1e-10 as above)."""
+    lattice(ext, (0.05, 1.0, 0.9, 1.1))
+    vol = ext[0] * ext[1] * ext[2]
+    rng = np.random.default_rng(5)
+    g = nrq.GaugeConfiguration(prec)
+    g.upload(None, 0.1 * rng.normal(size=(8, 3, vol)))
+    g.Update(1.0, 10)
+    prop = [rng.normal(size=(6, 6, vol)) + 1j * rng.normal(size=(6, 6, vol)) for _ in range(2)]
+    default = nrq.cn_get_shape()
+    nrq.nrqcd_init(1.0, C1, 1.0, 1e-12)
+    try:
+        for kind in ("GMRES_FP64", "GMRES_MIXED", "CHEBYSHEV_FP64", "CHEBYSHEV_MIXED"):
+            _say(f"LDS tiles on {ext}, {prec}-bit links, {kind}")
+            nrq.nrqcd_set_solver(getattr(nrq, "NRQ_SOLVER_" + kind), 30, 10000)
+            got = []
+            for shape in (default, (2, 4, 3, 1)):
+                nrq.cn_set_shape(*shape)
+                h = nrq.NRQCDField()
+                h.upload(*prop)
+                assert h.Update(g, 1.0, C1).max_true_relres <= 1e-12
+                got.append(h.download())
+            assert default == (2, 4, 4, 8)
+            for a, b in zip(*got):
+                assert _rel(a, b) < 1e-10
+    finally:
+        nrq.cn_set_shape(*default)
+        nrq.nrqcd_finalize()
+
+
 def test_batch_graph_follows_a_change_of_spacings(nrq, lattice, monkeypatch):
     """The hipGraph of a batched leapfrog carries the lattice by value.  After
     the lattice module is re-initialised with the same extents and other
