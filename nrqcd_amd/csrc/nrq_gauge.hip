@@ -413,19 +413,43 @@ constexpr int NOBS = 5; // E-field energy, magnetic energy, sum Re Tr P/3, gauss
 // part of G(x) and one plaquette plane ((0,1), (1,2), (0,2) for i = 0, 1, 2);
 // the three parts of G(x) meet in LDS and are added in direction order
 // before the maximum is taken.  One thread per site would hold three
-// directions' links at once (over 256 registers, one wave per SIMD).
+// directions' links at once (over 256 registers, one wave per SIMD).  128^3 FP32
+// 375 us (693 before the XCD order, with two wavefronts per SIMD), 64^3 FP64
+// 63 us (93).
 constexpr int OBS_SITES = 64;
 constexpr int OBS_THREADS = 3 * OBS_SITES;
+
+// A stored link in FP64, formed here and not further up: the scheduling fence
+// keeps the next product's loads from being hoisted over the previous product
+// (with all of a site's links in flight the kernel takes 246 registers and two
+// wavefronts per SIMD; with one product's at a time 140 and three).
 template <typename R>
-__global__ __launch_bounds__(OBS_THREADS) void k_obs(const cplx<R> *__restrict__ u, const R *__restrict__ ef, geom g,
-                                                     double *__restrict__ partials)
+__device__ __forceinline__ mat3<double> obs_link(const cplx<R> *__restrict__ u, int64_t vol, int dir, int64_t s)
+{
+    __builtin_amdgcn_sched_barrier(0);
+    mat3<double> m;
+    const cplx<R> *p = u + (int64_t)dir * 9 * vol;
+#pragma unroll
+    for (int e = 0; e < 9; ++e) {
+        const cplx<R> a = *at32(p + (int64_t)e * vol, (uint32_t)s);
+        m.m[e] = {(double)a.re, (double)a.im};
+    }
+    return m;
+}
+
+template <typename R>
+__global__ __launch_bounds__(OBS_THREADS, 3) void k_obs(const cplx<R> *__restrict__ u, const R *__restrict__ ef, geom g,
+                                                        double *__restrict__ partials)
 {
     double acc[NOBS] = {0, 0, 0, 0, 0};
     const double a0 = g.a[0];
-    const int lane = threadIdx.x & 63, i = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, i = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     __shared__ cplx<double> gpart[3][9][OBS_SITES];
     const int pi = i == 2 ? 0 : i, pj = i == 0 ? 1 : 2; // plaquette plane of this thread
-    for (int64_t base = (int64_t)blockIdx.x * OBS_SITES; base < g.vol; base += (int64_t)gridDim.x * OBS_SITES) {
+    // at any time an XCD works on one contiguous range of sites, so that the
+    // neighbours' links are found in its L2
+    const int64_t first = (int64_t)xcd_block(gridDim.x, 8) * OBS_SITES;
+    for (int64_t base = first; base < g.vol; base += (int64_t)gridDim.x * OBS_SITES) {
         const int64_t s = base + lane;
         const bool in = s < g.vol;
         if (in) {
@@ -434,60 +458,61 @@ __global__ __launch_bounds__(OBS_THREADS) void k_obs(const cplx<R> *__restrict__
             double ed[8], en[8];
             const int64_t sm = site_dn(g, p, i).s;
             double esq = 0;
+#pragma unroll
             for (int a = 0; a < 8; ++a) {
-                ed[a] = (double)ef[((int64_t)i * 8 + a) * g.vol + s];
-                en[a] = (double)ef[((int64_t)i * 8 + a) * g.vol + sm];
+                ed[a] = (double)*at32(ef + ((int64_t)i * 8 + a) * g.vol, (uint32_t)s);
+                en[a] = (double)*at32(ef + ((int64_t)i * 8 + a) * g.vol, (uint32_t)sm);
                 const double v = ed[a] / ai / a0;
                 esq += v * v;
             }
             acc[0] += esq / 2.0;
-            mat3<double> um;
             {
-                mat3<R> t = load_link(u, g.vol, i, sm);
-                for (int m = 0; m < 9; ++m) um.m[m] = {(double)t.m[m].re, (double)t.m[m].im};
-            }
-            // M = E_i(x) - U_i(x-i)^+ E_i(x-i) U_i(x-i)   (algebra matrices)
-            mat3<double> emat = algebra_matrix(ed);
-            mat3<double> t = mul(mul_dn(um, algebra_matrix(en)), um);
-            mat3<double> dm;
-            for (int m = 0; m < 9; ++m) dm.m[m] = emat.m[m] - t.m[m];
-            // reference Gauss deviation: D = M / a_i^2 / a0, sum_a 2|Im Tr(T^a D)|
-            {
+                const mat3<double> um = obs_link(u, g.vol, i, sm);
+                // M = E_i(x) - U_i(x-i)^+ E_i(x-i) U_i(x-i)   (algebra matrices)
+                const mat3<double> emat = algebra_matrix(ed);
+                const mat3<double> t = mul(mul_dn(um, algebra_matrix(en)), um);
+                mat3<double> dm;
+#pragma unroll
+                for (int m = 0; m < 9; ++m) dm.m[m] = emat.m[m] - t.m[m];
+                // reference Gauss deviation: D = M / a_i^2 / a0, sum_a 2|Im Tr(T^a D)|
                 mat3<double> d;
                 const double sc = 1.0 / (ai * ai) / a0;
+#pragma unroll
                 for (int m = 0; m < 9; ++m) d.m[m] = sc * dm.m[m];
                 double tt[8];
                 two_im_trace_gen(d, tt);
+#pragma unroll
                 for (int a = 0; a < 8; ++a) acc[3] += fabs(tt[a]);
+#pragma unroll
+                for (int m = 0; m < 9; ++m) gpart[i][m][lane] = (1.0 / ai) * dm.m[m];
             }
-            for (int m = 0; m < 9; ++m) gpart[i][m][lane] = (1.0 / ai) * dm.m[m];
-            // magnetic part: plaquette P_{pi pj}
+            // magnetic part: Re Tr of the plaquette P_{pi pj}, the last product
+            // as a sum over its elements
             const int64_t xi = site_up(g, p, pi).s, xj = site_up(g, p, pj).s;
-            mat3<double> l1, l2, l3, l4;
-            {
-                mat3<R> a1 = load_link(u, g.vol, pi, s), a2 = load_link(u, g.vol, pj, xi);
-                mat3<R> a3 = load_link(u, g.vol, pi, xj), a4 = load_link(u, g.vol, pj, s);
-                for (int m = 0; m < 9; ++m) {
-                    l1.m[m] = {(double)a1.m[m].re, (double)a1.m[m].im};
-                    l2.m[m] = {(double)a2.m[m].re, (double)a2.m[m].im};
-                    l3.m[m] = {(double)a3.m[m].re, (double)a3.m[m].im};
-                    l4.m[m] = {(double)a4.m[m].re, (double)a4.m[m].im};
-                }
+            mat3<double> w = obs_link(u, g.vol, pi, s);
+            w = mul(w, obs_link(u, g.vol, pj, xi));
+            w = mul_nd(w, obs_link(u, g.vol, pi, xj));
+            const mat3<double> l4 = obs_link(u, g.vol, pj, s);
+            double tr = 0;
+#pragma unroll
+            for (int m = 0; m < 9; ++m) {
+                tr = fmx(w.m[m].re, l4.m[m].re, tr);
+                tr = fmx(w.m[m].im, l4.m[m].im, tr);
             }
-            mat3<double> pl = mul_nd(mul_nd(mul(l1, l2), l3), l4);
-            const double tr = trace(pl).re;
             acc[1] += 2.0 * 3.0 * (1.0 - tr / 3.0) / g.a[pi + 1] / g.a[pj + 1];
             acc[2] += tr / 3.0;
         }
         __syncthreads();
         if (in && i == 0) {
             mat3<double> gsum;
+#pragma unroll
             for (int m = 0; m < 9; ++m) {
                 const cplx<double> v = gpart[0][m][lane] + gpart[1][m][lane];
                 gsum.m[m] = (1.0 / a0) * (v + gpart[2][m][lane]);
             }
             double tt[8];
             two_re_trace_gen(gsum, tt);
+#pragma unroll
             for (int a = 0; a < 8; ++a) acc[4] = fmax(acc[4], fabs(tt[a]));
         }
         __syncthreads();
