@@ -232,23 +232,32 @@ __global__ __launch_bounds__(GF_THREADS) void k_gf_apply(cplx<R> *__restrict__ u
 // ---------------------------------------------------------------------------
 
 // The 24 real fields, two per complex plane (components 2q, 2q + 1 of
-// direction i in plane q + 4 i): AA (which = 0) or EE (which = 1)
+// direction i = blockIdx.y in plane q + 4 i): A^a_i = GetGroupLog(U_i)^a / a_i,
+// one thread per (site, direction).
 template <typename R>
-__global__ __launch_bounds__(GF_THREADS) void k_corr_fields(const cplx<R> *__restrict__ u, const R *__restrict__ ef, geom g,
-                                                          int which, cplx<double> *__restrict__ fld)
+__global__ __launch_bounds__(GF_THREADS) void k_aa_fields(const cplx<R> *__restrict__ u, geom g, cplx<double> *__restrict__ fld)
 {
     const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = blockIdx.y;
     if (s >= g.vol) return;
-    for (int i = 0; i < 3; ++i) {
-        double c[8];
-        if (which == 0) {
-            group_log_coords(load_link_d(u, g.vol, i, s), c);
-            for (int a = 0; a < 8; ++a) c[a] = c[a] / g.a[i + 1];
-        } else {
-            for (int a = 0; a < 8; ++a) c[a] = (double)ef[((int64_t)i * 8 + a) * g.vol + s] / g.a[i + 1] / g.a[0];
-        }
-        for (int q = 0; q < 4; ++q) fld[(int64_t)(q + 4 * i) * g.vol + s] = {c[2 * q], c[2 * q + 1]};
-    }
+    double c[8];
+    group_log_coords(load_link_d(u, g.vol, i, s), c);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) fld[(int64_t)(q + 4 * i) * g.vol + s] = {c[2 * q] / g.a[i + 1], c[2 * q + 1] / g.a[i + 1]};
+}
+
+// The same of E^a_i / (a_i a0): a copy, one thread per site and plane
+// (blockIdx.y).  One thread for all 24 values of a site, with the logarithm's
+// registers, ran at a quarter of the bandwidth (128^3 FP32 479 us).
+template <typename R>
+__global__ __launch_bounds__(GF_THREADS) void k_ee_fields(const R *__restrict__ ef, geom g, cplx<double> *__restrict__ fld)
+{
+    const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int pl = blockIdx.y, i = pl >> 2, q = pl & 3; // plane q + 4 i
+    if (s >= g.vol) return;
+    const R *e = ef + ((int64_t)i * 8 + 2 * q) * g.vol;
+    const double c0 = (double)*at32(e, (uint32_t)s), c1 = (double)*at32(e + g.vol, (uint32_t)s);
+    fld[(int64_t)pl * g.vol + s] = {c0 / g.a[i + 1] / g.a[0], c1 / g.a[i + 1] / g.a[0]};
 }
 
 // out[s] = Re sum_a sum_ij F^a_i P_ij conj(F^a_j) * scale, scale = fwd^2 / (8 V_phys),
@@ -356,17 +365,11 @@ static double max_momentum(const geom &g)
     return std::sqrt(sum);
 }
 
-// Device buffers of one call, freed on every exit path.
-struct gf_buffers {
-    cplx<double> *fld = nullptr;
-    double *partial = nullptr, *rows = nullptr, *hmax = nullptr;
+// Events of one call, released on every exit path.
+struct gf_events {
     hipEvent_t ev[2] = {nullptr, nullptr};
-    ~gf_buffers()
+    ~gf_events()
     {
-        if (fld) (void)hipFree(fld);
-        if (partial) (void)hipFree(partial);
-        if (rows) (void)hipFree(rows);
-        if (hmax) (void)hipHostFree(hmax);
         for (hipEvent_t e : ev)
             if (e) (void)hipEventDestroy(e);
     }
@@ -408,13 +411,11 @@ static int gaugefix_t(nrq_gauge *h, double tol, double alpha, int64_t maxit, int
     const geom g = lat().g;
     const int64_t v = g.vol;
     const unsigned nblk = (unsigned)((v + GF_THREADS - 1) / GF_THREADS);
-    gf_buffers b;
-    if (hipMalloc((void **)&b.fld, sizeof(cplx<double>) * GF_PLANES * (size_t)v) != hipSuccess ||
-        hipMalloc((void **)&b.rows, sizeof(double) * 3 * MAXROW) != hipSuccess ||
-        hipHostMalloc((void **)&b.hmax, sizeof(double) * 2, hipHostMallocDefault) != hipSuccess) {
-        (void)hipGetLastError();
-        return fail(NRQ_ERR_ALLOC, "gauge fixing: device allocation failed (V=%lld)", (long long)v);
-    }
+    // -i Delta (80 B per site) in the link buffer that the next leapfrog pass
+    // overwrites, the maxima in the handle's reduction buffers: no allocation
+    cplx<double> *fld = (cplx<double> *)h->u[h->cur ^ 1];
+    double *rows = (double *)h->partials, *hmax = h->result;
+    gf_events b;
     for (hipEvent_t &e : b.ev) NRQ_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     hipfftHandle plan = 0;
     if (int e = gf_plan(g, GF_PLANES, &plan)) return e;
@@ -424,11 +425,11 @@ static int gaugefix_t(nrq_gauge *h, double tol, double alpha, int64_t maxit, int
     const double pmax = max_momentum(g);
     // row n % 3 holds the divergence maximum before transformation n; the fold
     // of row n clears that of n + 1, last read by transformation n - 2
-    auto row = [&](int64_t n) { return b.rows + (n % 3) * MAXROW; };
-    NRQ_HIP(hipMemsetAsync(b.rows, 0, sizeof(double) * 3 * MAXROW, stream()));
+    auto row = [&](int64_t n) { return rows + (n % 3) * MAXROW; };
+    NRQ_HIP(hipMemsetAsync(rows, 0, sizeof(double) * 3 * MAXROW, stream()));
     auto measure = [&](int64_t n) -> int {
-        hipLaunchKernelGGL(k_gf_divergence<R>, dim3(nblk), dim3(GF_THREADS), 0, stream(), u, g, b.fld, row(n));
-        hipLaunchKernelGGL(k_gf_fold_max, dim3(1), dim3(MAXROW), 0, stream(), row(n), row(n + 1), b.hmax + (n & 1));
+        hipLaunchKernelGGL(k_gf_divergence<R>, dim3(nblk), dim3(GF_THREADS), 0, stream(), u, g, fld, row(n));
+        hipLaunchKernelGGL(k_gf_fold_max, dim3(1), dim3(MAXROW), 0, stream(), row(n), row(n + 1), hmax + (n & 1));
         NRQ_HIP(hipGetLastError());
         NRQ_HIP(hipEventRecord(b.ev[n & 1], stream()));
         return NRQ_OK;
@@ -443,18 +444,18 @@ static int gaugefix_t(nrq_gauge *h, double tol, double alpha, int64_t maxit, int
     for (int64_t done = 0;; ++done) {
         while (enqueued < maxit && enqueued <= done) {
             const int64_t n = enqueued;
-            hipfftResult fr = hipfftExecZ2Z(plan, (hipfftDoubleComplex *)b.fld, (hipfftDoubleComplex *)b.fld, HIPFFT_FORWARD);
+            hipfftResult fr = hipfftExecZ2Z(plan, (hipfftDoubleComplex *)fld, (hipfftDoubleComplex *)fld, HIPFFT_FORWARD);
             if (fr != HIPFFT_SUCCESS) return gf_fft_fail(fr, "exec (forward)");
-            hipLaunchKernelGGL(k_gf_accelerate, dim3(nblk), dim3(GF_THREADS), 0, stream(), b.fld, g, pmax, fwd * bwd * alpha);
-            fr = hipfftExecZ2Z(plan, (hipfftDoubleComplex *)b.fld, (hipfftDoubleComplex *)b.fld, HIPFFT_BACKWARD);
+            hipLaunchKernelGGL(k_gf_accelerate, dim3(nblk), dim3(GF_THREADS), 0, stream(), fld, g, pmax, fwd * bwd * alpha);
+            fr = hipfftExecZ2Z(plan, (hipfftDoubleComplex *)fld, (hipfftDoubleComplex *)fld, HIPFFT_BACKWARD);
             if (fr != HIPFFT_SUCCESS) return gf_fft_fail(fr, "exec (backward)");
-            hipLaunchKernelGGL(k_gf_apply<R>, dim3(nblk), dim3(GF_THREADS), 0, stream(), u, b.fld, g, row(n), tol);
+            hipLaunchKernelGGL(k_gf_apply<R>, dim3(nblk), dim3(GF_THREADS), 0, stream(), u, fld, g, row(n), tol);
             // n + 1 uses the event and host slot of n - 1, which the host has read
             if (int e = measure(n + 1)) return e;
             ++enqueued;
         }
         NRQ_HIP(hipEventSynchronize(b.ev[done & 1]));
-        dev = *(volatile double *)(b.hmax + (done & 1));
+        dev = *(volatile double *)(hmax + (done & 1));
         if (!std::isfinite(dev)) return fail(NRQ_ERR_NOCONV, "gauge fixing: non-finite divergence");
         if (dev <= tol || done >= maxit) {
             if (iterations) *iterations = done;
@@ -488,14 +489,11 @@ template <typename R> static int correlators_t(const nrq_gauge *h, double *aa, d
     const geom g = lat().g;
     const int64_t v = g.vol;
     const unsigned nblk = (unsigned)((v + GF_THREADS - 1) / GF_THREADS);
-    gf_buffers b;
-    double *dout = nullptr;
-    if (hipMalloc((void **)&b.fld, sizeof(cplx<double>) * CORR_PLANES * (size_t)v) != hipSuccess ||
-        hipMalloc((void **)&b.partial, sizeof(double) * (size_t)v) != hipSuccess) {
-        (void)hipGetLastError();
-        return fail(NRQ_ERR_ALLOC, "correlators: device allocation failed (V=%lld)", (long long)v);
-    }
-    dout = b.partial;
+    // the planes and the result (200 B per site) in the link buffer that the
+    // next leapfrog pass overwrites (216 B per site in FP32): no allocation
+    static_assert(CORR_PLANES * sizeof(cplx<double>) + sizeof(double) <= 27 * sizeof(cplx<R>) || sizeof(R) == 8, "scratch");
+    cplx<double> *fld = (cplx<double> *)h->u[h->cur ^ 1];
+    double *dout = (double *)(fld + (int64_t)CORR_PLANES * v);
     hipfftHandle plan = 0;
     if (int e = gf_plan(g, CORR_PLANES, &plan)) return e;
     const double fwd = g.a[1] * g.a[2] * g.a[3];
@@ -506,11 +504,14 @@ template <typename R> static int correlators_t(const nrq_gauge *h, double *aa, d
     for (int which = 0; which < 2; ++which) {
         double *host = which == 0 ? aa : ee;
         if (!host) continue;
-        hipLaunchKernelGGL(k_corr_fields<R>, dim3(nblk), dim3(GF_THREADS), 0, stream(), u, ef, g, which, b.fld);
+        if (which == 0)
+            hipLaunchKernelGGL(k_aa_fields<R>, dim3(nblk, 3), dim3(GF_THREADS), 0, stream(), u, g, fld);
+        else
+            hipLaunchKernelGGL(k_ee_fields<R>, dim3(nblk, CORR_PLANES), dim3(GF_THREADS), 0, stream(), ef, g, fld);
         NRQ_HIP(hipGetLastError());
-        hipfftResult fr = hipfftExecZ2Z(plan, (hipfftDoubleComplex *)b.fld, (hipfftDoubleComplex *)b.fld, HIPFFT_FORWARD);
+        hipfftResult fr = hipfftExecZ2Z(plan, (hipfftDoubleComplex *)fld, (hipfftDoubleComplex *)fld, HIPFFT_FORWARD);
         if (fr != HIPFFT_SUCCESS) return gf_fft_fail(fr, "exec (forward)");
-        hipLaunchKernelGGL(k_corr_project_packed, dim3(nblk), dim3(GF_THREADS), 0, stream(), b.fld, g, scale, dout);
+        hipLaunchKernelGGL(k_corr_project_packed, dim3(nblk), dim3(GF_THREADS), 0, stream(), fld, g, scale, dout);
         NRQ_HIP(hipGetLastError());
         NRQ_HIP(hipMemcpyAsync(host, dout, sizeof(double) * (size_t)v, hipMemcpyDeviceToHost, stream()));
         NRQ_HIP(hipStreamSynchronize(stream()));

@@ -69,7 +69,9 @@ struct scratch_buf {
 struct nrq_gauge {
     int precision = 64;       // 64: double storage, 32: float storage
     int64_t vol = 0;
-    void *u[2] = {nullptr, nullptr}; // ping-pong link buffers [dir][elem][site] complex
+    // ping-pong link buffers [dir][elem][site] complex; u[cur ^ 1] holds nothing
+    // between calls (a leapfrog pass writes it whole), so calls use it as scratch
+    void *u[2] = {nullptr, nullptr};
     int cur = 0;              // which u[] holds the current links
     void *e = nullptr;        // E field [dir][a][site] real
     void *partials = nullptr; // reduction partials
