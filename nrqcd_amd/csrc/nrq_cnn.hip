@@ -11,10 +11,8 @@
 // commutes with the scale of its input.
 //
 // Convolutions are implicit GEMMs on BF16 matrix cores with FP32
-// accumulation: a wavefront computes eight runs of 16 consecutive sites x 32
-// output channels with one v_mfma_f32_16x16x32_bf16 per (run, tap, 16 output
-// channels), each tap's weights loaded once for the eight runs;
-// K = 32 input channels per tap.  Activations are channels-last BF16
+// accumulation, one v_mfma_f32_16x16x32_bf16 per (16 sites, tap, 16 output
+// channels), K = 32 input channels per tap (k_conv).  Activations are channels-last BF16
 // [site][32] (channels past 18 are zero in the outer layers), weights
 // [layer][tap][co][ci] with tap = 9 (dz+1) + 3 (dy+1) + (dx+1).  Backward:
 // d(input) is the same convolution with mirrored, transposed weights; the
@@ -22,10 +20,12 @@
 // the same matrix cores.  Adam updates FP32 master weights.
 #include "nrq_cnn.h"
 #include "nrq_krylov.h"
+#include "nrq_map.h"
 #include <algorithm>
 #include <cmath>
 #include <complex>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 using namespace nrq;
@@ -40,6 +40,9 @@ constexpr int DW_SITES = 4096;       // sites per block of the weight-gradient k
 typedef uint16_t bf16;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
+typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
 
 __host__ __device__ inline bf16 f2bf(float f)
 {
@@ -58,189 +61,172 @@ __host__ __device__ inline float bf2f(bf16 h)
 
 __device__ __forceinline__ int wrap(int a, int n) { return a < 0 ? a + n : (a >= n ? a - n : a); }
 
-// out[s][co] = sum_{tap, ci} w[tap][co][ci] in[s + off(tap)][ci] for one
-// layer.  out_f != null: FP32 output; else BF16 output, with ReLU when relu,
-// and zeroed where mask[s][co] <= 0 when mask != null (the ReLU derivative of
-// the backward pass).  Grid: 4 wavefronts per block; a wavefront computes
-// CONV_SEG consecutive 16-site x runs (in x, then y, then z order) and loads
-// each tap's weights once for all of them.
-constexpr int CONV_SEG = 8;
-__global__ __launch_bounds__(256) void k_conv(const bf16 *__restrict__ in, const bf16 *__restrict__ w,
-                                              bf16 *__restrict__ out_b, float *__restrict__ out_f,
-                                              const bf16 *__restrict__ mask, int relu, geom g)
-{
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int nsx = g.n0 >> 4;
-    const int64_t nseg = (int64_t)nsx * g.n1 * g.n2;
-    const int64_t seg0 = ((int64_t)blockIdx.x * 4 + wv) * CONV_SEG;
-    if (seg0 >= nseg) return;
-    const int m = lane & 15, kq = lane >> 4;
-    int xs[CONV_SEG], ys[CONV_SEG], zs[CONV_SEG];
-#pragma unroll
-    for (int j = 0; j < CONV_SEG; ++j) {
-        const int64_t sg = seg0 + j < nseg ? seg0 + j : seg0; // a run past the end repeats the first
-        xs[j] = (int)(sg % nsx);
-        const int64_t yz = sg / nsx;
-        ys[j] = (int)(yz % g.n1);
-        zs[j] = (int)(yz / g.n1);
-    }
-    f32x4 acc0[CONV_SEG], acc1[CONV_SEG];
-#pragma unroll
-    for (int j = 0; j < CONV_SEG; ++j) acc0[j] = acc1[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    int tap = 0;
-    for (int dz = -1; dz <= 1; ++dz)
-        for (int dy = -1; dy <= 1; ++dy)
-            for (int dx = -1; dx <= 1; ++dx, ++tap) {
-                // B[k][n] = w[tap][co n][ci k], shared by the runs
-                const bf16x8 b0 = *(const bf16x8 *)(w + ((int64_t)tap * CH + m) * CH + 8 * kq);
-                const bf16x8 b1 = *(const bf16x8 *)(w + ((int64_t)tap * CH + 16 + m) * CH + 8 * kq);
-#pragma unroll
-                for (int j = 0; j < CONV_SEG; ++j) {
-                    const int xx = wrap(xs[j] * 16 + m + dx, g.n0);
-                    const int yy = wrap(ys[j] + dy, g.n1), zz = wrap(zs[j] + dz, g.n2);
-                    const int64_t nb = xx + (int64_t)g.n0 * (yy + (int64_t)g.n1 * zz);
-                    // A[m][k] = in[site m][ci k]
-                    const bf16x8 a = *(const bf16x8 *)(in + nb * CH + 8 * kq);
-                    acc0[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b0, acc0[j], 0, 0, 0);
-                    acc1[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b1, acc1[j], 0, 0, 0);
-                }
-            }
-    // lane holds D[site 4 kq + i][co m] and D[site 4 kq + i][co 16 + m] of each run
-#pragma unroll
-    for (int j = 0; j < CONV_SEG; ++j) {
-        if (seg0 + j >= nseg) break;
-        const int64_t base = (int64_t)xs[j] * 16 + (int64_t)g.n0 * (ys[j] + (int64_t)g.n1 * zs[j]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int64_t s = base + 4 * kq + i;
-            float v0 = acc0[j][i], v1 = acc1[j][i];
-            if (out_f) {
-                out_f[s * CH + m] = v0;
-                out_f[s * CH + 16 + m] = v1;
-            } else {
-                if (relu) {
-                    v0 = fmaxf(v0, 0.f);
-                    v1 = fmaxf(v1, 0.f);
-                }
-                if (mask) {
-                    if (!(bf2f(mask[s * CH + m]) > 0.f)) v0 = 0.f;
-                    if (!(bf2f(mask[s * CH + 16 + m]) > 0.f)) v1 = 0.f;
-                }
-                out_b[s * CH + m] = f2bf(v0);
-                out_b[s * CH + 16 + m] = f2bf(v1);
-            }
-        }
-    }
-}
+// One layer: out[s][co] = sum_{tap, ci} w[tap][co][ci] in[s + off(tap)][ci] for
+// gridDim.y fields of V sites each (n0 a multiple of 16, other extents any).
+// HALVES = 2: all 32 output channels, as FP32 (out_f, [site][32]) or as BF16
+// with ReLU when relu, and zeroed where mask[s][co] <= 0 when mask is not null
+// (the ReLU derivative of the backward pass).  HALVES = 1: the first eight
+// channels as FP32 (out_f, [site][8]), all that the preconditioner uses of the
+// last layer.
+//
+// A block of eight wavefronts owns a tile of 16 XR x 4 (8 / XR) sites of (x, y)
+// and sweeps zc output planes; a wavefront owns 16 x sites by 4 rows of it.  The
+// sweep runs over input planes: plane p adds to the outputs p - 1, p, p + 1,
+// whose accumulators (three sets of 4 rows) stay in registers, so only the plane
+// being read and the next one are in LDS (with a one-site halo, 64 B per site),
+// beside the layer's weights in the lane order of the MFMA operands.  An input
+// row serves the three output rows around it: (6 rows + 6 weights) operands of
+// 1 KB per 24 MFMAs, 128 B per clock and CU, the LDS's rate, where one operand
+// pair per tap, as a kernel that gathers per output has it, needs 192.  Eight
+// rows per wavefront would need 83 B, but with one wavefront per SIMD nothing
+// overlaps the waits (128^3 481 us an apply).  The weights are the A
+// operand and the sites the B operand, so that a lane ends up with four
+// consecutive channels of one site and stores them as 8 (BF16) or 16 bytes.
+// Measured, four layers of one field: 128^3 353 us (1.03 PFLOP/s algorithmic;
+// the sweep this replaces, with a 128 x 2 tile and three planes in LDS, 615 us),
+// 64^3 75 us (a gather from the caches, for extents the sweep did not take,
+// 156 us), 16^3 43 us (89 us).
+constexpr int CV_ROWS = 4, CV_WAVES = 8, CV_TH = 64 * CV_WAVES;
+template <int XR> struct conv_tile {
+    static constexpr int YG = CV_WAVES / XR;
+    static constexpr int TX = 16 * XR, TY = CV_ROWS * YG, HX = TX + 2, HY = TY + 2;
+    static constexpr int PLANE = HX * HY * 4;            // bf16x8 per plane
+    static constexpr int PER = (PLANE + CV_TH - 1) / CV_TH;      // per thread and plane
+};
 
-// k_conv with the input staged in LDS, for lattices with n0 % 128 == 0, even
-// n1 and n2 % ZC == 0: a block of 4 wavefronts owns a 128 x 2 tile of (x, y)
-// and sweeps ZC planes in z.  LDS holds the layer's weights in the lane order
-// of the MFMA B operands (55 KB, read once per block instead of from L2 at
-// every tap) and a ring of three input planes of the tile with a one-site
-// halo (130 x 4 sites x 32 BF16 channels each, 100 KB);
-// output plane z reads planes z - 1, z, z + 1 there instead of re-reading each
-// input site 27 times through L1, while plane z + 2 streams into registers
-// and then replaces plane z - 1.  Wavefront w computes row y0 + (w & 1), x runs
-// 4 (w >> 1) .. 4 (w >> 1) + 3.  Same arguments, same arithmetic and summation
-// order per output as k_conv.
-constexpr int LT_X = 128, LT_HX = LT_X + 2, LT_HY = 4;
-constexpr int LT_PLANE = LT_HX * LT_HY * 4;                     // bf16x8 per plane
-constexpr int LT_PER = (LT_PLANE + 255) / 256;                  // per thread and plane
-template <int ZC>
-__global__ __launch_bounds__(256) void k_conv_lds(const bf16 *__restrict__ in, const bf16 *__restrict__ w,
-                                                  bf16 *__restrict__ out_b, float *__restrict__ out_f,
-                                                  const bf16 *__restrict__ mask, int relu, geom g)
+template <int XR, int HALVES>
+__global__ __launch_bounds__(CV_TH, CV_WAVES / 4) void k_conv(const bf16 *__restrict__ in, const bf16 *__restrict__ w, bf16 *__restrict__ out_b,
+                                                 float *__restrict__ out_f, const bf16 *__restrict__ mask, int relu, geom g,
+                                                 int zc)
 {
-    __shared__ bf16x8 lds[3 * LT_PLANE];
-    // the layer's weights as the MFMA B operands: [tap][half][lane]
-    __shared__ bf16x8 wl[27 * 2 * 64];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    for (int q = threadIdx.x; q < 27 * 2 * 64; q += 256) {
-        const int l = q & 63, hf = (q >> 6) & 1, tp = q >> 7;
+    using C = conv_tile<XR>;
+    __shared__ bf16x8 pl[2][C::PLANE];
+    __shared__ bf16x8 wl[TAPS * HALVES * 64]; // [tap][half][lane]
+    const int t = threadIdx.x, lane = t & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int m = lane & 15, kq = lane >> 4;
+    for (int q = t; q < TAPS * HALVES * 64; q += CV_TH) {
+        const int l = q & 63, hf = HALVES == 2 ? (q >> 6) & 1 : 0, tp = q / (64 * HALVES);
         wl[q] = *(const bf16x8 *)(w + ((int64_t)tp * CH + 16 * hf + (l & 15)) * CH + 8 * (l >> 4));
     }
-    const int ntx = g.n0 / LT_X, nty = g.n1 / 2;
-    const int b = blockIdx.x;
-    const int x0 = (b % ntx) * LT_X, y0 = ((b / ntx) % nty) * 2, z0 = (b / (ntx * nty)) * ZC;
-    bf16x8 pre[LT_PER];
-    auto gload = [&](int z) {
-        const int gz = wrap(z, g.n2);
+    const unsigned ntx = (unsigned)(g.n0 / C::TX), nty = (unsigned)((g.n1 + C::TY - 1) / C::TY);
+    const unsigned lb = xcd_block(gridDim.x, 8);
+    const int x0 = (int)(lb % ntx) * C::TX, y0 = (int)((lb / ntx) % nty) * C::TY, z0 = (int)(lb / (ntx * nty)) * zc;
+    const int nz = g.n2 - z0 < zc ? g.n2 - z0 : zc;
+    const int64_t field = (int64_t)blockIdx.y * g.vol;
+    in += field * CH;
+    const int64_t plane = (int64_t)g.n0 * g.n1;
+
+    // this thread's pieces of a plane: 16 bytes of the site at these offsets
+    int src[C::PER];
 #pragma unroll
-        for (int k = 0; k < LT_PER; ++k) {
-            const int q = threadIdx.x + 256 * k;
-            if (q < LT_PLANE) {
-                const int c4 = q & 3, site = q >> 2;
-                const int hx = site % LT_HX, hy = site / LT_HX;
-                const int gx = wrap(x0 - 1 + hx, g.n0), gy = wrap(y0 - 1 + hy, g.n1);
-                const int64_t gs = gx + (int64_t)g.n0 * (gy + (int64_t)g.n1 * gz);
-                pre[k] = *(const bf16x8 *)(in + gs * CH + 8 * c4);
-            }
-        }
-    };
-    auto sstore = [&](int slot) {
-#pragma unroll
-        for (int k = 0; k < LT_PER; ++k) {
-            const int q = threadIdx.x + 256 * k;
-            if (q < LT_PLANE) lds[slot * LT_PLANE + q] = pre[k];
-        }
-    };
-    for (int p = 0; p < 3; ++p) {
-        gload(z0 - 1 + p);
-        sstore(p);
+    for (int k = 0; k < C::PER; ++k) {
+        const int q = t + CV_TH * k < C::PLANE ? t + CV_TH * k : t;
+        const int site = q >> 2, hx = site % C::HX, hy = site / C::HX;
+        const int gx = (x0 - 1 + hx + g.n0) % g.n0, gy = (y0 - 1 + hy + g.n1) % g.n1;
+        src[k] = (gx + g.n0 * gy) * 4 + (q & 3);
     }
+    bf16x8 pre[C::PER];
+    auto load = [&](int z) {
+        const bf16x8 *b = (const bf16x8 *)in + 4 * plane * ((z + g.n2) % g.n2);
+#pragma unroll
+        for (int k = 0; k < C::PER; ++k) pre[k] = b[src[k]];
+    };
+    auto store = [&](int buf) {
+#pragma unroll
+        for (int k = 0; k < C::PER; ++k)
+            if (t + CV_TH * k < C::PLANE) pl[buf][t + CV_TH * k] = pre[k];
+    };
+    const int xr = wv % XR, yg = wv / XR;
+    const bool on = y0 + CV_ROWS * yg < g.n1;
+    f32x4 acc[3][CV_ROWS][HALVES];
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+        for (int r = 0; r < CV_ROWS; ++r)
+#pragma unroll
+            for (int h = 0; h < HALVES; ++h) acc[a][r][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+    load(z0 - 1);
+    store(0);
     __syncthreads();
-    const int m = lane & 15, kq = lane >> 4;
-    const int ry = wv & 1, xr0 = 4 * (wv >> 1);
-#pragma unroll 1
-    for (int kz = 0; kz < ZC; ++kz) {
-        const bool more = kz + 1 < ZC;
-        if (more) gload(z0 + kz + 2);
-        f32x4 acc0[4], acc1[4];
+    // input plane z0 - 1 + k; accumulator set (k + j) % 3 belongs to the output
+    // plane z0 - 2 + k + j (j = 0, 1, 2: the input is its plane dz = 1, 0, -1)
+    auto step = [&](auto kc, int k) {
+        constexpr int K = decltype(kc)::value;
+        if (k < nz + 1) load(z0 + k);
+        if (on) {
+            const bf16x8 *X = pl[k & 1] + ((CV_ROWS * yg) * C::HX + 16 * xr + m) * 4 + kq;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc0[j] = acc1[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-        int tap = 0;
-        for (int dz = -1; dz <= 1; ++dz) {
-            const int slot = (kz + 1 + dz) % 3; // slots hold planes z0 - 1 + p at p mod 3
-            for (int dy = -1; dy <= 1; ++dy)
-                for (int dx = -1; dx <= 1; ++dx, ++tap) {
-                    const bf16x8 b0 = wl[(tap * 2 + 0) * 64 + lane];
-                    const bf16x8 b1 = wl[(tap * 2 + 1) * 64 + lane];
-                    const bf16x8 *row = lds + slot * LT_PLANE + ((ry + dy + 1) * LT_HX + 16 * xr0 + m + dx + 1) * 4 + kq;
+            for (int j = 0; j < 3; ++j) {
+                const int o = k - 2 + j; // output plane - z0
+                if (o < 0 || o >= nz) continue;
+                const int dz = 2 - j; // tap index of the plane
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const bf16x8 a = row[16 * j * 4];
-                        acc0[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b0, acc0[j], 0, 0, 0);
-                        acc1[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b1, acc1[j], 0, 0, 0);
+                for (int dx = 0; dx < 3; ++dx) {
+                    bf16x8 wf[3][HALVES];
+#pragma unroll
+                    for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+                        for (int h = 0; h < HALVES; ++h) wf[dy][h] = wl[((9 * dz + 3 * dy + dx) * HALVES + h) * 64 + lane];
+#pragma unroll
+                    for (int r = 0; r < CV_ROWS + 2; ++r) {
+                        const bf16x8 x = X[(r * C::HX + dx) * 4];
+#pragma unroll
+                        for (int dy = 0; dy < 3; ++dy) {
+                            const int y = r - dy;
+                            if (y < 0 || y >= CV_ROWS) continue;
+#pragma unroll
+                            for (int h = 0; h < HALVES; ++h)
+                                acc[(K + j) % 3][y][h] =
+                                    __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[dy][h], x, acc[(K + j) % 3][y][h], 0, 0, 0);
+                        }
                     }
-                }
-        }
-        const int64_t base = x0 + 16 * xr0 + (int64_t)g.n0 * ((y0 + ry) + (int64_t)g.n1 * (z0 + kz));
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int64_t s = base + 16 * j + 4 * kq + i;
-                float v0 = acc0[j][i], v1 = acc1[j][i];
-                if (out_f) {
-                    out_f[s * CH + m] = v0;
-                    out_f[s * CH + 16 + m] = v1;
-                } else {
-                    if (relu) {
-                        v0 = fmaxf(v0, 0.f);
-                        v1 = fmaxf(v1, 0.f);
-                    }
-                    if (mask) {
-                        if (!(bf2f(mask[s * CH + m]) > 0.f)) v0 = 0.f;
-                        if (!(bf2f(mask[s * CH + 16 + m]) > 0.f)) v1 = 0.f;
-                    }
-                    out_b[s * CH + m] = f2bf(v0);
-                    out_b[s * CH + 16 + m] = f2bf(v1);
                 }
             }
-        __syncthreads(); // plane z - 1 is no longer read
-        if (more) sstore(kz % 3);
+        }
+        // output plane z0 - 2 + k is complete: lane holds channels 4 kq + i of site m of each row
+        if (k >= 2) {
+#pragma unroll
+            for (int r = 0; r < CV_ROWS; ++r) {
+                const int y = y0 + CV_ROWS * yg + r;
+                const int64_t s = field + x0 + 16 * xr + m + (int64_t)g.n0 * y + plane * (z0 + k - 2);
+#pragma unroll
+                for (int h = 0; h < HALVES; ++h) {
+                    f32x4 v = acc[K % 3][r][h];
+                    acc[K % 3][r][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    if (y >= g.n1) continue;
+                    if constexpr (HALVES == 1) {
+                        if (kq < 2) *(f32x4 *)(out_f + s * 8 + 4 * kq) = v;
+                    } else if (out_f) {
+                        *(f32x4 *)(out_f + s * CH + 16 * h + 4 * kq) = v;
+                    } else {
+                        const int64_t at = s * CH + 16 * h + 4 * kq;
+                        if (relu)
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) v[i] = fmaxf(v[i], 0.f);
+                        if (mask) {
+                            const u16x4 mk = *(const u16x4 *)(mask + at);
+#pragma unroll
+                            for (int i = 0; i < 4; ++i)
+                                if (!(bf2f(mk[i]) > 0.f)) v[i] = 0.f;
+                        }
+                        bf16x4 o; // round to nearest even, as f2bf
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) o[i] = (__bf16)v[i];
+                        *(bf16x4 *)(out_b + at) = o;
+                    }
+                }
+            }
+        }
+        // one barrier a plane: the buffer written here was last read before the previous one
+        if (k < nz + 1) store((k + 1) & 1);
         __syncthreads();
+    };
+#pragma unroll 1
+    for (int k = 0; k < nz + 2; k += 3) {
+        step(std::integral_constant<int, 0>(), k);
+        if (k + 1 < nz + 2) step(std::integral_constant<int, 1>(), k + 1);
+        if (k + 2 < nz + 2) step(std::integral_constant<int, 2>(), k + 2);
     }
 }
 
@@ -395,41 +381,62 @@ __device__ __forceinline__ cplx<double> cmuld(cplx<double> a, cplx<double> b)
     return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
 }
 
-// BF16 network input of one colour field v (complex colour-major, 3V) and
-// its features f1 = beta K v, f2 = beta K f1: channel 6 q + 2 c + {re, im}
-// of feature q (v, f1 s1, f2 s2) and colour c; channels >= 18 zero.
+// Columns of one batched network pass.
+constexpr int PC_COLS = 12;
+template <typename T> struct pc_cols {
+    const cplx<T> *v[PC_COLS], *f1[PC_COLS], *f2[PC_COLS];
+    cplx<T> *z[PC_COLS];
+    col_scale sc[PC_COLS];
+};
+
+// BF16 network input of colour field blockIdx.y: v (complex colour-major, 3V)
+// and its features f1 = beta K v, f2 = beta K f1; channel 6 q + 2 c + {re, im}
+// of feature q (v, f1 s1, f2 s2) and colour c, channels >= 18 zero.  A lane
+// writes its site's 64 bytes as four vectors.
 template <typename T>
-__global__ void k_pack(const cplx<T> *__restrict__ v, const cplx<T> *__restrict__ f1, const cplx<T> *__restrict__ f2,
-                       bf16 *__restrict__ act, int64_t vol, col_scale sc)
+__global__ __launch_bounds__(256) void k_pack(pc_cols<T> col, bf16 *__restrict__ act, int64_t vol)
 {
-    for (int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; s < vol; s += (int64_t)gridDim.x * blockDim.x) {
-        const cplx<T> *f[3] = {v, f1, f2};
-        const cplx<double> m[3] = {{1.0, 0.0}, sc.s1, sc.s2};
-        for (int q = 0; q < 3; ++q)
-            for (int c = 0; c < 3; ++c) {
-                const cplx<T> a0 = f[q][(int64_t)c * vol + s];
-                const cplx<double> a = cmuld({(double)a0.re, (double)a0.im}, m[q]);
-                act[s * CH + 6 * q + 2 * c] = f2bf((float)a.re);
-                act[s * CH + 6 * q + 2 * c + 1] = f2bf((float)a.im);
-            }
-        for (int c = CIN; c < CH; ++c) act[s * CH + c] = 0;
-    }
+    const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int k = blockIdx.y;
+    if (s >= vol) return;
+    const cplx<T> *f[3] = {col.v[k], col.f1[k], col.f2[k]};
+    const cplx<double> m[3] = {{1.0, 0.0}, col.sc[k].s1, col.sc[k].s2};
+    u16x8 o[4] = {};
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const cplx<T> a0 = f[q][(int64_t)c * vol + s];
+            const cplx<double> a = cmuld({(double)a0.re, (double)a0.im}, m[q]);
+            const int ch = 6 * q + 2 * c;
+            o[ch / 8][ch % 8] = f2bf((float)a.re);
+            o[ch / 8][ch % 8 + 1] = f2bf((float)a.im);
+        }
+    u16x8 *d = (u16x8 *)(act + ((int64_t)k * vol + s) * CH);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) d[q] = o[q];
 }
 
 // z = v - f1 + f2 + c N(v, f1 s1, f2 s2): the second-order Neumann
 // polynomial of (1 + beta K)^-1 plus the network's correction, output
-// channels 0..5 (colour c at 2 c, 2 c + 1) scaled by c = -(beta kmax)^3
+// channels 0..5 (colour c at 2 c, 2 c + 1; o holds eight channels per site)
+// scaled by c = -(beta kmax)^3
 template <typename T>
-__global__ void k_unpack(const float *__restrict__ o, const cplx<T> *__restrict__ v, const cplx<T> *__restrict__ f1,
-                         const cplx<T> *__restrict__ f2, cplx<T> *__restrict__ z, int64_t vol, col_scale sc)
+__global__ __launch_bounds__(256) void k_unpack(const float *__restrict__ o, pc_cols<T> col, int64_t vol)
 {
-    for (int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; s < vol; s += (int64_t)gridDim.x * blockDim.x)
-        for (int c = 0; c < 3; ++c) {
-            const int64_t at = (int64_t)c * vol + s;
-            const cplx<T> a = v[at], b = f1[at], d = f2[at];
-            const cplx<double> n = cmuld({(double)o[s * CH + 2 * c], (double)o[s * CH + 2 * c + 1]}, sc.c);
-            z[at] = {(T)((a.re - b.re + d.re) + n.re), (T)((a.im - b.im + d.im) + n.im)};
-        }
+    const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int k = blockIdx.y;
+    if (s >= vol) return;
+    const f32x4 *p = (const f32x4 *)(o + ((int64_t)k * vol + s) * 8);
+    const f32x4 lo = p[0], hi = p[1];
+    const float n6[6] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1]};
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        const int64_t at = (int64_t)c * vol + s;
+        const cplx<T> a = col.v[k][at], b = col.f1[k][at], d = col.f2[k][at];
+        const cplx<double> n = cmuld({(double)n6[2 * c], (double)n6[2 * c + 1]}, col.sc[k].c);
+        col.z[k][at] = {(T)((a.re - b.re + d.re) + n.re), (T)((a.im - b.im + d.im) + n.im)};
+    }
 }
 
 // Training sample of one column of a CN solve: right-hand side y, solution
@@ -501,6 +508,9 @@ struct nrq_cnn {
     bf16 *d0 = nullptr, *d1 = nullptr;
     float *out = nullptr;                 // [V][32] FP32 network output
     float *part = nullptr;                // weight-gradient partials
+    bf16 *pact[2] = {};                   // preconditioner: layer inputs of pcols columns, by turns
+    float *pout = nullptr;                // and the first eight output channels
+    int pcols = 0;
     double *lpart = nullptr, *loss = nullptr;
     // training set (on its harvest geometry)
     geom data_g{};
@@ -516,9 +526,12 @@ static void free_geom_buffers(nrq_cnn *n)
 {
     for (auto &a : n->act)
         if (a) (void)hipFree(a), a = nullptr;
-    void *p[] = {n->d0, n->d1, n->out, n->part, n->lpart, n->loss};
+    void *p[] = {n->d0, n->d1, n->out, n->part, n->lpart, n->loss, n->pact[0], n->pact[1], n->pout};
     for (void *q : p)
         if (q) (void)hipFree(q);
+    n->pact[0] = n->pact[1] = nullptr;
+    n->pout = nullptr;
+    n->pcols = 0;
     n->d0 = n->d1 = nullptr;
     n->out = nullptr;
     n->part = nullptr;
@@ -548,25 +561,45 @@ static int ensure_geom(nrq_cnn *n, const geom &g)
     return NRQ_OK;
 }
 
-static unsigned conv_grid(const geom &g)
+// Planes per sweep: the split of n2 with the shortest run, at one block per CU
+// and CONV_START planes' time for a block's weights and first planes (64^3,
+// one field: 2 planes in one round of blocks 75 us, 4 in half a round 105 us).
+constexpr double CONV_START = 3.5;
+template <int XR> static int conv_zc(const geom &g, int nf)
 {
-    const int64_t waves = ((int64_t)(g.n0 / 16) * g.n1 * g.n2 + CONV_SEG - 1) / CONV_SEG;
-    return (unsigned)((waves + 3) / 4);
+    const int64_t tiles = (int64_t)(g.n0 / conv_tile<XR>::TX) * ((g.n1 + conv_tile<XR>::TY - 1) / conv_tile<XR>::TY) * nf;
+    int best = g.n2;
+    double cost = 1e300;
+    for (int runs = 1; runs <= g.n2; ++runs) {
+        const int zc = (g.n2 + runs - 1) / runs;
+        if (zc < 2 && runs > 1) break;
+        const int64_t rounds = (tiles * ((g.n2 + zc - 1) / zc) + 255) / 256;
+        const double c = (double)rounds * (zc + CONV_START);
+        if (c < cost) {
+            cost = c;
+            best = zc;
+        }
+    }
+    return best;
 }
 
-// One convolution layer (k_conv arguments), LDS-staged where the extents
-// allow it.
-static void conv(const geom &g, const bf16 *in, const bf16 *w, bf16 *out_b, float *out_f, const bf16 *mask, int relu)
+template <int XR, int HALVES>
+static void launch_conv(const geom &g, int nf, const bf16 *in, const bf16 *w, bf16 *out_b, float *out_f, const bf16 *mask, int relu)
 {
-    if (g.n0 % LT_X == 0 && g.n1 % 2 == 0 && g.n2 % 16 == 0) {
-        const unsigned blocks = (unsigned)((g.n0 / LT_X) * (g.n1 / 2) * (g.n2 / 16));
-        hipLaunchKernelGGL(k_conv_lds<16>, dim3(blocks), dim3(256), 0, stream(), in, w, out_b, out_f, mask, relu, g);
-    } else if (g.n0 % LT_X == 0 && g.n1 % 2 == 0 && g.n2 % 8 == 0) {
-        const unsigned blocks = (unsigned)((g.n0 / LT_X) * (g.n1 / 2) * (g.n2 / 8));
-        hipLaunchKernelGGL(k_conv_lds<8>, dim3(blocks), dim3(256), 0, stream(), in, w, out_b, out_f, mask, relu, g);
-    } else {
-        hipLaunchKernelGGL(k_conv, dim3(conv_grid(g)), dim3(256), 0, stream(), in, w, out_b, out_f, mask, relu, g);
-    }
+    const int zc = conv_zc<XR>(g, nf);
+    const unsigned blocks = (unsigned)(g.n0 / conv_tile<XR>::TX) *
+                            (unsigned)((g.n1 + conv_tile<XR>::TY - 1) / conv_tile<XR>::TY) * (unsigned)((g.n2 + zc - 1) / zc);
+    hipLaunchKernelGGL((k_conv<XR, HALVES>), dim3(blocks, nf), dim3(CV_TH), 0, stream(), in, w, out_b, out_f, mask, relu, g, zc);
+}
+
+// One convolution layer of nf fields (k_conv arguments), with the widest tile
+// that n0 is a multiple of.
+template <int HALVES = 2>
+static void conv(const geom &g, int nf, const bf16 *in, const bf16 *w, bf16 *out_b, float *out_f, const bf16 *mask, int relu)
+{
+    if (g.n0 % 64 == 0) launch_conv<4, HALVES>(g, nf, in, w, out_b, out_f, mask, relu);
+    else if (g.n0 % 32 == 0) launch_conv<2, HALVES>(g, nf, in, w, out_b, out_f, mask, relu);
+    else launch_conv<1, HALVES>(g, nf, in, w, out_b, out_f, mask, relu);
 }
 
 // forward pass from n->act[0]; FP32 output in n->out
@@ -576,9 +609,9 @@ static int forward(nrq_cnn *n)
     for (int l = 0; l < NL; ++l) {
         const bf16 *w = n->wb + (int64_t)l * WL;
         if (l < NL - 1)
-            conv(g, n->act[l], w, n->act[l + 1], nullptr, nullptr, 1);
+            conv(g, 1, n->act[l], w, n->act[l + 1], nullptr, nullptr, 1);
         else
-            conv(g, n->act[l], w, nullptr, n->out, nullptr, 0);
+            conv(g, 1, n->act[l], w, nullptr, n->out, nullptr, 0);
     }
     NRQ_HIP(hipGetLastError());
     return NRQ_OK;
@@ -604,7 +637,7 @@ static int backward(nrq_cnn *n, const float *tgt, double norm, bf16 *dtrace = nu
                            n->grad + (int64_t)l * WL);
         if (l > 0) {
             // d(pre-activation of layer l-1) = conv(d, mirrored W_l^T) where act[l] > 0
-            conv(g, d, n->wt + (int64_t)l * WL, dn, nullptr, n->act[l], 0);
+            conv(g, 1, d, n->wt + (int64_t)l * WL, dn, nullptr, n->act[l], 0);
             std::swap(d, dn);
         }
     }
@@ -626,21 +659,58 @@ static double spectrum_top(const geom &g)
     return 2.0 / (g.a[1] * g.a[1]) + 2.0 / (g.a[2] * g.a[2]) + 2.0 / (g.a[3] * g.a[3]);
 }
 
+// Buffers for as many of R columns per network pass as make four million sites
+// (several blocks per CU in every layer), at most PC_COLS.
+static int reserve_columns(nrq_cnn *n, const geom &g, int R)
+{
+    const int want = (int)std::max<int64_t>(1, std::min<int64_t>(std::min(R, PC_COLS), ((int64_t)4 << 20) / g.vol));
+    if (want <= n->pcols) return NRQ_OK;
+    void *p[] = {n->pact[0], n->pact[1], n->pout};
+    for (void *q : p)
+        if (q) (void)hipFree(q);
+    n->pact[0] = n->pact[1] = nullptr;
+    n->pout = nullptr;
+    n->pcols = 0;
+    const size_t sites = (size_t)g.vol * (size_t)want;
+    if (hipMalloc(&n->pact[0], sites * CH * sizeof(bf16)) != hipSuccess ||
+        hipMalloc(&n->pact[1], sites * CH * sizeof(bf16)) != hipSuccess ||
+        hipMalloc(&n->pout, sites * 8 * sizeof(float)) != hipSuccess) {
+        (void)hipGetLastError();
+        free_geom_buffers(n);
+        return fail(NRQ_ERR_ALLOC, "cnn: buffer allocation failed (V=%lld, %d columns)", (long long)g.vol, want);
+    }
+    n->pcols = want;
+    return NRQ_OK;
+}
+
 template <typename T>
 int cnn_precondition(nrq_cnn *net, const cplx<T> *const *v, const cplx<T> *const *f1, const cplx<T> *const *f2,
                      cplx<T> *const *z, int R, const int *act, const cplx<double> *beta)
 {
     const geom g = lat().g;
     if (int e = ensure_geom(net, g)) return e;
+    if (int e = reserve_columns(net, g, R)) return e;
     const double kmax = spectrum_top(g);
+    const dim3 blk((unsigned)((g.vol + 255) / 256));
+    pc_cols<T> col = {};
+    int n = 0;
     for (int r = 0; r < R; ++r) {
-        if (act && !act[r]) continue;
-        const col_scale sc = make_col_scale(beta[r], kmax);
-        hipLaunchKernelGGL(k_pack<T>, dim3(1024), dim3(256), 0, stream(), v[r], f1[r], f2[r], net->act[0], g.vol, sc);
-        if (int e = forward(net)) return e;
-        hipLaunchKernelGGL(k_unpack<T>, dim3(1024), dim3(256), 0, stream(), (const float *)net->out, v[r], f1[r], f2[r],
-                           z[r], g.vol, sc);
+        if (!act || act[r]) {
+            col.v[n] = v[r];
+            col.f1[n] = f1[r];
+            col.f2[n] = f2[r];
+            col.z[n] = z[r];
+            col.sc[n] = make_col_scale(beta[r], kmax);
+            ++n;
+        }
+        if (n == 0 || (n < net->pcols && r + 1 < R)) continue;
+        hipLaunchKernelGGL(k_pack<T>, dim3(blk.x, n), dim3(256), 0, stream(), col, net->pact[0], g.vol);
+        for (int l = 0; l < NL - 1; ++l)
+            conv(g, n, net->pact[l & 1], net->wb + (int64_t)l * WL, net->pact[(l + 1) & 1], nullptr, nullptr, 1);
+        conv<1>(g, n, net->pact[(NL - 1) & 1], net->wb + (int64_t)(NL - 1) * WL, nullptr, net->pout, nullptr, 0);
+        hipLaunchKernelGGL(k_unpack<T>, dim3(blk.x, n), dim3(256), 0, stream(), (const float *)net->pout, col, g.vol);
         NRQ_HIP(hipGetLastError());
+        n = 0;
     }
     return NRQ_OK;
 }

@@ -156,6 +156,61 @@ def test_fgmres_zero_network_is_the_neumann_polynomial(nrq, oracle, lattice):
         nrq.nrqcd_finalize()
 
 
+@pytest.mark.parametrize("ext", [
+    (64, 3, 1), (192, 5, 7),             # 64-wide tiles: partial rows of four, one plane, a last short sweep
+    (32, 17, 3), (96, 8, 2),             # 32-wide: wavefronts without rows
+    (16, 33, 2), (48, 31, 5), (80, 4, 9) # 16-wide
+])
+def test_forward_on_ragged_tiles_matches_oracle(nrq, lattice, ext):
+    """Tile widths 64, 32 and 16 with rows and planes that do not fill them
+    (the bar of test_forward_matches_oracle)."""
+    test_forward_matches_oracle(nrq, lattice, ext)
+
+
+@pytest.mark.parametrize("ext", [(64, 6, 5), (32, 9, 4), (16, 5, 7)])
+def test_fgmres_with_a_network_that_is_the_next_neumann_term(nrq, lattice, ext):
+    """On cold links K is a convolution, so a network can be written down that
+    returns (K / kmax) of its input K^2 v / kmax^2 (ReLU pairs carry the signs):
+    the preconditioner is then the third-order Neumann polynomial up to BF16
+    rounding, |beta K| <= 0.3 here.  All 24 columns of a random propagator, two
+    batched network passes per step, must need fewer iterations than with the
+    zero network (the second-order polynomial)."""
+    _say(f"FGMRES with the third Neumann term {ext}")
+    lattice(ext, SP)
+    v = ext[0] * ext[1] * ext[2]
+    w = np.zeros((4, 27, 32, 32), np.float32)
+    for k in range(6):
+        for sign in range(2):
+            ch = 2 * k + sign
+            w[0, 13, ch, 12 + k] = 1.0 - 2.0 * sign
+            w[1, 13, ch, ch] = w[2, 13, ch, ch] = 1.0
+            w[3, 13, k, ch] = (1.0 - 2.0 * sign) * 3.0 / 6.0
+            for tap in (4, 10, 12, 14, 16, 22):  # the six neighbours
+                w[3, tap, k, ch] = (1.0 - 2.0 * sign) * -0.5 / 6.0
+    rng = np.random.default_rng(3)
+    prop = [rng.normal(size=(6, 6, v)) + 1j * rng.normal(size=(6, 6, v)) for _ in range(2)]
+    g = nrq.GaugeConfiguration()
+    net = nrq.PreconditionerNet(1)
+    nrq.nrqcd_init(0.5, C1, 1.0, 1e-12)
+    try:
+        nrq.nrqcd_set_solver(nrq.NRQ_SOLVER_FGMRES_CNN, 20, 10000)
+        its, got = {}, {}
+        for name, weights in (("zero", 0 * w), ("third", w)):
+            net.weights = weights.ravel()
+            nrq.nrqcd_set_preconditioner(net)
+            h = nrq.NRQCDField()
+            h.upload(*prop)
+            st = h.Update(g, 0.5, C1)
+            assert st.max_true_relres <= 1e-12 and st.solves == 24
+            its[name], got[name] = st.iterations, h.download()[0]
+        _say(f"iterations {its}")
+        assert its["third"] <= its["zero"] - 24  # at least one less per column
+        assert np.max(np.abs(got["third"] - got["zero"])) < 1e-10 * np.max(np.abs(got["zero"]))
+        nrq.nrqcd_set_preconditioner(None)
+    finally:
+        nrq.nrqcd_finalize()
+
+
 def test_training_and_gain(nrq, oracle, lattice):
     """Train on pairs from plain GMRES solves at Ma = 1, 2, 5 on an evolved
     configuration, then solve held-out masses 3 and 8 with FGMRES + the trained
