@@ -54,6 +54,17 @@ def test_product_rng_long_stream_in_uneven_draws(oracle, seed):
     assert np.array_equal(np.concatenate(got), oracle.ranlxd(200000))
 
 
+@pytest.mark.parametrize("seed", [1, 2, 3, 2**30, 2**31 - 1])
+def test_product_rng_from_the_edges_of_the_seeds(oracle, seed):
+    """First blocks of the smallest and largest seeds, reseeded in the middle of a block."""
+    import nrqcd_amd as nrq
+    nrq.random_init(77)
+    nrq.random_uniform(17)
+    nrq.random_init(seed)
+    oracle.ranlxd_init(2, seed)
+    assert np.array_equal(nrq.random_uniform(12 * 500 + 5), oracle.ranlxd(12 * 500 + 5))
+
+
 def test_product_rng_rejects_bad_seed():
     import nrqcd_amd as nrq
 
