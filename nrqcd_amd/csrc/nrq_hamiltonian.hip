@@ -32,7 +32,7 @@
 // logarithms per site) and the colour matrices Dsum and G (k_ham_blocks) are
 // built once per step; k_ham_apply applies S or S^+ to several columns at
 // once.
-#include "nrq_internal.h"
+#include "nrq_gmres.h"
 #include "nrq_grouplog.h"
 #include "nrq_map.h"
 #include <algorithm>
@@ -50,8 +50,10 @@ constexpr int HAM_THREADS = 256;
 constexpr int HAM_FLD = 36;   // doubles per site: F0_j (3 x 9), Bsum (9)
 constexpr int HAM_BLK = 13;   // colour matrices per site: Dsum, G[i][sign][p]
 constexpr int HAM_MAXCOL = 12; // columns per apply launch (6 per propagator)
+constexpr int HAM_NC = 2;      // columns per thread of the operator (k_ham_apply has the figures)
+constexpr int HAM_FIELD_THREADS = 3 * 64; // k_ham_fields: three wavefronts, 64 sites
+constexpr int HAM_SITES = 64;  // threads per block of the operator: one wavefront
 constexpr size_t HAM_BATCH_BYTES = (size_t)16 << 30; // Krylov storage of the columns solved together
-constexpr int HAM_DOT_BLOCKS = 512;
 
 template <typename R> __device__ __forceinline__ mat3<double> ham_link(const cplx<R> *u, int64_t vol, int dir, int64_t s)
 {
@@ -74,36 +76,47 @@ __device__ __forceinline__ mat3<double> madd(const mat3<double> &a, const mat3<d
 }
 
 // F0_j(x) and Bsum(x) into fld[(q * 9 + e) V + s], q = 0..2 for F0_j, 3 for Bsum.
+// Bound by the 9 matrix logarithms of a site, long dependent chains of FP64
+// arithmetic, so they are spread over wavefronts: for 64 sites the three of a block
+// with blockIdx.y = 0 take the two plaquette orders of one plane each (the terms of
+// Bsum meet in LDS, summed in a fixed order), the three of the other block F0_j.
+// 33x30x27: 107 us with one thread per site, 76 us so.
 template <typename R>
-__global__ __launch_bounds__(HAM_THREADS) void k_ham_fields(const cplx<R> *__restrict__ u, const R *__restrict__ ef, geom g,
-                                                           double *__restrict__ fld)
+__global__ __launch_bounds__(HAM_FIELD_THREADS) void k_ham_fields(const cplx<R> *__restrict__ u, const R *__restrict__ ef, geom g,
+                                                       double *__restrict__ fld)
 {
-    const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= g.vol) return;
-    const int64_t V = g.vol;
-    for (int j = 0; j < 3; ++j) {
+    __shared__ double part[3][9][64];
+    const int lane = threadIdx.x & 63, i = threadIdx.x >> 6;
+    const int64_t V = g.vol, s0 = (int64_t)blockIdx.x * 64 + lane;
+    const bool in = s0 < V;
+    const int64_t s = in ? s0 : V - 1;
+    if (blockIdx.y == 1) {
         double al[8];
-        for (int a = 0; a < 8; ++a) al[a] = (double)ef[((int64_t)j * 8 + a) * V + s];
+        for (int a = 0; a < 8; ++a) al[a] = (double)ef[((int64_t)i * 8 + a) * V + s];
         const mat3<double> H = group_log_matrix(exp_i_hermitian(algebra_matrix(al)));
-        const double sc = 1.0 / (g.a[0] * g.a[j + 1]);
-        for (int e = 0; e < 9; ++e) fld[((int64_t)j * 9 + e) * V + s] = H.m[e].re * sc;
+        const double sc = 1.0 / (g.a[0] * g.a[i + 1]);
+        if (in)
+            for (int e = 0; e < 9; ++e) fld[((int64_t)i * 9 + e) * V + s] = H.m[e].re * sc;
+        return;
     }
+    const int j = (i + 1) % 3, k = (i + 2) % 3;
     const lsite p = make_site(g, s);
     double b[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    for (int i = 0; i < 3; ++i) {
-        const int j = (i + 1) % 3, k = (i + 2) % 3;
-        for (int o = 0; o < 2; ++o) {
-            // P_mn(x) = U_m(x) U_n(x+m) U_m(x+n)^+ U_n(x)^+ for (m, n) = (j, k), then (k, j)
-            const int m = o == 0 ? j : k, n = o == 0 ? k : j;
-            const mat3<double> P = mul_nd(mul_nd(mul(ham_link(u, V, m, s), ham_link(u, V, n, site_up(g, p, m).s)),
-                                                 ham_link(u, V, m, site_up(g, p, n).s)),
-                                          ham_link(u, V, n, s));
-            const mat3<double> H = group_log_matrix(P);
-            const double sc = (o == 0 ? 0.5 : -0.5) / (g.a[m + 1] * g.a[n + 1]);
-            for (int e = 0; e < 9; ++e) b[e] += H.m[e].re * sc;
-        }
+    for (int o = 0; o < 2; ++o) {
+        // P_mn(x) = U_m(x) U_n(x+m) U_m(x+n)^+ U_n(x)^+ for (m, n) = (j, k), then (k, j)
+        const int m = o == 0 ? j : k, n = o == 0 ? k : j;
+        const mat3<double> P = mul_nd(mul_nd(mul(ham_link(u, V, m, s), ham_link(u, V, n, site_up(g, p, m).s)),
+                                             ham_link(u, V, m, site_up(g, p, n).s)),
+                                      ham_link(u, V, n, s));
+        const mat3<double> H = group_log_matrix(P);
+        const double sc = (o == 0 ? 0.5 : -0.5) / (g.a[m + 1] * g.a[n + 1]);
+        for (int e = 0; e < 9; ++e) b[e] += H.m[e].re * sc;
     }
-    for (int e = 0; e < 9; ++e) fld[((int64_t)27 + e) * V + s] = b[e];
+    for (int e = 0; e < 9; ++e) part[i][e][lane] = b[e];
+    __syncthreads();
+    if (!in) return;
+    for (int e = i; e < 9; e += 3)
+        fld[((int64_t)27 + e) * V + s] = part[0][e][lane] + part[1][e][lane] + part[2][e][lane];
 }
 
 __device__ __forceinline__ mat3<double> ham_e(const double *__restrict__ fld, int64_t V, int j, int64_t s)
@@ -157,16 +170,23 @@ struct ham_cols {
     const cplx<double> *in[HAM_MAXCOL];
     cplx<double> *out[HAM_MAXCOL];
     cplx<double> a[HAM_MAXCOL][4];
+    const cplx<double> *b; // HAM_RESIDUAL: right-hand sides, column after column
+    const int *active;     // columns to work on (may be null: all)
+    double *partial;       // HAM_RHS, HAM_RESIDUAL: [column][site block] sums of |out|^2
     int n; // columns
 };
 
-// Pauli matrix entry sigma_k[r][c] of the reference's table (su2.f90:68-88):
-// k = 0: [[0,1],[1,0]], k = 1: [[0,i],[-i,0]], k = 2: diag(1,-1).
-__device__ __forceinline__ cplx<double> ham_sigma(int k, int r, int c)
+// w = sigma_k (a v) with the Pauli matrices of the reference's table
+// (su2.f90:68-88): [[0,1],[1,0]], [[0,i],[-i,0]], diag(1,-1).
+__device__ __forceinline__ void ham_pauli(int k, cplx<double> a, const cplx<double> (&v)[2][3], cplx<double> (&w)[2][3])
 {
-    if (k == 0) return {r != c ? 1.0 : 0.0, 0.0};
-    if (k == 1) return {0.0, r == c ? 0.0 : (r == 0 ? 1.0 : -1.0)};
-    return {r == c ? (r == 0 ? 1.0 : -1.0) : 0.0, 0.0};
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        const cplx<double> t0 = a * v[0][c], t1 = a * v[1][c];
+        if (k == 0) w[0][c] = t1, w[1][c] = t0;
+        else if (k == 1) w[0][c] = {-t1.im, t1.re}, w[1][c] = {t0.im, -t0.re};
+        else w[0][c] = t0, w[1][c] = {-t1.re, -t1.im};
+    }
 }
 
 __device__ __forceinline__ void ham_load(const cplx<double> *__restrict__ x, int64_t V, int64_t s, cplx<double> (&v)[2][3])
@@ -200,209 +220,159 @@ __device__ __forceinline__ void ham_colour(const mat3<double> &M, const cplx<dou
             }
 }
 
-// acc += Kron(G, sigma_k) v (ADJ: Kron(G^+, sigma_k) v; sigma is Hermitian)
-template <bool ADJ>
-__device__ __forceinline__ void ham_kron(const mat3<double> &G, int k, const cplx<double> (&v)[2][3], cplx<double> (&acc)[2][3])
-{
-    cplx<double> w[2][3];
-#pragma unroll
-    for (int sp = 0; sp < 2; ++sp)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            cplx<double> t = {0.0, 0.0};
-#pragma unroll
-            for (int q = 0; q < 2; ++q) mac(t, ham_sigma(k, sp, q), v[q][c]);
-            w[sp][c] = t;
-        }
-    ham_colour<ADJ>(G, w, acc);
-}
-
-// y = S x (ADJ = false) or S^+ x for the columns of `cols`.  The grid is
-// site blocks x columns with the column fastest, and each XCD walks one
-// contiguous range of it: the columns of a site block run on one XCD one
-// after the other and share its links, field strengths and colour blocks
-// (2.4 KB per site) through that XCD's L2.
-template <typename R, bool ADJ>
-__global__ __launch_bounds__(HAM_THREADS) void k_ham_apply(const cplx<R> *__restrict__ u, const double *__restrict__ fld,
-                                                          const cplx<double> *__restrict__ blk, geom g, ham_cols cols)
-{
-    const unsigned lb = xcd_block(gridDim.x, 8);
-    const int col = (int)(lb % (unsigned)cols.n);
-    const int64_t s = (int64_t)(lb / (unsigned)cols.n) * blockDim.x + threadIdx.x;
-    if (s >= g.vol) return;
-    const int64_t V = g.vol;
-    const cplx<double> *x = cols.in[col];
-    cplx<double> a[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) a[t] = ADJ ? cplx<double>{cols.a[col][t].re, -cols.a[col][t].im} : cols.a[col][t];
-    const lsite p = make_site(g, s);
-    cplx<double> v0[2][3], kin[2][3], c2[2][3], c3[2][3], c4[2][3];
-    ham_load(x, V, s, v0);
-#pragma unroll
-    for (int sp = 0; sp < 2; ++sp)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) kin[sp][c] = c2[sp][c] = c3[sp][c] = c4[sp][c] = {0.0, 0.0};
-    // c2, c3 (site-diagonal colour matrices)
-    {
-        mat3<double> B;
-        for (int e = 0; e < 9; ++e) B.m[e] = {fld[((int64_t)27 + e) * V + s], 0.0};
-        ham_colour<ADJ>(B, v0, c2);
-        ham_colour<ADJ>(ham_blk(blk, V, 0, s), v0, c3);
-    }
-    for (int i = 0; i < 3; ++i) {
-        const int64_t sp_ = site_up(g, p, i).s, sm = site_dn(g, p, i).s;
-        const double w2 = 1.0 / (g.a[i + 1] * g.a[i + 1]);
-        cplx<double> vp[2][3], vm[2][3], h[2][3];
-        ham_load(x, V, sp_, vp);
-        ham_load(x, V, sm, vm);
-        // kinetic: v0 - (U_i(x) v(x+i) + U_i(x-i)^+ v(x-i)) / 2
-#pragma unroll
-        for (int q = 0; q < 2; ++q)
-#pragma unroll
-            for (int c = 0; c < 3; ++c) h[q][c] = {0.0, 0.0};
-        ham_colour<false>(ham_link(u, V, i, s), vp, h);
-        ham_colour<true>(ham_link(u, V, i, sm), vm, h);
-#pragma unroll
-        for (int q = 0; q < 2; ++q)
-#pragma unroll
-            for (int c = 0; c < 3; ++c)
-                kin[q][c] = kin[q][c] + w2 * (v0[q][c] - 0.5 * h[q][c]);
-        // spin-orbit hops
-        for (int q = 0; q < 2; ++q) {
-            const int k = q == 0 ? (i + 2) % 3 : (i + 1) % 3;
-            const int mp = 1 + (2 * i + 0) * 2 + q, mm = 1 + (2 * i + 1) * 2 + q;
-            if (!ADJ) {
-                ham_kron<false>(ham_blk(blk, V, mp, s), k, vp, c4);
-                ham_kron<false>(ham_blk(blk, V, mm, s), k, vm, c4);
-            } else {
-                ham_kron<true>(ham_blk(blk, V, mp, sm), k, vm, c4);
-                ham_kron<true>(ham_blk(blk, V, mm, sp_), k, vp, c4);
-            }
-        }
-    }
-    cplx<double> *y = cols.out[col];
-#pragma unroll
-    for (int q = 0; q < 2; ++q)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            cplx<double> r = v0[q][c];
-            mac(r, a[0], kin[q][c]);
-            mac(r, a[1], c2[q][c]);
-            mac(r, a[2], c3[q][c]);
-            mac(r, a[3], c4[q][c]);
-            y[((int64_t)q * 3 + c) * V + s] = r;
-        }
-}
-
-// ---- vector kernels (n complex doubles) -----------------------------------
-
-__device__ __forceinline__ double ham_wsum(double v)
+// Ends a stage of the operator: the accumulators are complete before any operand of
+// the next stage is loaded.  Without it the compiler gathers the loads of all stages
+// ahead of the arithmetic (228 to 489 spilled registers).
+template <int NC> __device__ __forceinline__ void ham_stage_end(cplx<double> (&acc)[NC][2][3])
 {
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-    return v;
+    for (int q = 0; q < NC; ++q)
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) asm volatile("" : "+v"(acc[q][r][c].re), "+v"(acc[q][r][c].im));
+    __builtin_amdgcn_sched_barrier(0);
 }
 
-__device__ __forceinline__ double ham_block_sum(double v, double *sh)
-{
-    v = ham_wsum(v);
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    __syncthreads();
-    if (lane == 0) sh[w] = v;
-    __syncthreads();
-    double t = 0;
-    if (threadIdx.x == 0)
-        for (int k = 0; k < (int)(blockDim.x >> 6); ++k) t += sh[k];
-    return t;
-}
-
-// Per-column pointers of the Krylov vector kernels: column q of a launch
-// (blockIdx.z for k_ham_dots, blockIdx.y for the others) works on basis[q],
-// w[q], partial[q], small[q] with scale[q]; every column's sums are the same
-// as in a launch of its own.
-struct ham_vecs {
-    const cplx<double> *basis[HAM_MAXCOL];
-    cplx<double> *w[HAM_MAXCOL];
-    double *partial[HAM_MAXCOL];
-    double *small[HAM_MAXCOL];
-    double scale[HAM_MAXCOL];
+enum ham_mode {
+    HAM_ADJOINT = 0,  // y = S^+ x
+    HAM_RHS = 1,      // y = S x, with the partial sums of |y|^2
+    HAM_RESIDUAL = 2, // y = b - S^+ x, with the partial sums of |y|^2
 };
 
-// partial[(2 i + {0: re, 1: im}) * gridDim.x + block] of <V_i, w>, i = blockIdx.y
-__global__ __launch_bounds__(HAM_THREADS) void k_ham_dots(ham_vecs t, int64_t n)
+// The operator for the columns of `cols`.  Bound by the reads through L2: per
+// site 20 colour matrices (links, field strengths and the colour blocks of the
+// derivative and spin-orbit terms, 2.8 KB) against 42 numbers of each column, so a
+// thread applies the matrices it has loaded to HAM_NC columns; and each term's
+// coefficient goes into the vector before the matrix, which leaves one accumulator
+// per column where the terms held four.  The grid is site blocks x column groups with the
+// group fastest, and each XCD walks one contiguous range of it, so the groups of a
+// site block share its matrices through that XCD's L2.  33x30x27,
+// 12 columns, FP64: 76 us with one column per thread, 46 us with two; three and four
+// (one wavefront per SIMD for their registers) make a whole step 5 and 17 % slower.
+template <typename R, int MODE>
+__global__ __launch_bounds__(HAM_SITES, 2) void k_ham_apply(const cplx<R> *__restrict__ u, const double *__restrict__ fld,
+                                                         const cplx<double> *__restrict__ blk, geom g, ham_cols cols)
 {
-    const int i = blockIdx.y, q = blockIdx.z;
-    const cplx<double> *vi = t.basis[q] + (int64_t)i * n;
-    const cplx<double> *__restrict__ w = t.w[q];
-    double *__restrict__ partial = t.partial[q];
-    cplx<double> acc = {0.0, 0.0};
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x)
-        mac_cn(acc, vi[e], w[e]);
-    __shared__ double sh[HAM_THREADS / 64];
-    const double re = ham_block_sum(acc.re, sh);
-    const double im = ham_block_sum(acc.im, sh);
-    if (threadIdx.x == 0) {
-        partial[(int64_t)(2 * i) * gridDim.x + blockIdx.x] = re;
-        partial[(int64_t)(2 * i + 1) * gridDim.x + blockIdx.x] = im;
+    constexpr bool ADJ = MODE != HAM_RHS;
+    const unsigned lb = xcd_block(gridDim.x, 8), ng = (unsigned)((cols.n + HAM_NC - 1) / HAM_NC);
+    const unsigned sb = lb / ng, c0 = lb % ng * HAM_NC;
+    int col[HAM_NC];
+    bool on[HAM_NC], any = false;
+#pragma unroll
+    for (int q = 0; q < HAM_NC; ++q) {
+        // the last group repeats the last column
+        const bool real = (int)c0 + q < cols.n;
+        col[q] = real ? (int)c0 + q : cols.n - 1;
+        on[q] = real && (!cols.active || cols.active[col[q]]);
+        any = any || on[q];
     }
-}
-
-// partial[block] = sum |w|^2
-__global__ __launch_bounds__(HAM_THREADS) void k_ham_norm2(ham_vecs t, int64_t n)
-{
-    const cplx<double> *__restrict__ w = t.w[blockIdx.y];
-    double *__restrict__ partial = t.partial[blockIdx.y];
-    double acc = 0;
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x)
-        acc += w[e].re * w[e].re + w[e].im * w[e].im;
-    __shared__ double sh[HAM_THREADS / 64];
-    const double tot = ham_block_sum(acc, sh);
-    if (threadIdx.x == 0) partial[blockIdx.x] = tot;
-}
-
-// out[q] = sum_b partial[q * nb + b] for q = blockIdx.x (fixed order), out =
-// small + offset of the column
-__global__ __launch_bounds__(HAM_THREADS) void k_ham_fold(ham_vecs t, int nb, int offset)
-{
-    const double *__restrict__ partial = t.partial[blockIdx.y];
-    double *__restrict__ out = t.small[blockIdx.y] + offset;
-    const int q = blockIdx.x;
-    double s = 0;
-    for (int b = threadIdx.x; b < nb; b += HAM_THREADS) s += partial[(int64_t)q * nb + b];
-    __shared__ double sh[HAM_THREADS / 64];
-    s = ham_block_sum(s, sh);
-    if (threadIdx.x == 0) out[q] = s;
-}
-
-// w += sign sum_{i < k} c_i V_i (c: complex coefficients on the device, the
-// column's small)
-__global__ __launch_bounds__(HAM_THREADS) void k_ham_combine(ham_vecs t, int64_t n, int k, double sign)
-{
-    cplx<double> *__restrict__ w = t.w[blockIdx.y];
-    const cplx<double> *__restrict__ basis = t.basis[blockIdx.y];
-    const double *__restrict__ c = t.small[blockIdx.y];
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x) {
-        cplx<double> acc = {0.0, 0.0};
-        for (int i = 0; i < k; ++i) mac(acc, cplx<double>{c[2 * i], c[2 * i + 1]}, basis[(int64_t)i * n + e]);
-        w[e] = {w[e].re + sign * acc.re, w[e].im + sign * acc.im};
+    if (!any) return;
+    const int64_t V = g.vol, t = (int64_t)sb * HAM_SITES + threadIdx.x;
+    const bool inside = t < V;
+    const int64_t s = inside ? t : V - 1;
+    const lsite p = make_site(g, s);
+    const double w2[3] = {1.0 / (g.a[1] * g.a[1]), 1.0 / (g.a[2] * g.a[2]), 1.0 / (g.a[3] * g.a[3])};
+    auto coef = [&](int q, int k) {
+        const cplx<double> a = cols.a[col[q]][k];
+        return ADJ ? cplx<double>{a.re, -a.im} : a;
+    };
+    cplx<double> acc[HAM_NC][2][3], v[HAM_NC][2][3], w[2][3];
+    {
+        double B[9];
+#pragma unroll
+        for (int e = 0; e < 9; ++e) B[e] = fld[((int64_t)27 + e) * V + s];
+        const mat3<double> D = ham_blk(blk, V, 0, s);
+#pragma unroll
+        for (int q = 0; q < HAM_NC; ++q) ham_load(cols.in[col[q]], V, s, v[q]);
+#pragma unroll
+        for (int q = 0; q < HAM_NC; ++q) {
+            // 1 + the site-diagonal part of the kinetic term, c2 and c3
+            const cplx<double> a0 = coef(q, 0), a1 = coef(q, 1), a2 = coef(q, 2);
+            const double ws = w2[0] + w2[1] + w2[2];
+            const cplx<double> d = {ws * a0.re, ws * a0.im};
+#pragma unroll
+            for (int r = 0; r < 2; ++r)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    acc[q][r][c] = v[q][r][c];
+                    mac(acc[q][r][c], d, v[q][r][c]);
+                    w[r][c] = a1 * v[q][r][c];
+                }
+#pragma unroll
+            for (int r = 0; r < 2; ++r)
+#pragma unroll
+                for (int c = 0; c < 3; ++c)
+#pragma unroll
+                    for (int e = 0; e < 3; ++e) {
+                        const double b = B[ADJ ? 3 * e + c : 3 * c + e];
+                        acc[q][r][c].re += b * w[r][e].re;
+                        acc[q][r][c].im += b * w[r][e].im;
+                    }
+#pragma unroll
+            for (int r = 0; r < 2; ++r)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) w[r][c] = a2 * v[q][r][c];
+            ham_colour<ADJ>(D, w, acc[q]);
+        }
+        ham_stage_end(acc);
     }
-}
-
-// w = scale w for the columns of the table
-__global__ __launch_bounds__(HAM_THREADS) void k_ham_scale(ham_vecs t, int64_t n)
-{
-    cplx<double> *__restrict__ w = t.w[blockIdx.y];
-    const double a = t.scale[blockIdx.y];
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x)
-        w[e] = {a * w[e].re, a * w[e].im};
-}
-
-// y = a x + b z (real a, b)
-__global__ __launch_bounds__(HAM_THREADS) void k_ham_axpby(cplx<double> *__restrict__ y, const cplx<double> *__restrict__ x,
-                                                          double a, const cplx<double> *__restrict__ z, double b, int64_t n)
-{
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x)
-        y[e] = {a * x[e].re + b * z[e].re, a * x[e].im + b * z[e].im};
+    // hops to x + i and x - i, one at a time: the operands of all six would not fit
+#pragma unroll 1
+    for (int h = 0; h < 6; ++h) {
+        const int i = h >> 1, dn = h & 1;
+        const int64_t sn = dn ? site_dn(g, p, i).s : site_up(g, p, i).s;
+        const double w2i = i == 0 ? w2[0] : i == 1 ? w2[1] : w2[2];
+#pragma unroll
+        for (int q = 0; q < HAM_NC; ++q) ham_load(cols.in[col[q]], V, sn, v[q]);
+        const mat3<double> U = ham_link(u, V, i, dn ? sn : s);
+        // kinetic: -(U_i(x) v(x+i) or U_i(x-i)^+ v(x-i)) / 2
+#pragma unroll
+        for (int q = 0; q < HAM_NC; ++q) {
+            const cplx<double> a0 = coef(q, 0), f = {-0.5 * w2i * a0.re, -0.5 * w2i * a0.im};
+#pragma unroll
+            for (int r = 0; r < 2; ++r)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) w[r][c] = f * v[q][r][c];
+            if (dn) ham_colour<true>(U, w, acc[q]);
+            else ham_colour<false>(U, w, acc[q]);
+        }
+        ham_stage_end(acc);
+        // spin-orbit: G of this site and hop, or the adjoint of the neighbour's G of
+        // the opposite hop
+        const int gm = 1 + (2 * i + (ADJ ? 1 - dn : dn)) * 2;
+#pragma unroll 1
+        for (int o = 0; o < 2; ++o) {
+            const mat3<double> G = ham_blk(blk, V, gm + o, ADJ ? sn : s);
+            const int k = o == 0 ? (i + 2) % 3 : (i + 1) % 3;
+#pragma unroll
+            for (int q = 0; q < HAM_NC; ++q) {
+                ham_pauli(k, coef(q, 3), v[q], w);
+                ham_colour<ADJ>(G, w, acc[q]);
+            }
+            ham_stage_end(acc);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < HAM_NC; ++q) {
+        if (!on[q]) continue;
+        cplx<double> *y = cols.out[col[q]];
+        double nrm = 0;
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const int64_t at = ((int64_t)r * 3 + c) * V + s;
+                cplx<double> z = acc[q][r][c];
+                if (MODE == HAM_RESIDUAL) z = cols.b[6 * V * col[q] + at] - z;
+                if (inside) y[at] = z;
+                nrm += nrm2(z);
+            }
+        if (MODE != HAM_ADJOINT) {
+            nrm = wsum(inside ? nrm : 0.0);
+            if (threadIdx.x == 0) cols.partial[(int64_t)col[q] * (gridDim.x / ng) + sb] = nrm;
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -410,16 +380,14 @@ __global__ __launch_bounds__(HAM_THREADS) void k_ham_axpby(cplx<double> *__restr
 // ---------------------------------------------------------------------------
 
 struct ham_workspace {
-    scratch_buf fld, blk, basis, vec, red, small;
-    double *host = nullptr; // pinned: 2 (m + 2) doubles, kept until the process ends
-    int host_m = -1;
+    scratch_buf fld, blk, basis, vec, cpart, rpart, spart, gmz, gmd, gmi, nrm;
+    // pinned, kept until the process ends: NSLOTS sums, then NSLOTS each of cycle
+    // flags of even and odd steps, columns used, and (unused here) network falls
+    double *sums = nullptr;
+    int *flags = nullptr;
+    hipEvent_t ev[2] = {nullptr, nullptr}; // end of even and odd Arnoldi steps
 };
 static ham_workspace g_ham;
-
-static unsigned ham_blocks(int64_t n)
-{
-    return (unsigned)std::min<int64_t>(std::max<int64_t>((n + HAM_THREADS - 1) / HAM_THREADS, 1), 8192);
-}
 
 struct ham_operator {
     const void *u;
@@ -427,252 +395,136 @@ struct ham_operator {
     geom g;
     const double *fld;
     const cplx<double> *blk;
+    unsigned nsb; // site blocks
 };
 
-static int ham_apply(const ham_operator &op, bool adj, int ncol, const cplx<double> *const *in, cplx<double> *const *out,
-                     const cplx<double> (*a)[4])
+template <int MODE> static void ham_apply(const ham_operator &op, const ham_cols &cols)
 {
-    ham_cols cols;
-    for (int c = 0; c < ncol; ++c) {
-        cols.in[c] = in[c];
-        cols.out[c] = out[c];
-        for (int t = 0; t < 4; ++t) cols.a[c][t] = a[c][t];
-    }
-    cols.n = ncol;
-    const dim3 grd((unsigned)((op.g.vol + HAM_THREADS - 1) / HAM_THREADS) * (unsigned)ncol);
-    if (op.precision == 64) {
-        if (adj)
-            hipLaunchKernelGGL((k_ham_apply<double, true>), grd, dim3(HAM_THREADS), 0, stream(), (const cplx<double> *)op.u, op.fld, op.blk, op.g, cols);
-        else
-            hipLaunchKernelGGL((k_ham_apply<double, false>), grd, dim3(HAM_THREADS), 0, stream(), (const cplx<double> *)op.u, op.fld, op.blk, op.g, cols);
-    } else {
-        if (adj)
-            hipLaunchKernelGGL((k_ham_apply<float, true>), grd, dim3(HAM_THREADS), 0, stream(), (const cplx<float> *)op.u, op.fld, op.blk, op.g, cols);
-        else
-            hipLaunchKernelGGL((k_ham_apply<float, false>), grd, dim3(HAM_THREADS), 0, stream(), (const cplx<float> *)op.u, op.fld, op.blk, op.g, cols);
-    }
+    const dim3 grd(op.nsb * (unsigned)((cols.n + HAM_NC - 1) / HAM_NC));
+    if (op.precision == 64)
+        hipLaunchKernelGGL((k_ham_apply<double, MODE>), grd, dim3(HAM_SITES), 0, stream(), (const cplx<double> *)op.u, op.fld, op.blk, op.g, cols);
+    else
+        hipLaunchKernelGGL((k_ham_apply<float, MODE>), grd, dim3(HAM_SITES), 0, stream(), (const cplx<float> *)op.u, op.fld, op.blk, op.g, cols);
+}
+
+// The squared norms of nc columns from the operator's partials, to g_ham.sums
+// (columns without active[c] keep what is there), once the stream is done.
+static int ham_norms(const ham_operator &op, int nc, const int *active)
+{
+    hipLaunchKernelGGL(k_fold_slots, dim3(nc), dim3(FOLD_THREADS), 0, stream(), (const double *)g_ham.spart.ptr,
+                       (int64_t)op.nsb, active, (double *)g_ham.nrm.ptr, g_ham.sums);
     NRQ_HIP(hipGetLastError());
+    NRQ_HIP(hipStreamSynchronize(stream()));
     return NRQ_OK;
 }
 
-// GMRES(m) for S^+ x_c = b_c on nc columns (n = 6V complex each), zero
-// initial guess, stopping on ||b_c - S^+ x_c|| <= tol ||b_c||.  The columns
-// run in lockstep, each through exactly the operations (and summation order)
-// it would take alone: one operator launch for all columns of an Arnoldi
-// step and one host synchronisation per step for all their Gram-Schmidt
-// coefficients.  Column c uses basis block c of the workspace.  A column
-// that reaches maxit leaves NRQ_ERR_NOCONV as the result; the others finish.
-static int ham_gmres(const ham_operator &op, int nc, const cplx<double> (*a)[4], cplx<double> *const *b,
+// Right-hand sides b = S x, then GMRES(m) for S^+ x_c = b_c on nc columns
+// (n = 6V complex each), zero initial guess, into x, stopping on
+// ||b_c - S^+ x_c|| <= tol ||b_c||.  The columns run in lockstep, each through exactly
+// the operations (and summation order) it would take alone.  The scalars of the
+// iteration stay on the device (nrq_gmres.h); the host looks at the cycle flags of one
+// step while the next is queued.  33x30x27, 12 columns: 1.07 ms a step where one
+// synchronisation per iteration, separate norm and scaling passes and launches per
+// column took 1.59 ms with the operator then used.  A column that reaches maxit leaves NRQ_ERR_NOCONV as the
+// result; the others finish.
+static int ham_solve(const ham_operator &op, int nc, const cplx<double> (*a)[4], cplx<double> *b, cplx<double> *res,
                      cplx<double> *const *x, int64_t n, int m, int64_t maxit, double tol, nrq_solve_stats *st)
 {
-    const int64_t ldb = (int64_t)(m + 1) * n;                 // basis block per column
-    const int64_t lred = 2 * (int64_t)(m + 2) * HAM_DOT_BLOCKS; // reduction partials per column
-    const int lsm = 2 * (m + 2);                               // small device / pinned host slots per column
-    auto basis = [&](int c) { return (cplx<double> *)g_ham.basis.ptr + c * ldb; };
-    auto rvec = [&](int c) { return (cplx<double> *)g_ham.vec.ptr + (int64_t)c * n; };
-    auto red = [&](int c) { return (double *)g_ham.red.ptr + c * lred; };
-    auto dsm = [&](int c) { return (double *)g_ham.small.ptr + (int64_t)c * lsm; };
-    auto hst = [&](int c) { return g_ham.host + (int64_t)c * lsm; };
-    const unsigned nb = ham_blocks(n);
-    // the Krylov-kernel table of the columns sel[0 .. ns) with vectors wv
-    auto table = [&](int ns, const int *sl, cplx<double> *const *wv) {
-        ham_vecs t{};
-        for (int q = 0; q < ns; ++q) {
-            t.basis[q] = basis(sl[q]);
-            t.w[q] = wv[q];
-            t.partial[q] = red(sl[q]);
-            t.small[q] = dsm(sl[q]);
-            t.scale[q] = 1.0;
-        }
-        return t;
-    };
-    // the small device slots of all columns to the pinned host slots
-    auto smalls_to_host = [&]() {
-        return hipMemcpyAsync(hst(0), dsm(0), sizeof(double) * (size_t)lsm * (size_t)nc, hipMemcpyDeviceToHost, stream());
-    };
-    using zc = std::complex<double>;
-    struct column {
-        std::vector<zc> H, cs, sn, g, y;
-        double bnorm = 0, rnorm = 0;
-        int64_t its = 0;
-        int k = 0;           // Arnoldi steps of the current cycle
-        bool active = false; // not yet converged
-        bool cycling = false;
-        bool failed = false;
-    };
-    std::vector<column> col(nc);
-    const cplx<double> *ins[HAM_MAXCOL];
-    cplx<double> *outs[HAM_MAXCOL];
-    cplx<double> cof[HAM_MAXCOL][4];
-    int sel[HAM_MAXCOL];
-    // ||b||^2 of every column, one synchronisation
+    const gm_state gm = gm_layout(m, (cplx<double> *)g_ham.gmz.ptr, (double *)g_ham.gmd.ptr, (int *)g_ham.gmi.ptr);
+    cplx<double> *basis = (cplx<double> *)g_ham.basis.ptr, *cpart = (cplx<double> *)g_ham.cpart.ptr;
+    double *rpart = (double *)g_ham.rpart.ptr;
+    const unsigned nb = vblocks(n);
+    int *const used = g_ham.flags + 2 * NSLOTS, *const fallen = g_ham.flags + 3 * NSLOTS;
+    ham_cols cols = {};
+    cols.n = nc;
+    cols.b = b;
+    cols.partial = (double *)g_ham.spart.ptr;
+    slots<double> xs = {};
     for (int c = 0; c < nc; ++c) {
-        sel[c] = c;
-        outs[c] = b[c];
+        xs.p[c] = x[c];
+        cols.in[c] = x[c];
+        cols.out[c] = b + (int64_t)c * n;
+        for (int t = 0; t < 4; ++t) cols.a[c][t] = a[c][t];
     }
-    {
-        const ham_vecs t = table(nc, sel, outs);
-        hipLaunchKernelGGL(k_ham_norm2, dim3(HAM_DOT_BLOCKS, nc), dim3(HAM_THREADS), 0, stream(), t, n);
-        hipLaunchKernelGGL(k_ham_fold, dim3(1, nc), dim3(HAM_THREADS), 0, stream(), t, HAM_DOT_BLOCKS, 0);
-    }
-    NRQ_HIP(smalls_to_host());
-    NRQ_HIP(hipGetLastError());
-    NRQ_HIP(hipStreamSynchronize(stream()));
+    ham_apply<HAM_RHS>(op, cols);
+    if (int e = ham_norms(op, nc, nullptr)) return e;
+    double bnorm[HAM_MAXCOL], rnorm[HAM_MAXCOL];
+    int64_t its[HAM_MAXCOL] = {};
+    unsigned long long act = 0; // not yet converged (x = 0, as KSPSolve returns for b = 0)
     for (int c = 0; c < nc; ++c) {
-        column &C = col[c];
-        const double bn2 = hst(c)[0];
-        NRQ_HIP(hipMemsetAsync(x[c], 0, sizeof(cplx<double>) * (size_t)n, stream()));
-        if (bn2 == 0.0) continue; // x = 0, as KSPSolve returns for b = 0
+        bnorm[c] = rnorm[c] = std::sqrt(g_ham.sums[c]);
+        if (g_ham.sums[c] == 0.0) continue;
         ++st->solves;
-        C.active = true;
-        C.bnorm = C.rnorm = std::sqrt(bn2);
-        C.H.assign((size_t)(m + 1) * m, 0.0);
-        C.cs.assign(m, 0.0);
-        C.sn.assign(m, 0.0);
-        C.g.assign(m + 1, 0.0);
-        C.y.assign(m, 0.0);
-        // r = b (x = 0)
-        hipLaunchKernelGGL(k_ham_axpby, dim3(nb), dim3(HAM_THREADS), 0, stream(), rvec(c), b[c], 1.0, b[c], 0.0, n);
+        act |= 1ull << c;
     }
-    while (true) {
-        int nact = 0;
-        for (int c = 0; c < nc; ++c) nact += col[c].active;
-        if (!nact) break;
-        // new cycle: V_0 = r / ||r||
+    if (!act) {
+        for (int c = 0; c < nc; ++c) NRQ_HIP(hipMemsetAsync(x[c], 0, sizeof(cplx<double>) * (size_t)n, stream()));
+        return NRQ_OK;
+    }
+    const cplx<double> *r0 = b; // residual the cycle starts from
+    int failed = -1;
+    for (bool first = true; act; first = false) {
+        gm_start in = {};
         for (int c = 0; c < nc; ++c) {
-            column &C = col[c];
-            if (!C.active) continue;
-            ++st->restarts;
-            hipLaunchKernelGGL(k_ham_axpby, dim3(nb), dim3(HAM_THREADS), 0, stream(), basis(c), rvec(c), 1.0 / C.rnorm,
-                               rvec(c), 0.0, n);
-            std::fill(C.g.begin(), C.g.end(), 0.0);
-            C.g[0] = C.rnorm;
-            C.k = 0;
-            C.cycling = true;
+            in.rn[c] = rnorm[c];
+            in.stop[c] = 0.5 * tol * bnorm[c];
+            in.left[c] = (int)std::min<int64_t>(m, std::max<int64_t>(1, maxit - its[c]));
+            st->restarts += (int64_t)(act >> c & 1ull);
         }
+        in.act = act;
+        hipLaunchKernelGGL(k_gm_begin, dim3(1), dim3(64), 0, stream(), gm, in);
+        const gm_basis<double> W = {r0, basis};
         for (int k = 0; k < m; ++k) {
-            int ns = 0;
+            if (k >= 2) {
+                NRQ_HIP(hipEventSynchronize(g_ham.ev[k & 1]));
+                bool busy = false;
+                for (int c = 0; c < nc; ++c) busy = busy || *(volatile int *)(g_ham.flags + (k & 1) * NSLOTS + c);
+                if (!busy) break;
+            }
+            cplx<double> *w = basis + (int64_t)(k + 1) * nc * n;
             for (int c = 0; c < nc; ++c) {
-                column &C = col[c];
-                if (C.active && C.cycling && C.its >= maxit) C.cycling = false;
-                if (!(C.active && C.cycling)) continue;
-                ++C.its;
-                sel[ns] = c;
-                ins[ns] = basis(c) + (int64_t)k * n;
-                outs[ns] = basis(c) + (int64_t)(k + 1) * n;
-                for (int t = 0; t < 4; ++t) cof[ns][t] = a[c][t];
-                ++ns;
+                cols.in[c] = W.at(k, c, nc, n);
+                cols.out[c] = w + (int64_t)c * n;
             }
-            if (!ns) break;
-            if (int e = ham_apply(op, true, ns, ins, outs, cof)) return e;
-            // classical Gram-Schmidt of every column: h = V^+ w, w -= V h, ||w||^2
-            ham_vecs tab = table(ns, sel, outs);
-            hipLaunchKernelGGL(k_ham_dots, dim3(HAM_DOT_BLOCKS, k + 1, ns), dim3(HAM_THREADS), 0, stream(), tab, n);
-            hipLaunchKernelGGL(k_ham_fold, dim3(2 * (k + 1), ns), dim3(HAM_THREADS), 0, stream(), tab, HAM_DOT_BLOCKS, 0);
-            hipLaunchKernelGGL(k_ham_combine, dim3(nb, ns), dim3(HAM_THREADS), 0, stream(), tab, n, k + 1, -1.0);
-            hipLaunchKernelGGL(k_ham_norm2, dim3(HAM_DOT_BLOCKS, ns), dim3(HAM_THREADS), 0, stream(), tab, n);
-            hipLaunchKernelGGL(k_ham_fold, dim3(1, ns), dim3(HAM_THREADS), 0, stream(), tab, HAM_DOT_BLOCKS, 2 * (k + 1));
-            NRQ_HIP(smalls_to_host());
+            cols.active = gm.cyc;
+            ham_apply<HAM_ADJOINT>(op, cols);
+            const int nv = k + 1;
+            hipLaunchKernelGGL(k_mdot<double>, dim3(nb, nc), dim3(VTHREADS), 0, stream(), W, nv, (const cplx<double> *)w, n, nc,
+                               (const int *)gm.cyc, cpart);
+            hipLaunchKernelGGL(k_gm_dots, dim3((nv * nc + 3) / 4), dim3(256), 0, stream(), cpart, (int)nb, nv, nc, gm);
+            hipLaunchKernelGGL(k_cgs_update<double>, dim3(nb, nc), dim3(VTHREADS), 0, stream(), W, nv, w, n, nc, gm, rpart);
+            hipLaunchKernelGGL(k_gm_step, dim3(nc), dim3(VTHREADS), 0, stream(), rpart, (int)nb, k, 0, gm,
+                               g_ham.flags + (k & 1) * NSLOTS);
             NRQ_HIP(hipGetLastError());
-            NRQ_HIP(hipStreamSynchronize(stream()));
-            int nsc = 0; // columns to normalise, in tab's first nsc slots
-            for (int q = 0; q < ns; ++q) {
-                const int c = sel[q];
-                column &C = col[c];
-                const double *host = hst(c);
-                std::vector<zc> &H = C.H;
-                for (int i = 0; i <= k; ++i) H[(size_t)i * m + k] = {host[2 * i], host[2 * i + 1]};
-                const double hk1 = std::sqrt(host[2 * (k + 1)]);
-                H[(size_t)(k + 1) * m + k] = hk1;
-                if (hk1 > 0) {
-                    tab.w[nsc] = outs[q];
-                    tab.scale[nsc] = 1.0 / hk1;
-                    ++nsc;
-                }
-                // Givens rotations
-                for (int i = 0; i < k; ++i) {
-                    const zc t = C.cs[i] * H[(size_t)i * m + k] + C.sn[i] * H[(size_t)(i + 1) * m + k];
-                    H[(size_t)(i + 1) * m + k] = -std::conj(C.sn[i]) * H[(size_t)i * m + k] + C.cs[i] * H[(size_t)(i + 1) * m + k];
-                    H[(size_t)i * m + k] = t;
-                }
-                const zc hkk = H[(size_t)k * m + k];
-                const double den = std::sqrt(std::norm(hkk) + hk1 * hk1);
-                if (den == 0.0) {
-                    C.cs[k] = 1.0;
-                    C.sn[k] = 0.0;
-                } else {
-                    C.cs[k] = std::abs(hkk) / den;
-                    const zc ph = std::abs(hkk) > 0 ? hkk / std::abs(hkk) : zc(1.0, 0.0);
-                    C.sn[k] = ph * hk1 / den;
-                }
-                H[(size_t)k * m + k] = C.cs[k] * hkk + C.sn[k] * hk1;
-                H[(size_t)(k + 1) * m + k] = 0.0;
-                C.g[k + 1] = -std::conj(C.sn[k]) * C.g[k];
-                C.g[k] = C.cs[k] * C.g[k];
-                C.k = k + 1;
-                if (std::abs(C.g[k + 1]) <= 0.5 * tol * C.bnorm || hk1 == 0.0) C.cycling = false;
-            }
-            if (nsc) hipLaunchKernelGGL(k_ham_scale, dim3(nb, nsc), dim3(HAM_THREADS), 0, stream(), tab, n);
+            NRQ_HIP(hipEventRecord(g_ham.ev[k & 1], stream()));
         }
-        // end of the cycle: y = H^-1 g (upper triangular, k x k), x += V y, then
-        // the true residual r = b - S^+ x of every column that ran
-        int ns = 0;
+        hipLaunchKernelGGL(k_gm_solve, dim3(nc), dim3(64), 0, stream(), gm, 0, used, fallen);
+        hipLaunchKernelGGL(k_xupdate<double>, dim3(nb, nc), dim3(VTHREADS), 0, stream(), xs, W, nc, n, gm, first ? 1 : 0);
+        // the true residual r = b - S^+ x of every column that ran; the others' rows of
+        // res are not read again
         for (int c = 0; c < nc; ++c) {
-            column &C = col[c];
-            if (!C.active) continue;
-            const int k = C.k;
-            for (int i = k - 1; i >= 0; --i) {
-                zc t = C.g[i];
-                for (int j = i + 1; j < k; ++j) t -= C.H[(size_t)i * m + j] * C.y[j];
-                C.y[i] = t / C.H[(size_t)i * m + i];
-            }
-            double *host = hst(c);
-            for (int i = 0; i < k; ++i) {
-                host[2 * i] = C.y[i].real();
-                host[2 * i + 1] = C.y[i].imag();
-            }
-            NRQ_HIP(hipMemcpyAsync(dsm(c), host, sizeof(double) * 2 * k, hipMemcpyHostToDevice, stream()));
-            {
-                const int one[1] = {c};
-                hipLaunchKernelGGL(k_ham_combine, dim3(nb, 1), dim3(HAM_THREADS), 0, stream(), table(1, one, &x[c]), n, k, 1.0);
-            }
-            sel[ns] = c;
-            ins[ns] = x[c];
-            outs[ns] = rvec(c);
-            for (int t = 0; t < 4; ++t) cof[ns][t] = a[c][t];
-            ++ns;
+            cols.in[c] = x[c];
+            cols.out[c] = res + (int64_t)c * n;
         }
-        if (int e = ham_apply(op, true, ns, ins, outs, cof)) return e;
-        for (int q = 0; q < ns; ++q) {
-            const int c = sel[q];
-            hipLaunchKernelGGL(k_ham_axpby, dim3(nb), dim3(HAM_THREADS), 0, stream(), rvec(c), b[c], 1.0, rvec(c), -1.0, n);
-        }
-        {
-            const ham_vecs t = table(ns, sel, outs);
-            hipLaunchKernelGGL(k_ham_norm2, dim3(HAM_DOT_BLOCKS, ns), dim3(HAM_THREADS), 0, stream(), t, n);
-            hipLaunchKernelGGL(k_ham_fold, dim3(1, ns), dim3(HAM_THREADS), 0, stream(), t, HAM_DOT_BLOCKS, 0);
-        }
-        NRQ_HIP(smalls_to_host());
-        NRQ_HIP(hipGetLastError());
-        NRQ_HIP(hipStreamSynchronize(stream()));
-        for (int q = 0; q < ns; ++q) {
-            column &C = col[sel[q]];
-            C.rnorm = std::sqrt(hst(sel[q])[0]);
-            st->iterations += C.k;
-            if (C.rnorm <= tol * C.bnorm) {
-                C.active = false;
-                st->max_true_relres = std::max(st->max_true_relres, C.rnorm / C.bnorm);
-            } else if (C.its >= maxit) {
-                C.active = false;
-                C.failed = true;
-                st->max_true_relres = std::max(st->max_true_relres, C.rnorm / C.bnorm);
-            }
+        cols.active = gm.act;
+        ham_apply<HAM_RESIDUAL>(op, cols);
+        r0 = res;
+        if (int e = ham_norms(op, nc, gm.act)) return e;
+        for (int c = 0; c < nc; ++c) {
+            if (!(act >> c & 1ull)) continue;
+            rnorm[c] = std::sqrt(g_ham.sums[c]);
+            its[c] += used[c];
+            st->iterations += used[c];
+            const bool conv = rnorm[c] <= tol * bnorm[c];
+            if (!conv && its[c] < maxit) continue;
+            act &= ~(1ull << c);
+            st->max_true_relres = std::max(st->max_true_relres, rnorm[c] / bnorm[c]);
+            if (!conv && failed < 0) failed = c;
         }
     }
-    for (int c = 0; c < nc; ++c)
-        if (col[c].failed)
-            return fail(NRQ_ERR_NOCONV, "CN (full Hamiltonian): no convergence after %lld iterations (relres %.3e)",
-                        (long long)col[c].its, col[c].rnorm / col[c].bnorm);
+    if (failed >= 0)
+        return fail(NRQ_ERR_NOCONV, "CN (full Hamiltonian): no convergence after %lld iterations (relres %.3e)",
+                    (long long)its[failed], rnorm[failed] / bnorm[failed]);
     return NRQ_OK;
 }
 
@@ -697,33 +549,41 @@ int ham_cn_update(nrq_heavy *const *hs, const double *mass, int n, const nrq_gau
     if (int r = g_ham.blk.reserve(sizeof(cplx<double>) * 9 * HAM_BLK * (size_t)V)) return r;
     if (int r = g_ham.basis.reserve(sizeof(cplx<double>) * (size_t)(m + 1) * (size_t)nvec * ncb)) return r;
     if (int r = g_ham.vec.reserve(sizeof(cplx<double>) * 2 * (size_t)nvec * ncb)) return r;
-    if (int r = g_ham.red.reserve(sizeof(double) * 2 * (size_t)(m + 2) * HAM_DOT_BLOCKS * ncb)) return r;
-    if (int r = g_ham.small.reserve(sizeof(double) * 2 * (size_t)(m + 2) * ncb)) return r;
-    const int host_need = (m + 2) * ncb;
-    if (g_ham.host_m < host_need) {
-        if (g_ham.host) (void)hipHostFree(g_ham.host);
-        g_ham.host = nullptr;
-        if (hipHostMalloc((void **)&g_ham.host, sizeof(double) * 2 * (size_t)host_need, hipHostMallocDefault) != hipSuccess) {
-            (void)hipGetLastError();
-            g_ham.host_m = -1;
-            return fail(NRQ_ERR_ALLOC, "CN (full Hamiltonian): pinned buffer allocation failed");
-        }
-        g_ham.host_m = host_need;
+    const int64_t nsb = (V + HAM_SITES - 1) / HAM_SITES;
+    if (int r = g_ham.cpart.reserve(sizeof(cplx<double>) * (size_t)ncb * (size_t)m * VBLOCKS)) return r;
+    if (int r = g_ham.rpart.reserve(sizeof(double) * (size_t)ncb * VBLOCKS)) return r;
+    if (int r = g_ham.spart.reserve(sizeof(double) * (size_t)ncb * (size_t)nsb)) return r;
+    if (int r = g_ham.gmz.reserve(sizeof(cplx<double>) * gm_zcount(m))) return r;
+    if (int r = g_ham.gmd.reserve(sizeof(double) * gm_dcount(m))) return r;
+    if (int r = g_ham.gmi.reserve(sizeof(int) * GM_ICOUNT)) return r;
+    if (int r = g_ham.nrm.reserve(sizeof(double) * NSLOTS)) return r;
+    if (!g_ham.sums && hipHostMalloc((void **)&g_ham.sums, sizeof(double) * NSLOTS, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        g_ham.sums = nullptr;
+        return fail(NRQ_ERR_ALLOC, "CN (full Hamiltonian): pinned buffer allocation failed");
     }
+    if (!g_ham.flags && hipHostMalloc((void **)&g_ham.flags, sizeof(int) * 4 * NSLOTS, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        g_ham.flags = nullptr;
+        return fail(NRQ_ERR_ALLOC, "CN (full Hamiltonian): pinned buffer allocation failed");
+    }
+    for (hipEvent_t &e : g_ham.ev)
+        if (!e) NRQ_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     ham_operator op;
     op.u = gauge_links(gf);
     op.precision = gf->precision;
     op.g = g;
     op.fld = (const double *)g_ham.fld.ptr;
     op.blk = (const cplx<double> *)g_ham.blk.ptr;
+    op.nsb = (unsigned)nsb;
     const unsigned nbs = (unsigned)((V + HAM_THREADS - 1) / HAM_THREADS);
     if (gf->precision == 64) {
-        hipLaunchKernelGGL(k_ham_fields<double>, dim3(nbs), dim3(HAM_THREADS), 0, stream(), (const cplx<double> *)op.u,
+        hipLaunchKernelGGL(k_ham_fields<double>, dim3(op.nsb, 2), dim3(HAM_FIELD_THREADS), 0, stream(), (const cplx<double> *)op.u,
                            (const double *)gf->e, g, (double *)g_ham.fld.ptr);
         hipLaunchKernelGGL(k_ham_blocks<double>, dim3(nbs), dim3(HAM_THREADS), 0, stream(), (const cplx<double> *)op.u,
                            (const double *)g_ham.fld.ptr, g, (cplx<double> *)g_ham.blk.ptr);
     } else {
-        hipLaunchKernelGGL(k_ham_fields<float>, dim3(nbs), dim3(HAM_THREADS), 0, stream(), (const cplx<float> *)op.u,
+        hipLaunchKernelGGL(k_ham_fields<float>, dim3(op.nsb, 2), dim3(HAM_FIELD_THREADS), 0, stream(), (const cplx<float> *)op.u,
                            (const float *)gf->e, g, (double *)g_ham.fld.ptr);
         hipLaunchKernelGGL(k_ham_blocks<float>, dim3(nbs), dim3(HAM_THREADS), 0, stream(), (const cplx<float> *)op.u,
                            (const double *)g_ham.fld.ptr, g, (cplx<double> *)g_ham.blk.ptr);
@@ -732,7 +592,7 @@ int ham_cn_update(nrq_heavy *const *hs, const double *mass, int n, const nrq_gau
     const double a0 = g.a[0];
     const std::complex<double> pre(0.0, -stepwidth / 2.0 * a0), I(0.0, 1.0);
     // right-hand sides after the ncb residual vectors
-    auto bvec = [&](int c) { return (cplx<double> *)g_ham.vec.ptr + (int64_t)(ncb + c) * nvec; };
+    cplx<double> *res = (cplx<double> *)g_ham.vec.ptr, *rhs = res + (int64_t)ncb * nvec;
     nrq_solve_stats st = {0, 0, 0, 0.0};
     int status = NRQ_OK;
     for (int hk = 0; hk < n; ++hk) {
@@ -760,18 +620,13 @@ int ham_cn_update(nrq_heavy *const *hs, const double *mass, int n, const nrq_gau
         }
         for (size_t c0 = 0; c0 < f0s.size(); c0 += (size_t)ncb) {
             const int nc = (int)std::min<size_t>((size_t)ncb, f0s.size() - c0);
-            const cplx<double> *xin[HAM_MAXCOL];
-            cplx<double> *xcol[HAM_MAXCOL], *bcol[HAM_MAXCOL];
+            cplx<double> *xcol[HAM_MAXCOL];
             cplx<double> cof[HAM_MAXCOL][4];
             for (int c = 0; c < nc; ++c) {
                 xcol[c] = (cplx<double> *)h->psi + (int64_t)f0s[c0 + c] * 3 * V;
-                xin[c] = xcol[c];
-                bcol[c] = bvec(c);
                 for (int t = 0; t < 4; ++t) cof[c][t] = coefs[c0 + c][t];
             }
-            // rhs = S psi for the batch, then S^+ psi' = rhs
-            if (int e = ham_apply(op, false, nc, xin, bcol, cof)) return e;
-            const int r = ham_gmres(op, nc, cof, bcol, xcol, nvec, m, maxit, tol, &st);
+            const int r = ham_solve(op, nc, cof, rhs, res, xcol, nvec, m, maxit, tol, &st);
             for (int c = 0; c < nc; ++c) h->live |= 3u << f0s[c0 + c]; // the spin-orbit term fills both spin rows
             if (r == NRQ_ERR_NOCONV) {
                 status = r;

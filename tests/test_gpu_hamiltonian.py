@@ -156,3 +156,28 @@ def test_full_hamiltonian_column_batches_are_bit_identical(nrq, oracle, cn, monk
     Qa, Aa = whole.download()
     Qb, Ab = parts.download()
     assert np.array_equal(Qa, Qb) and np.array_equal(Aa, Ab)
+
+
+@pytest.mark.parametrize("ext", [(4, 4, 4), (5, 13, 2), (3, 7, 9)])
+def test_full_hamiltonian_at_the_edges_of_wavefronts(nrq, oracle, cn, ext):
+    """Volumes of one whole, two and a fraction, and three minus a few
+    wavefronts of sites, with an odd number of columns on each propagator (a
+    thread of the operator takes two)."""
+    sp = (0.05, 1.0, 0.9, 1.2)
+    _say(f"full Hamiltonian, {ext}")
+    lat, g, U, E = _setup(nrq, oracle, cn, ext, sp, seed=5)
+    rng = np.random.default_rng(12)
+    v = lat.vol
+    Q = np.asfortranarray(rng.normal(size=(6, 6, v)) + 1j * rng.normal(size=(6, 6, v)))
+    A = np.asfortranarray(rng.normal(size=(6, 6, v)) + 1j * rng.normal(size=(6, 6, v)))
+    Q[:, 3] = 0.0
+    A[:, 1:4] = 0.0
+    c = [0.9, 1.1 + 0.3j, 0.6, -0.8]
+    h = nrq.NRQCDField()
+    h.upload(Q, A)
+    st = h.Update(g, 1.4, c, 0.7)
+    assert st.solves == 8 and st.max_true_relres <= 1e-12
+    ho.cn_update(lat, U, E, Q, A, 1.4, c, 0.7, _pauli(oracle))
+    Qg, Ag = h.download()
+    assert np.max(np.abs(Qg - Q)) < 1e-10 * np.max(np.abs(Q))
+    assert np.max(np.abs(Ag - A)) < 1e-10 * np.max(np.abs(A))
