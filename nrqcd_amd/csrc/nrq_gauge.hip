@@ -263,26 +263,44 @@ __global__ __launch_bounds__(BS) void k_fused(lf_batch<R> bt, geom g, R dt, lf_m
     store_link_out<NT>(uout, g.vol, i, s, evolve_link(ui, e, dt));
 }
 
+// Ends a stage: m is complete before the operands of the next stage are read.
+template <typename R> __device__ __forceinline__ void stage_end(mat3<R> &m)
+{
+#pragma unroll
+    for (int k = 0; k < 9; ++k) asm volatile("" : "+v"(m.m[k].re), "+v"(m.m[k].im));
+    __builtin_amdgcn_sched_barrier(0);
+}
+
 // The fused pass with the neighbour links staged in LDS.  A block owns a
 // TX x TY tile of (x, y) and ZC consecutive z planes of one configuration
 // (blockIdx.y); thread (site of the tile, direction i) works on (x, y, z, i)
-// for z in its run.  LDS holds a ring of three z planes of links, each the
-// tile with a one-site halo in x and y, all three directions and nine
-// elements ([slot][dir * 9 + e][halo site]); planes z - 1, z, z + 1 serve
-// every staple of plane z (the 13 links of (x, i) lie in them).  The next
-// plane streams into registers while plane z is computed and replaces plane
-// z - 1 afterwards, so each link is read from HBM once per run of ZC planes
+// for z in its run.  The staples of plane z take U_x and U_y from planes z and
+// z + 1, U_z from planes z - 1 and z, and from plane z - 1 the thread's own link,
+// which it keeps: LDS holds two planes of each, the tile with a one-site halo in x
+// and y and nine elements ([slot][dir * 9 + e][halo site] and [slot][e][halo site]).
+// The next planes of both stream into registers while plane z is computed and replace
+// the older ones afterwards, so each link is read from HBM once per run of ZC planes
 // (plus the x/y halo, from L2, and two planes per run).  Per (site, dir) the arithmetic is that
 // of k_fused with full neighbour links (reu as there).  The lattice extents
 // must be multiples of TX, TY and ZC.
+// Bound by cache line requests to L2 (each row of a tile costs its lines and two
+// for the halo), next to 52 % of the vector rate: wider rows ask for fewer.  128^3:
+// 422 us per pass with three planes of every direction in LDS, 16 x 8, one block of 6
+// wavefronts per CU; 409 with two planes and two blocks; 302 with 32 x 8 (one block
+// of 12) and 280 with runs of 32 planes, 4.7 TB/s of the 1.31 GB that must move.  The loads
+// come before the staples: after them 10 % slower.
 template <typename R, int TX, int TY, int ZC, bool NT>
-__global__ __launch_bounds__(TX *TY * 3) void k_fused_tile(lf_batch<R> bt, geom g, R dt, int xcd, int reu)
+__global__ __launch_bounds__(TX *TY * 3, 3) void k_fused_tile(lf_batch<R> bt, geom g, R dt, int xcd, int reu)
 {
     constexpr int HX = TX + 2, HY = TY + 2, HS = HX * HY;
     constexpr int NTH = TX * TY * 3;
-    constexpr int PL = 27 * HS;                 // complex numbers per plane
-    constexpr int PER = (PL + NTH - 1) / NTH;   // per thread and plane
-    __shared__ cplx<R> lds[3 * PL];
+    constexpr int PL = 27 * HS, PXY = 18 * HS;  // complex numbers per plane, and of U_x and U_y
+    // the wavefronts load the elements of a plane 64 halo sites at a time: a
+    // wavefront keeps to one chunk of halo sites and takes every DSTEP-th element
+    constexpr int NCH = (HS + 63) / 64, DSTEP = NTH / 64 / NCH, PER = (27 + DSTEP - 1) / DSTEP;
+    static_assert(NTH / 64 % NCH == 0, "whole chunks of halo sites for every wavefront");
+    static_assert(18 % DSTEP == 0, "an element step must not mix U_x, U_y with U_z");
+    __shared__ cplx<R> lxy[2 * PXY], lz[2 * (PL - PXY)];
     const cplx<R> *__restrict__ uin = bt.uin[blockIdx.y];
     cplx<R> *__restrict__ uout = bt.uout[blockIdx.y];
     R *__restrict__ ef = bt.ef[blockIdx.y];
@@ -297,34 +315,42 @@ __global__ __launch_bounds__(TX *TY * 3) void k_fused_tile(lf_batch<R> bt, geom 
     const int64_t plane = (int64_t)g.n0 * g.n1;
     auto wrapz = [&](int z) { return z < 0 ? z + g.n2 : (z >= g.n2 ? z - g.n2 : z); };
 
-    cplx<R> pre[PER];
-    auto gload = [&](int z) {
-        const int zz = wrapz(z);
-#pragma unroll
-        for (int k = 0; k < PER; ++k) {
-            const int q = t + k * NTH;
-            if (q < PL) {
-                const int hs = q % HS, de = q / HS;
-                const int hx = hs % HX, hy = hs / HX;
-                int gx = x0 - 1 + hx, gy = y0 - 1 + hy;
-                gx = gx < 0 ? gx + g.n0 : (gx >= g.n0 ? gx - g.n0 : gx);
-                gy = gy < 0 ? gy + g.n1 : (gy >= g.n1 ? gy - g.n1 : gy);
-                pre[k] = uin[(int64_t)de * vol + gx + (int64_t)g.n0 * gy + plane * zz];
-            }
-        }
-    };
-    auto sstore = [&](int slot) {
-#pragma unroll
-        for (int k = 0; k < PER; ++k) {
-            const int q = t + k * NTH;
-            if (q < PL) lds[slot * PL + q] = pre[k];
-        }
-    };
-    for (int p = 0; p < 3; ++p) {
-        gload(z0 - 1 + p);
-        sstore(p);
+    // U_x and U_y of plane z, U_z of plane z - 1
+    const int wv = __builtin_amdgcn_readfirstlane(t / 64), de0 = wv / NCH;
+    const int hs = wv % NCH * 64 + (t & 63);
+    uint32_t off;
+    {
+        const int h = hs < HS ? hs : HS - 1;
+        int gx = x0 - 1 + h % HX, gy = y0 - 1 + h / HX;
+        gx = gx < 0 ? gx + g.n0 : (gx >= g.n0 ? gx - g.n0 : gx);
+        gy = gy < 0 ? gy + g.n1 : (gy >= g.n1 ? gy - g.n1 : gy);
+        off = (uint32_t)(gx + g.n0 * gy);
     }
-    __syncthreads();
+    auto gload = [&](int z, cplx<R> (&pre)[PER]) {
+        const int64_t pxy = plane * wrapz(z), pz = plane * wrapz(z - 1);
+        uint32_t at = off;
+        asm volatile("" : "+v"(at)); // scalar base and 32-bit offset, not a 64-bit address per element kept over the run
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            // past the last element: read again, not stored
+            const int de = (k + 1) * DSTEP <= 27 || de0 + k * DSTEP < 27 ? de0 + k * DSTEP : 26;
+            pre[k] = *at32(uin + ((int64_t)de * vol + (k * DSTEP < 18 ? pxy : pz)), at);
+        }
+    };
+    auto sstore = [&](int slot, const cplx<R> (&pre)[PER]) {
+        if (hs >= HS) return;
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            const int de = de0 + k * DSTEP;
+            if ((k + 1) * DSTEP <= 27 || de < 27)
+                (k * DSTEP < 18 ? lxy + slot * PXY : lz + slot * (PL - PXY) - PXY)[de * HS + hs] = pre[k];
+        }
+    };
+    for (int p = 0; p < 2; ++p) {
+        cplx<R> first[PER];
+        gload(z0 + p, first);
+        sstore(p, first);
+    }
 
     // TX * TY is a multiple of 64, so the direction is the same for a whole
     // wavefront: made scalar, every offset derived from it is scalar too
@@ -332,11 +358,22 @@ __global__ __launch_bounds__(TX *TY * 3) void k_fused_tile(lf_batch<R> bt, geom 
     const int i = __builtin_amdgcn_readfirstlane(t / (TX * TY));
     const int r = t - i * (TX * TY);
     const int tx = r % TX, ty = r / TX;
-    // link of direction d at offset (dx, dy) in plane z + pz (pz = -1, 0, 1)
-    int slot_of[3];
+    const uint32_t col = (uint32_t)(x0 + tx + g.n0 * (y0 + ty));
+    // this thread's link of plane z - 1 (used for i = x, y)
+    mat3<R> below;
+    {
+        const cplx<R> *b = uin + ((int64_t)i * 9 * vol + plane * wrapz(z0 - 1));
+#pragma unroll
+        for (int e = 0; e < 9; ++e) below.m[e] = *at32(b + (int64_t)e * vol, col);
+    }
+    __syncthreads();
+
+    int par = 0; // slot of U_x, U_y at z and of U_z at z - 1
+    // link of direction d at offset (dx, dy) in plane z + pz
     auto lnk = [&](int pz, int d, int dx, int dy) {
         mat3<R> m;
-        const cplx<R> *b = lds + slot_of[pz + 1] * PL + d * 9 * HS + (tx + 1 + dx) + HX * (ty + 1 + dy);
+        const int h = (tx + 1 + dx) + HX * (ty + 1 + dy);
+        const cplx<R> *b = d == 2 ? lz + (par ^ (pz + 1)) * (PL - PXY) + h : lxy + (par ^ pz) * PXY + d * 9 * HS + h;
 #pragma unroll
         for (int e = 0; e < 9; ++e) m.m[e] = b[e * HS];
         return m;
@@ -344,10 +381,9 @@ __global__ __launch_bounds__(TX *TY * 3) void k_fused_tile(lf_batch<R> bt, geom 
     for (int kz = 0; kz < ZC; ++kz) {
         const int z = z0 + kz;
         const bool more = kz + 1 < ZC;
-        if (more) gload(z + 2);
-        slot_of[0] = kz % 3;
-        slot_of[1] = (kz + 1) % 3;
-        slot_of[2] = (kz + 2) % 3;
+        par = kz & 1;
+        cplx<R> next[PER];
+        if (more) gload(z + 2, next);
         // staples, k in increasing order as in the reference's sum
         mat3<R> sum;
         set_zero(sum);
@@ -359,24 +395,43 @@ __global__ __launch_bounds__(TX *TY * 3) void k_fused_tile(lf_batch<R> bt, geom 
             const int pk = k == 2 ? 1 : 0;                   // plane of x + k
             const int pmk = k == 2 ? -1 : 0;                 // plane of x - k
             const int pik = (i == 2 ? 1 : 0) + (k == 2 ? -1 : 0); // plane of x + i - k
-            const mat3<R> ss = staple_pair(lnk(pi, k, ix, iy), lnk(pk, i, kx, ky), lnk(0, k, 0, 0),
-                                           lnk(pik, k, ix - kx, iy - ky), lnk(pmk, i, -kx, -ky), lnk(pmk, k, -kx, -ky));
+            // upper, then lower staple: both at once do not fit the registers of
+            // three wavefronts per SIMD
+            mat3<R> ss = staple_up(lnk(pi, k, ix, iy), lnk(pk, i, kx, ky), lnk(0, k, 0, 0));
+            stage_end(ss);
+            const mat3<R> sd = staple_down(lnk(pik, k, ix - kx, iy - ky), k == 2 ? below : lnk(0, i, -kx, -ky),
+                                           lnk(pmk, k, -kx, -ky));
 #pragma unroll
-            for (int m = 0; m < 9; ++m) sum.m[m] = sum.m[m] + coef * ss.m[m];
+            for (int m = 0; m < 9; ++m) {
+                ss.m[m] = ss.m[m] + sd.m[m];
+                sum.m[m] = sum.m[m] + coef * ss.m[m];
+            }
+            stage_end(sum);
         }
-        const int64_t s = (x0 + tx) + (int64_t)g.n0 * (y0 + ty) + plane * z;
+        const int64_t pz = plane * z;
+        uint32_t at = col;
+        asm volatile("" : "+v"(at));
         R e[8];
 #pragma unroll
-        for (int a = 0; a < 8; ++a) e[a] = ld_e<NT>(ef + ((int64_t)i * 8 + a) * vol + s);
+        for (int a = 0; a < 8; ++a) e[a] = ld_e<NT>(at32(ef + (((int64_t)i * 8 + a) * vol + pz), at));
         mat3<R> ui = lnk(0, i, 0, 0);
+        below = ui;
         apply_force(ui, sum, e);
 #pragma unroll
-        for (int a = 0; a < 8; ++a) st_e<NT>(ef + ((int64_t)i * 8 + a) * vol + s, e[a]);
+        for (int a = 0; a < 8; ++a) st_e<NT>(at32(ef + (((int64_t)i * 8 + a) * vol + pz), at), e[a]);
         if (reu) project_su3(ui);
-        store_link_out<NT>(uout, vol, i, s, evolve_link(ui, e, dt));
-        __syncthreads(); // the oldest plane is no longer read
-        if (more) sstore(kz % 3);
-        __syncthreads();
+        const mat3<R> un = evolve_link(ui, e, dt);
+#pragma unroll
+        for (int q = 0; q < 9; ++q) {
+            cplx<R> *o = at32(uout + (((int64_t)i * 9 + q) * vol + pz), at);
+            if (NT) store_nt(o, un.m[q]);
+            else *o = un.m[q];
+        }
+        if (more) {
+            __syncthreads(); // the older planes are no longer read
+            sstore(par, next);
+            __syncthreads();
+        }
     }
 }
 
@@ -699,8 +754,8 @@ struct lf_variant {
     int nt;  // streaming loads/stores of E and of the new links
     int rec; // neighbour links read as two rows (third rebuilt)
 };
-// Modes 3 and 4 are the LDS-tiled fused pass (k_fused_tile, FP32, 16 x 8
-// tiles, three planes in LDS, runs of 16 or 8 z planes); bs is the tile's
+// Modes 3 and 4 are the LDS-tiled fused pass (k_fused_tile, FP32, 16 x 8 or
+// 32 x 8 tiles, runs of 16 (or 32) and 8 z planes); bs is the narrow tile's
 // thread count.  Their first and last half steps use the consecutive-site
 // map.
 static const lf_variant LF_VARIANTS[] = {
@@ -711,6 +766,8 @@ static const lf_variant LF_VARIANTS[] = {
 constexpr int LF_NVARIANTS = sizeof(LF_VARIANTS) / sizeof(LF_VARIANTS[0]);
 constexpr int LF_DEFAULT = 11; // {256, 8, 0, 0, 0}: used without tuning, valid on every lattice
 
+constexpr int64_t LF_CUS = 256;
+
 struct lf_choice {
     int precision;
     int n[3]; // lattice extents the choice was tuned on
@@ -720,8 +777,9 @@ static std::vector<lf_choice> g_lf_choice;
 static int g_autotune = -1; // -1: unset (env NRQ_AUTOTUNE, default on)
 
 // Whether shape `variant` applies to lattice g at storage precision prec
-// (64 or 32).  The LDS tiles are FP32 only: a 16 x 4 FP64 tile fits LDS, but
-// at one wavefront per SIMD its prefetch registers do not fit.
+// (64 or 32).  The LDS tiles are FP32 only: a 16 x 8 FP64 tile fits LDS, but its
+// registers do not fit two wavefronts per SIMD (240 bytes of scratch per thread):
+// 128^3 1351 us per step against 751 for the untiled kernel, 64^3 156 against 88.
 static bool variant_ok(int variant, const geom &g, int prec)
 {
     const lf_variant v = LF_VARIANTS[variant];
@@ -758,13 +816,40 @@ static lf_map make_map(int variant, const geom &g)
     return make_lf_map(g, v.bs, v.xcd, v.mode, 3);
 }
 
-template <typename R, int ZC, bool NTV>
-static void launch_tile(const lf_batch<R> &bt, int nb, const geom &g, R dt, int xcd, int reu)
+template <typename R, int TX, int ZC, bool NTV>
+static void launch_tile_of(const lf_batch<R> &bt, int nb, const geom &g, R dt, int xcd, int reu)
 {
-    constexpr int TX = 16, TY = 8;
+    constexpr int TY = 8;
     const unsigned total = (unsigned)(g.n0 / TX) * (unsigned)(g.n1 / TY) * (unsigned)(g.n2 / ZC);
     hipLaunchKernelGGL((k_fused_tile<R, TX, TY, ZC, NTV>), dim3(total, (unsigned)nb), dim3(TX * TY * 3), 0, stream(), bt,
                        g, dt, xcd, reu);
+}
+
+// 32 x 8 tiles where n0 allows them and they give work to more than half of the
+// CUs (one block of a 32 x 8 tile fills a CU, two of 16 x 8): us per step of the
+// fastest 16 x 8 shape and of the 32 x 8 one, and the latter's blocks: 128^3 409
+// and 302 (512), 160x96x96 298 and 225 (720), 96^3 197 and 142 (216),
+// 64x64x128 89 and 73 (256), 64x96x96 147 and 134 (144), 64^3 44 and 58 (128),
+// 96x64x64 with 16-plane runs 80 and 106 (96).
+template <typename R, int ZC, bool NTV>
+static void launch_tile(const lf_batch<R> &bt, int nb, const geom &g, R dt, int xcd, int reu)
+{
+    if (g.n0 % 32 == 0 && (int64_t)(g.n0 / 32) * (g.n1 / 8) * (g.n2 / ZC) * nb > LF_CUS / 2)
+        launch_tile_of<R, 32, ZC, NTV>(bt, nb, g, dt, xcd, reu);
+    else
+        launch_tile_of<R, 16, ZC, NTV>(bt, nb, g, dt, xcd, reu);
+}
+
+// Mode 3: runs of 32 planes (two extra planes are read per run) where 32 x 8 tiles
+// then still give every CU a block, else of 16: 128^3 280 us per step with 32 and
+// 302 with 16, 128x128x64 (128 blocks) 255 and 153.
+template <typename R, bool NTV>
+static void launch_runs(const lf_batch<R> &bt, int nb, const geom &g, R dt, int xcd, int reu)
+{
+    if (g.n0 % 32 == 0 && g.n2 % 32 == 0 && (int64_t)(g.n0 / 32) * (g.n1 / 8) * (g.n2 / 32) * nb >= LF_CUS)
+        launch_tile_of<R, 32, 32, NTV>(bt, nb, g, dt, xcd, reu);
+    else
+        launch_tile<R, 16, NTV>(bt, nb, g, dt, xcd, reu);
 }
 
 template <typename R> static void launch_links(int variant, const lf_batch<R> &bt, int nb, const geom &g, R dt)
@@ -796,7 +881,7 @@ static void launch_fused(int variant, const lf_batch<R> &bt, int nb, const geom 
     const lf_variant tv = LF_VARIANTS[variant];
     if constexpr (sizeof(R) == 4) if (tv.mode >= 3) {
         if (tv.mode == 3)
-            tv.nt ? launch_tile<R, 16, true>(bt, nb, g, dt, tv.xcd, reu) : launch_tile<R, 16, false>(bt, nb, g, dt, tv.xcd, reu);
+            tv.nt ? launch_runs<R, true>(bt, nb, g, dt, tv.xcd, reu) : launch_runs<R, false>(bt, nb, g, dt, tv.xcd, reu);
         else
             tv.nt ? launch_tile<R, 8, true>(bt, nb, g, dt, tv.xcd, reu) : launch_tile<R, 8, false>(bt, nb, g, dt, tv.xcd, reu);
         return;

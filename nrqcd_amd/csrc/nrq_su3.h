@@ -260,17 +260,29 @@ template <typename R> __device__ __forceinline__ void su3_row3(mat3<R> &m)
 // conjugated cross product of rows 1 and 2, 48 fewer multiply-adds per
 // staple.  The difference from the full product is of the order of the links'
 // unitarity error (FP64 rounding for FP64 links, FP32 rounding for FP32).
+template <typename R> __device__ __forceinline__ mat3<R> staple_up(const mat3<R> &a, const mat3<R> &b, const mat3<R> &c)
+{
+    mat3<R> su, t;
+    mul_nd_top(a, b, t);
+    mul_nd_top(t, c, su);
+    su3_row3(su);
+    return su;
+}
+
+template <typename R> __device__ __forceinline__ mat3<R> staple_down(const mat3<R> &d, const mat3<R> &e, const mat3<R> &f)
+{
+    mat3<R> sd, t;
+    mul_dd_top(d, e, t);
+    mul_top(t, f, sd);
+    su3_row3(sd);
+    return sd;
+}
+
 template <typename R>
 __device__ __forceinline__ mat3<R> staple_pair(const mat3<R> &a, const mat3<R> &b, const mat3<R> &c, const mat3<R> &d,
                                               const mat3<R> &e, const mat3<R> &f)
 {
-    mat3<R> su, sd, t;
-    mul_nd_top(a, b, t);
-    mul_nd_top(t, c, su);
-    su3_row3(su);
-    mul_dd_top(d, e, t);
-    mul_top(t, f, sd);
-    su3_row3(sd);
+    mat3<R> su = staple_up(a, b, c), sd = staple_down(d, e, f);
 #pragma unroll
     for (int k = 0; k < 9; ++k) su.m[k] = su.m[k] + sd.m[k];
     return su;

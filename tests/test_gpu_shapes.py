@@ -81,6 +81,33 @@ def test_every_leapfrog_shape_matches_oracle_fp32(nrq, oracle, lattice, pinned, 
     assert any(nrq.leapfrog_shapes()[k]["tiling"].startswith("LDS") for k in tried)
 
 
+# blocks of 32 x 8 tiles in the batch: 8-plane runs 136 and 128, 16-plane runs 144, 32-plane runs 256
+@pytest.mark.parametrize("ext,nb,runs", [((64, 16, 16), 17, "8-plane"), ((64, 16, 16), 16, "8-plane"),
+                                         ((32, 24, 48), 16, "16-plane"), ((64, 64, 32), 16, "16-plane")])
+def test_wide_lds_tiles_of_a_batch_match_single_updates(nrq, lattice, pinned, ext, nb, runs):
+    """A batch large enough for the 32 x 8 tiles (and just not) against each of two
+    different members advanced alone, which take 16 x 8 tiles and runs of 16: the same
+    arithmetic per site and direction, so equal bit for bit."""
+    _say(f"wide LDS tiles, {nb} x {ext}, {runs} runs")
+    lattice(ext, SP)
+    nrq.leapfrog_set_shape(next(k for k, s in enumerate(nrq.leapfrog_shapes())
+                                if s["tiling"].startswith("LDS") and f" {runs}" in s["tiling"]))
+    src = []
+    for k in range(2):
+        nrq.random_init(31 + k)
+        g = nrq.GaugeConfiguration(nrq.NRQ_PRECISION_FP32)
+        g.TransversePolarisedOccupiedInit_Box(0.5, 1.0, 1.0)
+        src.append(g)
+    ens = [src[k % 2].copy() for k in range(nb)]
+    nrq.leapfrog_batch(ens, 1.0, 4)
+    for g in src:
+        g.Update(1.0, 4)
+    want = [g.download() for g in src]
+    for k in (0, 1, nb - 2, nb - 1):
+        U, E = ens[k].download()
+        assert np.array_equal(U, want[k % 2][0]) and np.array_equal(E, want[k % 2][1]), k
+
+
 def test_pinned_shape_that_does_not_apply_is_an_error(nrq, lattice, pinned):
     ext = (5, 6, 7)  # the 16-wide tiles need an x extent of at least 16
     _say("pinned shape that does not apply")
