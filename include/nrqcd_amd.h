@@ -284,7 +284,7 @@ typedef struct {
     double max_true_relres;  /* worst FP64 true relative residual ||b-Ax||/||b|| */
 } nrq_solve_stats;
 
-#define NRQ_SOLVER_GMRES_FP64 0   /* GMRES(m), classical Gram-Schmidt, FP64, zero guess */
+#define NRQ_SOLVER_GMRES_FP64 0   /* GMRES(m), FP64, zero guess */
 #define NRQ_SOLVER_GMRES_MIXED 1  /* FP32 GMRES(m) corrections inside FP64 iterative
                                      refinement on the true residual, first-order
                                      initial guess */

@@ -1,6 +1,6 @@
 // nrq_cn.hip -- NRQCD heavy-quark Crank-Nicolson step (nrqcd.f90:1053-1168)
 // with a matrix-free covariant-Laplacian stencil and a batched restarted
-// GMRES(m) with classical Gram-Schmidt that replaces PETSc KSP.
+// GMRES(m) that replaces PETSc KSP.
 //
 // Storage.  For the kinetic Hamiltonian H = -c1 D^2/2M the 6x6 propagator
 // P(d, j, x), d = 2(colour-1) + spin-1 (the C2CS = U (x) 1_2 ordering of

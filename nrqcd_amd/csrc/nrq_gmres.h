@@ -1,8 +1,9 @@
 // nrq_gmres.h -- vector kernels and device-side scalars of batched GMRES(m),
 // shared by the kinetic Crank-Nicolson solvers and the full Hamiltonian.
 //
-// After the operator, an Arnoldi step of all slots is k_mdot, k_gm_dots,
-// k_cgs_update and k_gm_step; a cycle is k_gm_begin, its steps, k_gm_solve and
+// After the operator, an Arnoldi step of all slots is k_mdot, k_gm_dots (both
+// replaced by k_gm_lanczos for a shifted Hermitian operator), k_cgs_update and
+// k_gm_step; a cycle is k_gm_begin, its steps, k_gm_solve and
 // k_xupdate.  None of them needs the host, and every sum of a slot runs in an
 // order that depends on the vector length alone.
 #pragma once
@@ -212,6 +213,34 @@ static __global__ __launch_bounds__(256) void k_gm_dots(const cplx<double> *__re
     }
 }
 
+// Step j of slot r = blockIdx.x for A = 1 + beta K with K Hermitian: the Krylov
+// space of A is that of K, so <v_i, A v_j> vanishes for i < j - 1 (Lanczos), and
+//   <v_j, A v_j> = 1 + beta kappa,  kappa = <v_j, K v_j> from the operator's partials,
+//   <v_{j-1}, A v_j> = beta conj(<v_j, A v_{j-1}> / beta) = (beta / conj(beta)) ||W_j||.
+// The column of H and the two coefficients of the Gram-Schmidt update.
+static __global__ __launch_bounds__(VTHREADS) void k_gm_lanczos(const double *__restrict__ partial, int64_t nblk, int j,
+                                                                const cplx<double> *__restrict__ beta, gm_state st)
+{
+    const int r = blockIdx.x;
+    if (!st.cyc[r]) return;
+    __shared__ double sh[VTHREADS / 64];
+    double k = 0;
+    for (int64_t b = threadIdx.x; b < nblk; b += VTHREADS) k += partial[(int64_t)r * nblk + b];
+    k = block_sum(k, sh);
+    if (threadIdx.x != 0) return;
+    const double *sc = st.sc + (int64_t)r * (st.m + 1);
+    cplx<double> *H = st.H + ((int64_t)r * st.m + j) * (st.m + 1), *coef = st.coef + (int64_t)r * (st.m + 1);
+    const cplx<double> b = beta[r];
+    k *= sc[j] * sc[j];
+    H[j] = {1.0 + b.re * k, b.im * k};
+    coef[j] = sc[j] * H[j];
+    if (j == 0) return;
+    for (int i = 0; i < j - 1; ++i) H[i] = {0.0, 0.0};
+    const double b2 = b.re * b.re + b.im * b.im, h = b2 > 0 && sc[j] > 0 ? 1.0 / (sc[j] * b2) : 0.0;
+    H[j - 1] = h * (b * b);
+    coef[j - 1] = sc[j - 1] * H[j - 1];
+}
+
 // out[r] = sum_b partial[r * nblk + b] for the slot r = blockIdx.x if
 // active[r] (active may be null); fixed summation order.  FOLD_THREADS
 // threads with four independent sums each keep enough loads in flight for
@@ -241,10 +270,10 @@ static __global__ __launch_bounds__(FOLD_THREADS) void k_fold_slots(const double
     }
 }
 
-// Gram-Schmidt update W_nv = sc_j (A W_j) - sum_{i < nv} coef_i W_i (j = nv - 1,
-// A W_j in w, in place) and partial ||W_nv||^2
+// Gram-Schmidt update W_nv = sc_j (A W_j) - sum_{lo <= i < nv} coef_i W_i
+// (j = nv - 1, A W_j in w, in place) and partial ||W_nv||^2
 template <typename T>
-__global__ __launch_bounds__(VTHREADS) void k_cgs_update(gm_basis<T> basis, int nv, cplx<T> *__restrict__ w, int64_t n, int nf,
+__global__ __launch_bounds__(VTHREADS) void k_cgs_update(gm_basis<T> basis, int lo, int nv, cplx<T> *__restrict__ w, int64_t n, int nf,
                                                          gm_state st, double *__restrict__ partial)
 {
     const int r = blockIdx.y;
@@ -257,7 +286,7 @@ __global__ __launch_bounds__(VTHREADS) void k_cgs_update(gm_basis<T> basis, int 
     for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (int64_t)gridDim.x * blockDim.x) {
         const cplx<T> w0 = wr[k];
         cplx<double> a = {scj * (double)w0.re, scj * (double)w0.im};
-        for (int i = 0; i < nv; ++i) {
+        for (int i = lo; i < nv; ++i) {
             const cplx<T> v = basis.at(i, r, nf, n)[k];
             a = a - h[i] * cplx<double>{(double)v.re, (double)v.im};
         }

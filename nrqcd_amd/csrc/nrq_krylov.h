@@ -16,7 +16,7 @@ constexpr int NFIELDS_PER_HEAVY = 24; // colour-vector fields per NRQCDField
 constexpr int NSLOTS = 48;            // right-hand sides of one batched solve
 
 enum krylov_kind {
-    KRYLOV_GMRES_FP64 = 0,  // GMRES(m), classical Gram-Schmidt, FP64, zero guess
+    KRYLOV_GMRES_FP64 = 0,  // GMRES(m), FP64, zero guess
     KRYLOV_GMRES_MIXED = 1, // FP32 GMRES(m) corrections inside FP64 iterative refinement
     KRYLOV_CHEB_FP64 = 2,   // Chebyshev iteration on the known spectral segment, FP64
     KRYLOV_CHEB_MIXED = 3,  // FP32 Chebyshev corrections inside FP64 iterative refinement

@@ -403,3 +403,34 @@ def test_multi_mass_batch_matches_single_updates(nrq, oracle, cn, kind):
             oracle.cn_update(U, Q, A, m, C1, 1.0, 1e-13)
         assert np.max(np.abs(Qb - Q)) < 1e-10 * np.max(np.abs(Q))
         assert np.max(np.abs(Ab - A)) < 1e-10 * np.max(np.abs(A))
+
+
+@pytest.mark.parametrize("kind", ["GMRES_FP64", "GMRES_MIXED"])
+@pytest.mark.parametrize("restart,step", [(1, 1.0), (2, 1.0), (8, 1000.0), (30, 1000.0), (30, 0.0)])
+def test_gmres_recurrence_on_stiff_steps(nrq, oracle, cn, kind, restart, step):
+    """The Krylov basis is orthogonalised against its last two vectors only (K is
+    Hermitian): cycles of 1, 2, 8 and 30 on the usual step, one a thousand times as
+    long and none.  |beta| kmax = step * 0.05 / 4 * 6 = 75 at most; both sides leave
+    a residual of 1e-12 ||y||, ||y|| <= 76 ||psi||, and the inverse has norm <= 1:
+    propagators within 2 * 76e-12 of their norm."""
+    ext = (6, 5, 4)
+    _say(f"GMRES recurrence {kind} m={restart} step {step}")
+    cn(ext, SP)
+    oracle.lattice_init(ext, SP)
+    U, E = oracle.box_init(4, 0.7, 1.0, 1.0)
+    nrq.nrqcd_set_solver(getattr(nrq, "NRQ_SOLVER_" + kind), restart, 10000)
+    g = nrq.GaugeConfiguration()
+    g.upload(U, E)
+    rng = np.random.default_rng(8)
+    v = 6 * 5 * 4
+    Q = np.asfortranarray(rng.normal(size=(6, 6, v)) + 1j * rng.normal(size=(6, 6, v)))
+    A = np.asfortranarray(rng.normal(size=(6, 6, v)) + 1j * rng.normal(size=(6, 6, v)))
+    h = nrq.NRQCDField()
+    h.upload(Q, A)
+    st = h.Update(g, 2.0, C1, step)
+    assert st.max_true_relres <= 1e-12
+    rc, _ = oracle.cn_update(U, Q, A, 2.0, C1, step, 1e-12)
+    assert rc == 0
+    Qg, Ag = h.download()
+    assert np.linalg.norm(Qg - Q) < 1.6e-10 * np.linalg.norm(Q)
+    assert np.linalg.norm(Ag - A) < 1.6e-10 * np.linalg.norm(A)
