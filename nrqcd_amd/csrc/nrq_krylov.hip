@@ -310,7 +310,7 @@ __global__ __launch_bounds__(SBS_WAVE, CN_WAVES) void k_krylov_op(const cplx<RL>
 
 // Right-hand side and initial guess of a CN step for slot r:
 //   y_r = psi_r + alpha_r K psi_r                     (S psi, nrqcd.f90:1112)
-//   x_r = psi_r + g_r K psi_r  (guess != 0)  or  x_r = 0
+//   x_r = psi_r + g_r K psi_r  (guess != 0)  or  x_r = 0  (x.p[r] null: neither)
 // with g_r = alpha_r - beta_r the first-order expansion of
 // (1 + beta K)^-1 (1 + alpha K).  Partial ||y_r||^2 per site block.  With wk,
 // K psi_r also goes to kout in FP32: the guess's residual is exactly
@@ -350,7 +350,8 @@ __global__ __launch_bounds__(SBS_WAVE, CN_WAVES) void k_cn_rhs(const cplx<RL> *_
                 const cplx<double> kf = dsum * v0[q][c] - 0.5 * hop[q][c];
                 const cplx<double> yv = v0[q][c] + a * kf;
                 store_nt(at32(y.p[r] + cv, (uint32_t)s), yv);
-                store_nt(at32(x.p[r] + cv, (uint32_t)s), guess ? v0[q][c] + gc * kf : cplx<double>{0.0, 0.0});
+                if (x.p[r])
+                    store_nt(at32(x.p[r] + cv, (uint32_t)s), guess ? v0[q][c] + gc * kf : cplx<double>{0.0, 0.0});
                 if (wk) store_nt(at32(kout.p[r] + cv, (uint32_t)s), cplx<float>{(float)kf.re, (float)kf.im});
                 nrm[q] += nrm2(yv);
             }
@@ -1630,7 +1631,9 @@ static int cn_step_t(const cplx<RL> *u, int R, const std::vector<zc> &alpha, con
     const slots<double> tpsi = psi_slots(R), ty = ws_slots(g_ws.y, R), tx = ws_slots(g_ws.x, R);
     // mixed Chebyshev from the guess takes K psi (FP32) for its first correction
     const int wk = guess && p.kind == KRYLOV_CHEB_MIXED ? 1 : 0;
-    const int64_t nsb = launch_rhs<RL>(u, R, tpsi, ty, tx, guess ? 1 : 0, ws_slots(g_ws.t32, R), wk);
+    // GMRES from a zero guess writes x whole
+    const bool no_x = !guess && (p.kind == KRYLOV_GMRES_FP64 || p.kind == KRYLOV_FGMRES_CNN);
+    const int64_t nsb = launch_rhs<RL>(u, R, tpsi, ty, no_x ? slots<double>{} : tx, guess ? 1 : 0, ws_slots(g_ws.t32, R), wk);
     NRQ_HIP(hipGetLastError());
     if (int e = fold_slots(g_ws.spart, nsb, R, nullptr, g_ws.nrm + workspace::NRM_Y, g_ws.nbuf + workspace::NRM_Y)) return e;
     cplx<double> *xsol = g_ws.x;
