@@ -22,10 +22,11 @@ __device__ __forceinline__ double lane_max(double v)
 // Maximum of a row, in every lane (all 64 lanes must call).
 __device__ __forceinline__ double row_max(const double *__restrict__ row) { return lane_max(row[threadIdx.x & 63]); }
 
-// Raises the row to at least v >= 0 (one lane per block or wavefront calls).
+// Raises the row to at least v >= 0 (one lane per block or wavefront calls); a
+// NaN raises nothing, as fmax ignores it everywhere else.
 __device__ __forceinline__ void row_raise(double *row, double v)
 {
-    atomicMax((unsigned long long *)row + blockIdx.x % MAXROW, (unsigned long long)__double_as_longlong(v));
+    atomicMax((unsigned long long *)row + blockIdx.x % MAXROW, (unsigned long long)__double_as_longlong(fmax(v, 0.0)));
 }
 
 } // namespace nrq

@@ -51,6 +51,22 @@ def test_gaugefix_matches_oracle(nrq, oracle, lattice):
     assert g.GetEnergy() == pytest.approx(oracle.energy(U, E), rel=1e-12)
 
 
+def test_gaugefix_deviation_ignores_what_is_not_a_number(nrq, oracle, lattice):
+    """The deviation is a maximum that drops NaN.  With all of the first 64 links
+    of U_x not numbers, the rest of the lattice still gives a deviation above the
+    tolerance; the transformation spreads the NaN everywhere, which leaves 0."""
+    ext = (16, 6, 4)
+    _say("gauge fixing with NaN links")
+    _setup(nrq, oracle, lattice, ext)
+    U, E = _evolved(oracle)
+    U = U.copy(order="F")
+    U[:, :, 0, :64] = np.nan
+    g = nrq.GaugeConfiguration()
+    g.upload(U, E)
+    its, dev = g.CoulombGaugefixing(1e-10, 0.08, 20)
+    assert its == 1 and dev == 0.0
+
+
 def test_gaugefix_iteration_cap_and_defaults(nrq, oracle, lattice):
     ext = (6, 4, 4)
     _say("gauge fixing cap and defaults")
