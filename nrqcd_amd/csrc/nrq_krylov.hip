@@ -663,6 +663,36 @@ template <typename T, bool FIN> struct tile_cheb {
 // vector kernels (grid: VBLOCKS x slots)
 // ---------------------------------------------------------------------------
 
+// Coefficients of a CN step, passed by value (three small copies from pageable
+// memory held the queue for longer than the launch of this kernel): cpar = alpha and
+// alpha - beta, beta, and every slot of mask active.
+struct step_params {
+    cplx<double> alpha[NSLOTS], beta[NSLOTS];
+    unsigned long long mask;
+};
+__global__ __launch_bounds__(64) void k_set_step(step_params p, cplx<double> *__restrict__ cpar, cplx<double> *__restrict__ beta,
+                                                 int *__restrict__ active)
+{
+    const int r = threadIdx.x;
+    if (r >= NSLOTS) return;
+    cpar[r] = p.alpha[r];
+    cpar[NSLOTS + r] = p.alpha[r] - p.beta[r];
+    beta[r] = p.beta[r];
+    active[r] = (int)(p.mask >> r & 1ull);
+}
+
+// The Chebyshev coefficients of nf slots and k steps (2 nf k <= CHEB_ARGS) into the
+// table of stride 2 NSLOTS.
+constexpr int CHEB_ARGS = 192;
+struct cheb_args {
+    cplx<double> v[CHEB_ARGS];
+};
+__global__ __launch_bounds__(CHEB_ARGS) void k_set_cheb(cheb_args a, int nf, int k, cplx<double> *__restrict__ tab)
+{
+    const int t = threadIdx.x;
+    if (t < 2 * nf * k) tab[(int64_t)2 * NSLOTS * (t / (2 * nf)) + t % (2 * nf)] = a.v[t];
+}
+
 // active[r] = bit r of mask
 __global__ __launch_bounds__(64) void k_set_mask(int *__restrict__ active, unsigned long long mask)
 {
@@ -1361,6 +1391,13 @@ static int cheb_table(int R, const std::vector<zc> &beta, int k, double kmax)
             tab[(size_t)2 * NSLOTS * j + 2 * r + 1] = {rho.real(), rho.imag()};
         }
     }
+    if (2 * R * k <= CHEB_ARGS) { // 12 slots and 8 steps, 48 and 2
+        cheb_args a = {};
+        for (int j = 0; j < k; ++j) std::copy_n(&tab[(size_t)2 * NSLOTS * j], 2 * R, &a.v[2 * R * j]);
+        hipLaunchKernelGGL(k_set_cheb, dim3(1), dim3(CHEB_ARGS), 0, stream(), a, R, k, g_ws.cheb);
+        NRQ_HIP(hipGetLastError());
+        return NRQ_OK;
+    }
     NRQ_HIP(hipMemcpyAsync(g_ws.cheb, tab.data(), sizeof(cplx<double>) * tab.size(), hipMemcpyHostToDevice, stream()));
     return NRQ_OK;
 }
@@ -1720,22 +1757,19 @@ int krylov_cn_step(const nrq_gauge *gf, cplx<double> *const *fields, int R, cons
     if (R <= 0) return NRQ_OK;
     if (R > NSLOTS) return fail(NRQ_ERR_ARG, "CN: %d fields exceed the batch of %d", R, NSLOTS);
     if (g_ws.vol != lat().g.vol || g_ws.rcap < R) return fail(NRQ_ERR_STATE, "CN: workspace not reserved for this solve");
-    std::vector<int> act(R, 1);
-    std::vector<cplx<double>> par(2 * NSLOTS, cplx<double>{0.0, 0.0});
+    step_params par = {};
     std::vector<zc> a(R), b(R);
     for (int r = 0; r < R; ++r) {
         if (!fields[r]) return fail(NRQ_ERR_ARG, "CN: null field %d", r);
         g_ws.fptr[r] = fields[r];
         a[r] = zc(alpha[r].re, alpha[r].im);
         b[r] = zc(beta[r].re, beta[r].im);
-        par[r] = alpha[r];
-        g_beta_host[r] = beta[r];
-        const zc g = a[r] - b[r];
-        par[NSLOTS + r] = {g.real(), g.imag()};
+        par.alpha[r] = alpha[r];
+        par.beta[r] = g_beta_host[r] = beta[r];
+        par.mask |= 1ull << r;
     }
-    if (int e = upload_active(act)) return e;
-    NRQ_HIP(hipMemcpyAsync(g_ws.cpar, par.data(), sizeof(cplx<double>) * par.size(), hipMemcpyHostToDevice, stream()));
-    NRQ_HIP(hipMemcpyAsync(g_ws.beta, beta, sizeof(cplx<double>) * R, hipMemcpyHostToDevice, stream()));
+    hipLaunchKernelGGL(k_set_step, dim3(1), dim3(64), 0, stream(), par, g_ws.cpar, g_ws.beta, g_ws.active);
+    NRQ_HIP(hipGetLastError());
     if (gf->precision == 64) return cn_step_t<double>((const cplx<double> *)gauge_links(gf), R, a, b, p, st);
     return cn_step_t<float>((const cplx<float> *)gauge_links(gf), R, a, b, p, st);
 }
