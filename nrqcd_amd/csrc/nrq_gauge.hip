@@ -284,11 +284,12 @@ template <typename R> __device__ __forceinline__ void stage_end(mat3<R> &m)
 // of k_fused with full neighbour links (reu as there).  The lattice extents
 // must be multiples of TX, TY and ZC.
 // Bound by cache line requests to L2 (each row of a tile costs its lines and two
-// for the halo), next to 52 % of the vector rate: wider rows ask for fewer.  128^3:
-// 422 us per pass with three planes of every direction in LDS, 16 x 8, one block of 6
-// wavefronts per CU; 409 with two planes and two blocks; 302 with 32 x 8 (one block
-// of 12) and 280 with runs of 32 planes, 4.7 TB/s of the 1.31 GB that must move.  The loads
-// come before the staples: after them 10 % slower.
+// for the halo) and by VALU issue (204 us at 128^3): wider rows ask for fewer lines.
+// 128^3, evolved box initial condition, us per step: 403 with three planes of every
+// direction in LDS, 16 x 8, one block of 6 wavefronts per CU; 415 with two planes and
+// two blocks; 323 with 32 x 8 (one block of 12) and 311 with runs of 32 planes,
+// 4.2 TB/s of the 1.31 GB that must move.  The loads come before the staples: after
+// them 10 % slower.
 template <typename R, int TX, int TY, int ZC, bool NT>
 __global__ __launch_bounds__(TX *TY * 3, 3) void k_fused_tile(lf_batch<R> bt, geom g, R dt, int xcd, int reu)
 {
@@ -779,7 +780,8 @@ static int g_autotune = -1; // -1: unset (env NRQ_AUTOTUNE, default on)
 // Whether shape `variant` applies to lattice g at storage precision prec
 // (64 or 32).  The LDS tiles are FP32 only: a 16 x 8 FP64 tile fits LDS, but its
 // registers do not fit two wavefronts per SIMD (240 bytes of scratch per thread):
-// 128^3 1351 us per step against 751 for the untiled kernel, 64^3 156 against 88.
+// 128^3 1351 us per step against 751 for the untiled kernel, 64^3 156 against 88
+// (cold links).
 static bool variant_ok(int variant, const geom &g, int prec)
 {
     const lf_variant v = LF_VARIANTS[variant];
@@ -827,10 +829,10 @@ static void launch_tile_of(const lf_batch<R> &bt, int nb, const geom &g, R dt, i
 
 // 32 x 8 tiles where n0 allows them and they give work to more than half of the
 // CUs (one block of a 32 x 8 tile fills a CU, two of 16 x 8): us per step of the
-// fastest 16 x 8 shape and of the 32 x 8 one, and the latter's blocks: 128^3 409
-// and 302 (512), 160x96x96 298 and 225 (720), 96^3 197 and 142 (216),
-// 64x64x128 89 and 73 (256), 64x96x96 147 and 134 (144), 64^3 44 and 58 (128),
-// 96x64x64 with 16-plane runs 80 and 106 (96).
+// fastest 16 x 8 shape and of the 32 x 8 one, and the latter's blocks: 128^3 415
+// and 323 (512), 160x96x96 303 and 242 (720), 96^3 201 and 147 (216),
+// 64x64x128 93 and 83 (256), 64x96x96 148 and 131 (144), 64^3 46 and 59 (128),
+// 96x64x64 with 16-plane runs 83 and 110 (96).
 template <typename R, int ZC, bool NTV>
 static void launch_tile(const lf_batch<R> &bt, int nb, const geom &g, R dt, int xcd, int reu)
 {
@@ -841,8 +843,8 @@ static void launch_tile(const lf_batch<R> &bt, int nb, const geom &g, R dt, int 
 }
 
 // Mode 3: runs of 32 planes (two extra planes are read per run) where 32 x 8 tiles
-// then still give every CU a block, else of 16: 128^3 280 us per step with 32 and
-// 302 with 16, 128x128x64 (128 blocks) 255 and 153.
+// then still give every CU a block, else of 16: 128^3 311 us per step with 32 and
+// 323 with 16, 128x128x64 (128 blocks) 257 and 162.
 template <typename R, bool NTV>
 static void launch_runs(const lf_batch<R> &bt, int nb, const geom &g, R dt, int xcd, int reu)
 {
