@@ -1,9 +1,9 @@
 // nrq_gmres.h -- vector kernels and device-side scalars of batched GMRES(m),
 // shared by the kinetic Crank-Nicolson solvers and the full Hamiltonian.
 //
-// After the operator, an Arnoldi step of all slots is k_mdot, k_gm_dots (both
-// replaced by k_gm_lanczos for a shifted Hermitian operator), k_cgs_update and
-// k_gm_step; a cycle is k_gm_begin, its steps, k_gm_solve and
+// After the operator, an Arnoldi step of all slots is k_mdot, k_gm_dots,
+// k_cgs_update and k_gm_step; for a shifted Hermitian operator k_lanczos_update
+// (after k_gm_lanczos on large lattices) and k_gm_step; a cycle is k_gm_begin, its steps, k_gm_solve and
 // k_xupdate.  None of them needs the host, and every sum of a slot runs in an
 // order that depends on the vector length alone.
 #pragma once
@@ -217,28 +217,94 @@ static __global__ __launch_bounds__(256) void k_gm_dots(const cplx<double> *__re
 // space of A is that of K, so <v_i, A v_j> vanishes for i < j - 1 (Lanczos), and
 //   <v_j, A v_j> = 1 + beta kappa,  kappa = <v_j, K v_j> from the operator's partials,
 //   <v_{j-1}, A v_j> = beta conj(<v_j, A v_{j-1}> / beta) = (beta / conj(beta)) ||W_j||.
-// The column of H and the two coefficients of the Gram-Schmidt update.
+// The column of H (written by the block with `write`) and the two coefficients of the
+// Gram-Schmidt update, which thread 0 returns in c.
+__device__ __forceinline__ void lanczos_column(const double *__restrict__ partial, int64_t nblk, int r, int j,
+                                               const cplx<double> *__restrict__ beta, const gm_state &st, double *sh, bool write,
+                                               cplx<double> (&c)[2])
+{
+    double k = 0;
+    for (int64_t b = threadIdx.x; b < nblk; b += VTHREADS) k += partial[(int64_t)r * nblk + b];
+    k = block_sum(k, sh);
+    if (threadIdx.x != 0) return;
+    const double *sc = st.sc + (int64_t)r * (st.m + 1);
+    cplx<double> *H = st.H + ((int64_t)r * st.m + j) * (st.m + 1);
+    const cplx<double> b = beta[r];
+    k *= sc[j] * sc[j];
+    const cplx<double> hj = {1.0 + b.re * k, b.im * k};
+    c[0] = sc[j] * hj;
+    c[1] = {0.0, 0.0};
+    if (write) H[j] = hj;
+    if (j == 0) return;
+    const double b2 = b.re * b.re + b.im * b.im, h = b2 > 0 && sc[j] > 0 ? 1.0 / (sc[j] * b2) : 0.0;
+    const cplx<double> hp = h * (b * b);
+    c[1] = sc[j - 1] * hp;
+    if (!write) return;
+    for (int i = 0; i < j - 1; ++i) H[i] = {0.0, 0.0};
+    H[j - 1] = hp;
+}
+
+// coef[j], coef[j - 1] and the column of H, where k_lanczos_update is not to form them
 static __global__ __launch_bounds__(VTHREADS) void k_gm_lanczos(const double *__restrict__ partial, int64_t nblk, int j,
                                                                 const cplx<double> *__restrict__ beta, gm_state st)
 {
     const int r = blockIdx.x;
     if (!st.cyc[r]) return;
     __shared__ double sh[VTHREADS / 64];
-    double k = 0;
-    for (int64_t b = threadIdx.x; b < nblk; b += VTHREADS) k += partial[(int64_t)r * nblk + b];
-    k = block_sum(k, sh);
+    cplx<double> c[2];
+    lanczos_column(partial, nblk, r, j, beta, st, sh, true, c);
     if (threadIdx.x != 0) return;
-    const double *sc = st.sc + (int64_t)r * (st.m + 1);
-    cplx<double> *H = st.H + ((int64_t)r * st.m + j) * (st.m + 1), *coef = st.coef + (int64_t)r * (st.m + 1);
-    const cplx<double> b = beta[r];
-    k *= sc[j] * sc[j];
-    H[j] = {1.0 + b.re * k, b.im * k};
-    coef[j] = sc[j] * H[j];
-    if (j == 0) return;
-    for (int i = 0; i < j - 1; ++i) H[i] = {0.0, 0.0};
-    const double b2 = b.re * b.re + b.im * b.im, h = b2 > 0 && sc[j] > 0 ? 1.0 / (sc[j] * b2) : 0.0;
-    H[j - 1] = h * (b * b);
-    coef[j - 1] = sc[j - 1] * H[j - 1];
+    cplx<double> *coef = st.coef + (int64_t)r * (st.m + 1);
+    coef[j] = c[0];
+    if (j) coef[j - 1] = c[1];
+}
+
+// W_{j+1} = sc_j (A W_j) - coef_j W_j - coef_{j-1} W_{j-1} (A W_j in w, in place)
+// and partial ||W_{j+1}||^2.  With FOLD every block sums the operator's partials itself
+// and forms the coefficients, one launch of 3.6 us less per step; it does so where
+// there are at most LANCZOS_FOLD of them (each block reads them all).  Without and
+// with it: 10 meson steps at 9x14x15 3.83 and 3.60 ms, 45x22x13 with 24 fields (202
+// partials) 606 and 589 us, 64^3 with 12 fields (tiles) 1.80 and 1.78 ms a step.
+constexpr int64_t LANCZOS_FOLD = 1024;
+template <typename T, bool FOLD>
+__global__ __launch_bounds__(VTHREADS) void k_lanczos_update(gm_basis<T> basis, int j, cplx<T> *__restrict__ w, int64_t n, int nf,
+                                                             gm_state st, double *__restrict__ partial,
+                                                             const double *__restrict__ kpart, int64_t nblk,
+                                                             const cplx<double> *__restrict__ beta)
+{
+    const int r = blockIdx.y;
+    if (!st.cyc[r]) return;
+    __shared__ double sh[8];
+    __shared__ cplx<double> cs[2];
+    cplx<double> c[2];
+    if (FOLD) {
+        lanczos_column(kpart, nblk, r, j, beta, st, sh, blockIdx.x == 0, c);
+        if (threadIdx.x == 0) cs[0] = c[0], cs[1] = c[1];
+        __syncthreads();
+        c[0] = cs[0], c[1] = cs[1];
+    } else {
+        const cplx<double> *coef = st.coef + (int64_t)r * (st.m + 1);
+        c[0] = coef[j];
+        c[1] = j ? coef[j - 1] : cplx<double>{0.0, 0.0};
+    }
+    const double scj = st.sc[(int64_t)r * (st.m + 1) + j];
+    cplx<T> *wr = w + (int64_t)r * n;
+    const cplx<T> *vj = basis.at(j, r, nf, n), *vp = j ? basis.at(j - 1, r, nf, n) : nullptr;
+    double nrm = 0;
+    for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (int64_t)gridDim.x * blockDim.x) {
+        const cplx<T> w0 = wr[k], v = vj[k];
+        cplx<double> a = {scj * (double)w0.re, scj * (double)w0.im};
+        if (vp) {
+            const cplx<T> q = vp[k];
+            a = a - c[1] * cplx<double>{(double)q.re, (double)q.im};
+        }
+        a = a - c[0] * cplx<double>{(double)v.re, (double)v.im};
+        const cplx<T> o = {(T)a.re, (T)a.im};
+        wr[k] = o;
+        nrm += nrm2(o);
+    }
+    nrm = block_sum(nrm, sh);
+    if (threadIdx.x == 0) partial[(int64_t)r * gridDim.x + blockIdx.x] = nrm;
 }
 
 // out[r] = sum_b partial[r * nblk + b] for the slot r = blockIdx.x if
@@ -270,10 +336,10 @@ static __global__ __launch_bounds__(FOLD_THREADS) void k_fold_slots(const double
     }
 }
 
-// Gram-Schmidt update W_nv = sc_j (A W_j) - sum_{lo <= i < nv} coef_i W_i
-// (j = nv - 1, A W_j in w, in place) and partial ||W_nv||^2
+// Gram-Schmidt update W_nv = sc_j (A W_j) - sum_{i < nv} coef_i W_i (j = nv - 1,
+// A W_j in w, in place) and partial ||W_nv||^2
 template <typename T>
-__global__ __launch_bounds__(VTHREADS) void k_cgs_update(gm_basis<T> basis, int lo, int nv, cplx<T> *__restrict__ w, int64_t n, int nf,
+__global__ __launch_bounds__(VTHREADS) void k_cgs_update(gm_basis<T> basis, int nv, cplx<T> *__restrict__ w, int64_t n, int nf,
                                                          gm_state st, double *__restrict__ partial)
 {
     const int r = blockIdx.y;
@@ -286,7 +352,7 @@ __global__ __launch_bounds__(VTHREADS) void k_cgs_update(gm_basis<T> basis, int 
     for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (int64_t)gridDim.x * blockDim.x) {
         const cplx<T> w0 = wr[k];
         cplx<double> a = {scj * (double)w0.re, scj * (double)w0.im};
-        for (int i = lo; i < nv; ++i) {
+        for (int i = 0; i < nv; ++i) {
             const cplx<T> v = basis.at(i, r, nf, n)[k];
             a = a - h[i] * cplx<double>{(double)v.re, (double)v.im};
         }

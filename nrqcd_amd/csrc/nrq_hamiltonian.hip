@@ -492,7 +492,7 @@ static int ham_solve(const ham_operator &op, int nc, const cplx<double> (*a)[4],
             hipLaunchKernelGGL(k_mdot<double>, dim3(nb, nc), dim3(VTHREADS), 0, stream(), W, nv, (const cplx<double> *)w, n, nc,
                                (const int *)gm.cyc, cpart);
             hipLaunchKernelGGL(k_gm_dots, dim3((nv * nc + 3) / 4), dim3(256), 0, stream(), cpart, (int)nb, nv, nc, gm);
-            hipLaunchKernelGGL(k_cgs_update<double>, dim3(nb, nc), dim3(VTHREADS), 0, stream(), W, 0, nv, w, n, nc, gm, rpart);
+            hipLaunchKernelGGL(k_cgs_update<double>, dim3(nb, nc), dim3(VTHREADS), 0, stream(), W, nv, w, n, nc, gm, rpart);
             hipLaunchKernelGGL(k_gm_step, dim3(nc), dim3(VTHREADS), 0, stream(), rpart, (int)nb, k, 0, gm,
                                g_ham.flags + (k & 1) * NSLOTS);
             NRQ_HIP(hipGetLastError());

@@ -1170,8 +1170,8 @@ static cplx<double> g_beta_host[NSLOTS];
 // up to 5,000 times the usual one (77 iterations a column, m = 30 and 8; FP32 corrections
 // with m = 8 there need 976 in place of 982 iterations in all).
 //
-// A step is four launches (operator, its scalars, Gram-Schmidt
-// update, rotation; five with a network) that need nothing from the host: the rotations and the
+// A step is three launches (operator, Gram-Schmidt update, rotation; four on the
+// largest lattices, five with a network) that need nothing from the host: the rotations and the
 // decision whether a slot goes on are made on the device (k_gm_step), which
 // every kernel of the next step looks at.  The host enqueues step j + 2 once it
 // has seen step j end, so the queue does not run empty; the one step enqueued
@@ -1282,12 +1282,18 @@ static int gmres_core(const cplx<RL> *links, int R, const cplx<T> *b, const slot
                 hipLaunchKernelGGL(k_mdot<T>, dim3(nb, R), dim3(VTHREADS), 0, stream(), W, nv, (const cplx<T> *)w, n, R,
                                    (const int *)gm.cyc, g_ws.cpart);
                 hipLaunchKernelGGL(k_gm_dots, dim3((nv * R + 3) / 4), dim3(256), 0, stream(), g_ws.cpart, (int)nb, nv, R, gm);
+                hipLaunchKernelGGL(k_cgs_update<T>, dim3(nb, R), dim3(VTHREADS), 0, stream(), W, nv, w, n, R, gm, g_ws.rpart);
             } else {
                 const int64_t nsb = launch_krylov_op<RL, T>(links, R, vj, ws_slots(w, R), gm.cyc);
-                hipLaunchKernelGGL(k_gm_lanczos, dim3(R), dim3(VTHREADS), 0, stream(), g_ws.spart, nsb, j, g_ws.beta, gm);
+                if (nsb <= LANCZOS_FOLD) {
+                    hipLaunchKernelGGL((k_lanczos_update<T, true>), dim3(nb, R), dim3(VTHREADS), 0, stream(), W, j, w, n, R, gm,
+                                       g_ws.rpart, g_ws.spart, nsb, g_ws.beta);
+                } else {
+                    hipLaunchKernelGGL(k_gm_lanczos, dim3(R), dim3(VTHREADS), 0, stream(), g_ws.spart, nsb, j, g_ws.beta, gm);
+                    hipLaunchKernelGGL((k_lanczos_update<T, false>), dim3(nb, R), dim3(VTHREADS), 0, stream(), W, j, w, n, R, gm,
+                                       g_ws.rpart, g_ws.spart, nsb, g_ws.beta);
+                }
             }
-            hipLaunchKernelGGL(k_cgs_update<T>, dim3(nb, R), dim3(VTHREADS), 0, stream(), W, net ? 0 : std::max(0, nv - 2), nv, w, n,
-                               R, gm, g_ws.rpart);
             hipLaunchKernelGGL(k_gm_step, dim3(R), dim3(VTHREADS), 0, stream(), g_ws.rpart, (int)nb, j, net ? 1 : 0, gm,
                                g_ws.ibuf + (j & 1) * NSLOTS);
             NRQ_HIP(hipGetLastError());

@@ -434,3 +434,25 @@ def test_gmres_recurrence_on_stiff_steps(nrq, oracle, cn, kind, restart, step):
     Qg, Ag = h.download()
     assert np.linalg.norm(Qg - Q) < 1.6e-10 * np.linalg.norm(Q)
     assert np.linalg.norm(Ag - A) < 1.6e-10 * np.linalg.norm(A)
+
+
+@pytest.mark.parametrize("ext", [(64, 32, 32), (64, 32, 33), (37, 45, 41)])
+def test_gmres_at_the_edge_of_the_folded_partials(nrq, cn, ext):
+    """1,024 and more partial sums of 64 sites per field: a single-dof source (two
+    fields: no LDS tiles) by GMRES against Chebyshev.  Both leave 1e-12 ||y||, ||y|| <=
+    1.1 ||psi|| and the inverse has norm <= 1: within 2.2e-12 of the norm."""
+    _say(f"GMRES, two fields on {ext}")
+    cn(ext, SP)
+    nrq.random_init(6)
+    g = nrq.GaugeConfiguration()
+    g.TransversePolarisedOccupiedInit_Box(0.5, 1.0, 1.0)
+    got = []
+    for kind in (nrq.NRQ_SOLVER_GMRES_FP64, nrq.NRQ_SOLVER_CHEBYSHEV_FP64):
+        nrq.nrqcd_set_solver(kind, 30, 10000)
+        h = nrq.NRQCDField()
+        h.InitSinglePointSingleDoF(1, 2, 5, 2, 3, 7)
+        st = h.Update(g, 2.0, C1)
+        assert st.max_true_relres <= 1e-12
+        got.append(h.download())
+    for a, b in zip(*got):
+        assert np.linalg.norm(a - b) < 3e-12 * np.linalg.norm(b)
