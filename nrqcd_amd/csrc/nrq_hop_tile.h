@@ -25,10 +25,11 @@
 //
 // Sites beyond an extent that is not a multiple of the tile are filled with
 // their periodic images, so the neighbours of the last row and column are found
-// like any others; such lanes store nothing.  Any extents work; hop_tiles_for
-// says where it pays.
+// like any others; such lanes store nothing.  Any extents work; hop_tiles_pay
+// says where it is faster.
 #pragma once
 #include "nrq_map.h"
+#include <cmath>
 
 namespace nrq {
 
@@ -38,6 +39,7 @@ constexpr int HT_CELLS = HT_HX * (HT_Y + 2);
 constexpr int HT_HALO = 2 * HT_Y + 2 * HT_X; // halo cells of a plane (no corners)
 constexpr int HT_F = 12;                    // fields (wavefronts) per block
 constexpr int HT_THREADS = 64 * HT_F;
+constexpr int HT_CUS = 256; // one block per CU: LDS and the registers of its 12 wavefronts
 // links of a plane that the tile needs: U_x from x - 1, U_y from y - 1, U_z
 constexpr int HT_LX = (HT_X + 1) * HT_Y, HT_LY = HT_X * (HT_Y + 1), HT_LZ = HT_X * HT_Y;
 constexpr int HT_L = HT_LX + HT_LY + HT_LZ;
@@ -370,38 +372,53 @@ __global__ __launch_bounds__(HT_THREADS) void k_hop_tile(const cplx<RL> *__restr
     }
 }
 
-// The tiling of lattice g for nf slots.  groups = 0 where the wave items of
-// nrq_map.h are faster, by the times of a CN step of both (us, wave items /
-// tiles, mixed Chebyshev with 12 slots unless said):
-//  - a group with idle wavefronts costs as much as a full one: tiles for at
-//    least 4/5 full groups (64^3 with 2 slots: 311 / 401);
-//  - rows that do not start on a cache line and lanes past a row's end cost
-//    tiles a quarter to a half more: n0 a multiple of 16 (64^3: 1010 / 769,
-//    48^3: 486 / 396, 33 x 64 x 64: 618 / 800, 100^3: 4139 / 4501), unless n1 is
-//    such that wave items find only bands of one or two rows (17 x 17 x 64:
-//    296 / 198, 18 x 70 x 70: 569 / 436, 45 x 37 x 54: 517 / 486);
-//  - small lattices leave CUs idle: 16^3 152 / 178, 28^3 192 / 206,
-//    32^3 200 / 202, with 48 slots 690 / 516.
+// The tiling of lattice g for nf slots.
 inline hop_tiles hop_tiles_for(const geom &g, int nf)
 {
     hop_tiles t{};
     t.ntx = (g.n0 + HT_X - 1) / HT_X;
     t.nty = (g.n1 + HT_Y - 1) / HT_Y;
-    const int groups = (nf + HT_F - 1) / HT_F;
+    t.groups = (nf + HT_F - 1) / HT_F;
     const int64_t tiles = (int64_t)t.ntx * t.nty;
     // at least two blocks per CU, runs of at least four planes
-    int nzr = (int)((512 + tiles * groups - 1) / (tiles * groups));
+    int nzr = (int)((2 * HT_CUS + tiles * t.groups - 1) / (tiles * t.groups));
     nzr = nzr < g.n2 / 4 ? nzr : g.n2 / 4;
     if (nzr < 1) nzr = 1;
     t.zc = (g.n2 + nzr - 1) / nzr;
     t.nzr = (g.n2 + t.zc - 1) / t.zc;
-    const int64_t work = g.vol * nf;
-    const bool full = 5 * nf >= 4 * HT_F * groups;
-    const bool narrow = g.n1 % 4 != 0; // wave-item bands of one or two rows
-    if (full && ((g.n0 % HT_X == 0 && work >= 390000) || (narrow && work >= 200000))) t.groups = groups;
     return t;
 }
 
 inline unsigned hop_grid(const hop_tiles &t) { return (unsigned)t.ntx * (unsigned)t.nty * (unsigned)t.nzr * (unsigned)t.groups; }
+
+// What a kernel computes: the wave items that cost as much as one z plane of a
+// tile on every CU, from the fit below.
+enum hop_op { HOP_FP32 = 667, HOP_FP64 = 1250, HOP_FP64_CHEB = 1350 };
+
+// Whether the tiles of lattice g are faster than the wave items of nrq_map.h for nf slots.
+// The time of the tiles goes with the planes of a run times the rounds of blocks, one block per CU (half way
+// between whole rounds and their exact number fits best); that of the wave items with their
+// number, whatever part of their lanes is used, so that bands that fill 64 lanes badly favour
+// the tiles and tiles that reach past the lattice the wave items.  Above two groups (more than 24
+// slots) FP64 wave items gain on the tiles, as their chunks share more link lines.
+// Fitted to each operator taken alone both ways in CN steps of four solvers on 230 lattices of 10 to 112
+// a side, 12, 24 and 48 slots, both storages: against wave items everywhere steps are 1.11 times as
+// fast in the mean and no less than 0.95 times.  us per step, wave items / tiles, 12 slots:
+// FP64 Chebyshev 64^3 1497 / 1142, 90x62x58 2112 / 2099, 33x30x27 401 / 335, 32^3 238 / 271, 48x25x17
+// 212 / 308; mixed Chebyshev 64^3 1001 / 759, 48^3 462 / 383, 8x81x27 437 / 210, 32^3 185 / 190,
+// 90x62x58 1379 / 1459; GMRES 64^3 2071 / 1689, 40^3 613 / 646, 30x34x22 397 / 393; with 48 slots
+// mixed Chebyshev 48^3 2212 / 1731, FP64 Chebyshev 28^3 596 / 633.
+// A group with idle wavefronts costs as much as a full one: tiles for at least 4/5 full
+// groups (64^3 with 2 slots, mixed Chebyshev: 311 / 401).
+inline bool hop_tiles_pay(const geom &g, const hop_tiles &t, int nf, hop_op op)
+{
+    if (5 * nf < 4 * HT_F * t.groups) return false;
+    const int nc = op == HOP_FP32 ? 4 : 2; // fields per thread of the default wave items
+    const lf_map mp = make_lf_map(g, 64, 8, 4, 1);
+    double items = (double)mp.nsb * ((nf + nc - 1) / nc);
+    if (op != HOP_FP32 && t.groups > 2) items *= 0.85;
+    const double blocks = (double)hop_grid(t) / HT_CUS;
+    return items > 0.5 * (std::ceil(blocks) + blocks) * (t.zc - 0.5) * (double)op;
+}
 
 } // namespace nrq

@@ -945,13 +945,14 @@ static lf_map cn_map(int nf, int nc)
 }
 
 // Whether a launch of nf slots goes through the LDS tiles: where they pay
-// (hop_tiles_for) and no other shape than the default was chosen.
-static bool use_tiles(int nf, hop_tiles *t)
+// (hop_tiles_pay) and no other shape than the default was chosen.
+static bool use_tiles(int nf, hop_op op, hop_tiles *t)
 {
     if (shape().mode != 4 || shape().xcd != 8) return false;
     *t = hop_tiles_for(lat().g, nf);
-    return t->groups > 0;
+    return hop_tiles_pay(lat().g, *t, nf, op);
 }
+template <typename T> constexpr hop_op op_of() { return sizeof(T) == 8 ? HOP_FP64 : HOP_FP32; }
 static dim3 tile_grid(const hop_tiles &t) { return dim3(hop_grid(t)); }
 
 // Runs the statements after `nc` with the compile-time chunk width NCV equal
@@ -1011,7 +1012,7 @@ static void launch_stencil(const cplx<RL> *u, const slots<T> &in, const slots<T>
                            const int *active, const cplx<double> *gco = nullptr)
 {
     hop_tiles tl;
-    if (use_tiles(nf, &tl)) {
+    if (use_tiles(nf, op_of<T>(), &tl)) {
         const tile_stencil<T> op = {in, out, g_ws.beta, gco, active};
         hipLaunchKernelGGL((k_hop_tile<RL, T, tile_stencil<T>>), tile_grid(tl), dim3(HT_THREADS), 0, stream(), u, op, nf,
                            lat().g, tl);
@@ -1029,7 +1030,7 @@ template <typename RL, typename T>
 static int64_t launch_krylov_op(const cplx<RL> *u, int R, const slots<T> &v, const slots<T> &w, const int *active)
 {
     hop_tiles tl;
-    if (use_tiles(R, &tl)) {
+    if (use_tiles(R, op_of<T>(), &tl)) {
         const int64_t nsb = (int64_t)tl.ntx * tl.nty * tl.nzr;
         const tile_krylov_op<T> op = {v, w, g_ws.beta, active, g_ws.spart, nsb};
         hipLaunchKernelGGL((k_hop_tile<RL, T, tile_krylov_op<T>>), tile_grid(tl), dim3(HT_THREADS), 0, stream(), u, op, R,
@@ -1049,16 +1050,17 @@ static void launch_cheb(const cplx<RL> *links, const slots<T> &xk, const slots<T
                         const cplx<double> *cf, int R, int mode, int fin, const slots<double> &fi, const slots<double> &fo)
 {
     hop_tiles tl;
-    if (use_tiles(R, &tl)) {
-        if (fin) {
-            const tile_cheb<T, true> op = {xk, xnext, xnext, b, fi, fo, g_ws.beta, cf, g_ws.active, mode};
-            hipLaunchKernelGGL((k_hop_tile<RL, T, tile_cheb<T, true>>), tile_grid(tl), dim3(HT_THREADS), 0, stream(), links,
-                               op, R, lat().g, tl);
-        } else {
-            const tile_cheb<T, false> op = {xk, xnext, xnext, b, fi, fo, g_ws.beta, cf, g_ws.active, mode};
-            hipLaunchKernelGGL((k_hop_tile<RL, T, tile_cheb<T, false>>), tile_grid(tl), dim3(HT_THREADS), 0, stream(), links,
-                               op, R, lat().g, tl);
-        }
+    if (use_tiles(R, sizeof(T) == 8 ? HOP_FP64_CHEB : HOP_FP32, &tl)) {
+        if constexpr (sizeof(T) == 4) // the FP64 iterate is a correction's
+            if (fin) {
+                const tile_cheb<T, true> op = {xk, xnext, xnext, b, fi, fo, g_ws.beta, cf, g_ws.active, mode};
+                hipLaunchKernelGGL((k_hop_tile<RL, T, tile_cheb<T, true>>), tile_grid(tl), dim3(HT_THREADS), 0, stream(),
+                                   links, op, R, lat().g, tl);
+                return;
+            }
+        const tile_cheb<T, false> op = {xk, xnext, xnext, b, fi, fo, g_ws.beta, cf, g_ws.active, mode};
+        hipLaunchKernelGGL((k_hop_tile<RL, T, tile_cheb<T, false>>), tile_grid(tl), dim3(HT_THREADS), 0, stream(), links, op, R,
+                           lat().g, tl);
         return;
     }
     const int nc = nc_of<T>();
@@ -1075,7 +1077,7 @@ static int64_t launch_resid(const cplx<RL> *u, int R, const slots<T> &x, const s
                             const int *active)
 {
     hop_tiles tl;
-    if (use_tiles(R, &tl)) {
+    if (use_tiles(R, op_of<T>(), &tl)) {
         const int64_t nsb = (int64_t)tl.ntx * tl.nty * tl.nzr;
         const tile_resid<T, TR, WRITE> op = {x, y, res, g_ws.beta, active, g_ws.spart, nsb};
         hipLaunchKernelGGL((k_hop_tile<RL, T, tile_resid<T, TR, WRITE>>), tile_grid(tl), dim3(HT_THREADS), 0, stream(), u, op,
@@ -1096,7 +1098,7 @@ static int64_t launch_rhs(const cplx<RL> *u, int R, const slots<double> &psi, co
                           const slots<double> &x, int guess, const slots<float> &kout, int wk)
 {
     hop_tiles tl;
-    if (use_tiles(R, &tl)) {
+    if (use_tiles(R, HOP_FP64, &tl)) {
         const int64_t nsb = (int64_t)tl.ntx * tl.nty * tl.nzr;
         const tile_rhs op = {psi, y, x, kout, g_ws.cpar, g_ws.cpar + NSLOTS, g_ws.spart, nsb, guess, wk};
         hipLaunchKernelGGL((k_hop_tile<RL, double, tile_rhs>), tile_grid(tl), dim3(HT_THREADS), 0, stream(), u, op, R,

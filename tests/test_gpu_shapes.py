@@ -218,6 +218,54 @@ def test_lds_tiles_match_wave_items(nrq, lattice, ext, prec):
         nrq.nrqcd_finalize()
 
 
+@pytest.mark.parametrize("ext,prec", [
+    ((8, 81, 27), 64),   # a tile twice as wide as the lattice
+    ((13, 37, 45), 32),
+    ((17, 3, 397), 64),  # fewer rows than a tile has
+    ((20, 4, 601), 32),  # one row of tiles, runs of different lengths
+    ((48, 6, 198), 64),  # half tiles along y
+])
+def test_lds_tiles_on_narrow_lattices_match_wave_items(nrq, lattice, ext, prec):
+    """The same on lattices whose extents are small beside a tile, or whose wave items
+    leave most lanes idle."""
+    test_lds_tiles_match_wave_items(nrq, lattice, ext, prec)
+
+
+@pytest.mark.parametrize("ext,kind", [((48, 25, 17), "CHEBYSHEV_FP64"), ((80, 18, 18), "CHEBYSHEV_FP64"),
+                                      ((48, 25, 17), "CHEBYSHEV_MIXED")])
+def test_default_cn_shape_is_not_slower_than_wave_items(nrq, lattice, ext, kind):
+    """Lattices too small to fill the LDS tiles' blocks: the default shape takes no longer
+    than wave items (the same map without its XCD order), 15 % allowed for noise and
+    that order; through tiles such steps took 1.25 to 1.45 times as long."""
+    lattice(ext, (0.05, 1.0, 0.9, 1.1))
+    _say(f"default CN shape on {ext}, {kind}")
+    g = nrq.GaugeConfiguration()
+    g.upload(None, 0.1 * np.random.default_rng(5).normal(size=(8, 3, ext[0] * ext[1] * ext[2])))
+    g.Update(1.0, 10)
+    default = nrq.cn_get_shape()
+    nrq.nrqcd_init(2.0, C1, 1.0, 1e-10)
+    nrq.nrqcd_set_solver(getattr(nrq, "NRQ_SOLVER_" + kind), 30, 10000)
+    best = {}
+    try:
+        h = nrq.NRQCDField()
+        h.InitSinglePoint(1, 1)
+        for rep in range(12):
+            for shape in (default, (2, 4, 4, 1)):
+                nrq.cn_set_shape(*shape)
+                h.Update(g, 2.0, C1)
+                nrq.event_record(0)
+                for _ in range(5):
+                    h.Update(g, 2.0, C1)
+                nrq.event_record(1)
+                nrq.synchronize()
+                t = nrq.event_elapsed_ms(0, 1)
+                best[shape] = min(best.get(shape, t), t)
+    finally:
+        nrq.cn_set_shape(*default)
+        nrq.nrqcd_finalize()
+    assert best[default] < 1.15 * best[(2, 4, 4, 1)], best
+
+
 def test_batch_graph_follows_a_change_of_spacings(nrq, lattice, monkeypatch):
     """The hipGraph of a batched leapfrog carries the lattice by value.  After
     the lattice module is re-initialised with the same extents and other
