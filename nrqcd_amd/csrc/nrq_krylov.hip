@@ -1573,14 +1573,16 @@ static int cheb_solve(const cplx<RL> *u, int R, const std::vector<zc> &alpha, co
             bnd[r] *= cheb_bound(sig[r], k) + FP32_CORR_ERR;
         }
     }
-    if (int e = wait_sums()) return e;
-    bn_from_host();
     if (!*in_psi) {
-        // no correction was needed: the guess goes to the heavy field
+        // the bound asks for no correction: the guess goes to the heavy field, and its
+        // residual is measured like any other's
         hipLaunchKernelGGL(k_copy_slots, dim3(vblocks(3 * g_ws.vol), R), dim3(VTHREADS), 0, stream(), tx, tpsi, 3 * g_ws.vol);
         NRQ_HIP(hipGetLastError());
         *in_psi = true;
+        if (int e = cn_resid<RL>(u, R, tpsi, g_ws.y32)) return e;
     }
+    if (int e = wait_sums()) return e;
+    bn_from_host();
     // measured corrections (in place) until converged
     for (int round = 0; round < 8; ++round) {
         if (!check_slots(R, bn, p.tol, act, rel, need)) break;

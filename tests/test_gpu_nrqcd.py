@@ -456,3 +456,30 @@ def test_gmres_at_the_edge_of_the_folded_partials(nrq, cn, ext):
         got.append(h.download())
     for a, b in zip(*got):
         assert np.linalg.norm(a - b) < 3e-12 * np.linalg.norm(b)
+
+
+def test_mixed_chebyshev_measures_a_guess_that_needs_no_correction(nrq, cn):
+    """A step so short that the first-order guess is exact to rounding: no correction is
+    planned, and convergence is judged on this step's residual, not on what an
+    earlier solve left (here GMRES stopped after one iteration)."""
+    ext = (6, 5, 4)
+    _say("mixed Chebyshev without a correction")
+    cn(ext, SP)
+    rng = np.random.default_rng(2)
+    v = 6 * 5 * 4
+    g = nrq.GaugeConfiguration()
+    g.upload(None, 0.3 * rng.normal(size=(8, 3, v)))
+    g.Update(1.0, 10)
+    Q, A = (rng.normal(size=(6, 6, v)) + 1j * rng.normal(size=(6, 6, v)) for _ in range(2))
+    h = nrq.NRQCDField()
+    h.upload(Q, A)
+    nrq.nrqcd_set_solver(nrq.NRQ_SOLVER_GMRES_FP64, 30, 1)
+    with pytest.raises(nrq.NRQError):
+        h.Update(g, 2.0, C1, 100.0)
+    nrq.nrqcd_set_solver(nrq.NRQ_SOLVER_CHEBYSHEV_MIXED, 30, 10000)
+    h.upload(Q, A)
+    st = h.Update(g, 2.0, C1, 1e-9)
+    assert st.iterations == 0 and 0 < st.max_true_relres <= 1e-15
+    Qg, _ = h.download()
+    # K has norm <= 6, so the step changes Q by at most 2 * 6 * 1e-9 * 0.05 / 4 of its norm
+    assert 0 < np.linalg.norm(Qg - Q) < 2e-10 * np.linalg.norm(Q)
