@@ -367,8 +367,9 @@ __global__ __launch_bounds__(VTHREADS) void k_cgs_update(gm_basis<T> basis, int 
 // End of Arnoldi step j of slot r = blockIdx.x: ||W_{j+1}|| from its partials,
 // the Givens rotation of column j and the residual estimate; the slot's cycle
 // ends at `stop`, at its iteration cap, or (net) when a coefficient is not
-// finite, which leaves the columns before j.  Whether it goes on is also
-// written to *host_cyc (pinned).
+// finite, which leaves the columns before j (without net such a column ends the
+// cycle too and stays in it: x, and the residual that the host then sees, are not
+// finite either).  Whether it goes on is also written to *host_cyc (pinned).
 static __global__ __launch_bounds__(VTHREADS) void k_gm_step(const double *__restrict__ partial, int nblk, int j, int net, gm_state st,
                                                       int *__restrict__ host_cyc)
 {
@@ -395,7 +396,7 @@ static __global__ __launch_bounds__(VTHREADS) void k_gm_step(const double *__res
             return;
         }
     }
-    const double hn = sqrt(fmax(v, 0.0));
+    const double hn = v < 0 ? 0.0 : sqrt(v); // what is not a number stays so
     st.sc[(int64_t)r * (m + 1) + j + 1] = hn > 0 ? 1.0 / hn : 0.0;
     cplx<double> a = H[0];
     for (int i = 0; i < j; ++i) {
@@ -418,7 +419,8 @@ static __global__ __launch_bounds__(VTHREADS) void k_gm_step(const double *__res
     g[j + 1] = {-gn.re, -gn.im};
     g[j] = c * gj;
     st.used[r] = j + 1;
-    const bool end = sqrt(gn.re * gn.re + gn.im * gn.im) <= st.stop[r] || j + 1 >= st.left[r];
+    // not finite: the cycle ends here, and the true residual tells the host
+    const bool end = sqrt(gn.re * gn.re + gn.im * gn.im) <= st.stop[r] || j + 1 >= st.left[r] || !isfinite(hn);
     if (end) st.cyc[r] = 0;
     host_cyc[r] = end ? 0 : 1;
 }

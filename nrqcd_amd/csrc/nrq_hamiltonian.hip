@@ -516,9 +516,10 @@ static int ham_solve(const ham_operator &op, int nc, const cplx<double> (*a)[4],
             its[c] += used[c];
             st->iterations += used[c];
             const bool conv = rnorm[c] <= tol * bnorm[c];
-            if (!conv && its[c] < maxit) continue;
+            // a residual that is not finite stays so
+            if (!conv && its[c] < maxit && std::isfinite(rnorm[c])) continue;
             act &= ~(1ull << c);
-            st->max_true_relres = std::max(st->max_true_relres, rnorm[c] / bnorm[c]);
+            st->max_true_relres = worse(st->max_true_relres, rnorm[c] / bnorm[c]);
             if (!conv && failed < 0) failed = c;
         }
     }

@@ -24,6 +24,9 @@ enum krylov_kind {
     KRYLOV_FGMRES_CNN_MIXED = 5, // FP32 FGMRES(m) with the network inside FP64 iterative refinement
 };
 
+// The larger of two relative residuals; one that is not a number is larger than any other.
+inline double worse(double a, double b) { return a >= b || a != a ? a : b; }
+
 struct krylov_params {
     int kind = KRYLOV_GMRES_FP64;
     int restart = 30;          // GMRES restart length m (PETSc default 30)

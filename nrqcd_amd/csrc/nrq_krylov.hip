@@ -1150,6 +1150,12 @@ int krylov_rhs_features(const nrq_gauge *gf, int R, const cplx<double> **f1, con
     return NRQ_OK;
 }
 
+// ||r|| / ||y||; 0 for a zero right-hand side (x = 0 solves it), and not a number
+// where one of the two is not finite, so that `rel <= tol` fails
+static double rel_of(double rn, double bn) { return bn == 0.0 ? 0.0 : rn / bn; }
+// a norm from its square, which rounding may have left below zero
+static double norm_of(double v) { return v < 0 ? 0.0 : std::sqrt(v); }
+
 // column solves handed from FGMRES to plain GMRES since the library loaded
 static int64_t g_fallbacks = 0;
 // CN coefficients beta of the slots of the current step, on the host (the
@@ -1213,11 +1219,11 @@ static int gmres_core(const cplx<RL> *links, int R, const cplx<T> *b, const slot
         if (int e = upload_active(act)) return e;
         if (int e = residual(true, g_ws.active)) return e;
         if (int e = wait_sums()) return e;
-        for (int r = 0; r < R; ++r) rn[r] = act[r] ? std::sqrt(std::max(g_ws.nbuf[r], 0.0)) : 0.0;
+        for (int r = 0; r < R; ++r) rn[r] = act[r] ? norm_of(g_ws.nbuf[r]) : 0.0;
     }
     for (int r = 0; r < R; ++r) {
         if (!act[r]) continue;
-        rel_out[r] = bnorm[r] > 0 ? rn[r] / bnorm[r] : 0.0;
+        rel_out[r] = rel_of(rn[r], bnorm[r]);
         if (rn[r] <= tol * bnorm[r]) act[r] = 0;
     }
     std::vector<int> ncycles(R, 0);
@@ -1315,9 +1321,10 @@ static int gmres_core(const cplx<RL> *links, int R, const cplx<T> *b, const slot
             its[r] += g_ws.ibuf[workspace::I_USED + r];
             const bool fell = net && g_ws.ibuf[workspace::I_FALLEN + r];
             if (fell) (*fallen)[r] = 1;
-            rn[r] = std::sqrt(std::max(g_ws.nbuf[r], 0.0));
-            rel_out[r] = bnorm[r] > 0 ? rn[r] / bnorm[r] : 0.0;
-            if (rn[r] <= tol * bnorm[r] || its[r] >= maxit) {
+            rn[r] = norm_of(g_ws.nbuf[r]);
+            rel_out[r] = rel_of(rn[r], bnorm[r]);
+            // a residual that is not finite stays so (with a network plain GMRES takes over)
+            if (rn[r] <= tol * bnorm[r] || its[r] >= maxit || (!net && !std::isfinite(rn[r]))) {
                 act[r] = 0;
                 continue;
             }
@@ -1466,9 +1473,9 @@ static bool check_slots(int R, const std::vector<double> &bn, double tol, std::v
     bool any = false;
     for (int r = 0; r < R; ++r) {
         if (!act[r]) continue;
-        const double rr = std::sqrt(std::max(g_ws.nbuf[r], 0.0));
-        rel[r] = bn[r] > 0 ? rr / bn[r] : 0.0;
-        if (rr <= tol * bn[r]) {
+        const double rr = norm_of(g_ws.nbuf[r]);
+        rel[r] = rel_of(rr, bn[r]);
+        if (rr <= tol * bn[r] || !std::isfinite(rr)) { // not finite: no step mends that
             act[r] = 0;
             continue;
         }
@@ -1502,7 +1509,7 @@ static int cheb_solve(const cplx<RL> *u, int R, const std::vector<zc> &alpha, co
         return k;
     };
     auto bn_from_host = [&]() {
-        for (int r = 0; r < R; ++r) bn[r] = std::sqrt(std::max(g_ws.nbuf[workspace::NRM_Y + r], 0.0));
+        for (int r = 0; r < R; ++r) bn[r] = norm_of(g_ws.nbuf[workspace::NRM_Y + r]);
     };
     *in_psi = false;
     if (p.kind == KRYLOV_CHEB_FP64) {
@@ -1623,9 +1630,9 @@ static int gmres_mixed(const cplx<RL> *u, int R, std::vector<double> &bn, const 
         bool any = false;
         for (int r = 0; r < R; ++r) {
             if (!act[r]) continue;
-            const double rr = std::sqrt(std::max(g_ws.nbuf[r], 0.0));
-            rel[r] = bn[r] > 0 ? rr / bn[r] : 0.0;
-            if (rr <= p.tol * bn[r] || its[r] >= p.maxit) act[r] = 0;
+            const double rr = norm_of(g_ws.nbuf[r]);
+            rel[r] = rel_of(rr, bn[r]);
+            if (rr <= p.tol * bn[r] || its[r] >= p.maxit || !std::isfinite(rr)) act[r] = 0;
             any = any || act[r];
         }
         if (!any) break;
@@ -1705,7 +1712,7 @@ static int cn_step_t(const cplx<RL> *u, int R, const std::vector<zc> &alpha, con
         }
     } else {
         if (int e = wait_sums()) return e;
-        for (int r = 0; r < R; ++r) bn[r] = std::sqrt(std::max(g_ws.nbuf[workspace::NRM_Y + r], 0.0));
+        for (int r = 0; r < R; ++r) bn[r] = norm_of(g_ws.nbuf[workspace::NRM_Y + r]);
         if (p.kind == KRYLOV_GMRES_FP64) {
             // from a zero guess, straight into the heavy field
             status = gmres_core<double, RL>(u, R, g_ws.y, tpsi, (cplx<double> *)g_ws.basis, g_ws.t, g_ws.res, true,
@@ -1747,15 +1754,15 @@ static int cn_step_t(const cplx<RL> *u, int R, const std::vector<zc> &alpha, con
     double worst = 0;
     int64_t total = 0;
     for (int r = 0; r < R; ++r) {
-        worst = std::max(worst, rel[r]);
+        worst = worse(worst, rel[r]);
         total += its[r];
     }
     if (st) {
         st->iterations += total;
         st->restarts += cycles;
-        st->max_true_relres = std::max(st->max_true_relres, worst);
+        st->max_true_relres = worse(st->max_true_relres, worst);
     }
-    if (worst > p.tol)
+    if (!(worst <= p.tol))
         return fail(NRQ_ERR_NOCONV, "CN: Krylov solver stopped (maxit=%lld) with true relative residual %.3e > %.1e",
                     (long long)p.maxit, worst, p.tol);
     return NRQ_OK;

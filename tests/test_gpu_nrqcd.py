@@ -483,3 +483,60 @@ def test_mixed_chebyshev_measures_a_guess_that_needs_no_correction(nrq, cn):
     Qg, _ = h.download()
     # K has norm <= 6, so the step changes Q by at most 2 * 6 * 1e-9 * 0.05 / 4 of its norm
     assert 0 < np.linalg.norm(Qg - Q) < 2e-10 * np.linalg.norm(Q)
+
+
+@pytest.mark.parametrize("kind", ["GMRES_FP64", "GMRES_MIXED", "CHEBYSHEV_FP64", "CHEBYSHEV_MIXED", None])
+def test_a_step_that_is_not_a_number_is_an_error(nrq, cn, kind):
+    """One link that is not a number: no solver (None: the full Hamiltonian's) reports a
+    propagator that is not a number as converged, and the field does not look like a
+    result.  The next step, on sound links, is not affected."""
+    ext = (6, 5, 4)
+    _say(f"CN step with a NaN link, {kind}")
+    cn(ext, SP)
+    v = 6 * 5 * 4
+    g = nrq.GaugeConfiguration()
+    g.upload(None, 0.3 * np.random.default_rng(2).normal(size=(8, 3, v)))
+    g.Update(1.0, 10)
+    bad = g.copy()
+    U, E = g.download()
+    U = U.copy(order="F")
+    U[1, 1, 2, 17] = np.nan
+    bad.upload(U, E)
+    c = C1 if kind else [1.0, 1.0, 1.0, 1.0]
+    if kind:
+        nrq.nrqcd_set_solver(getattr(nrq, "NRQ_SOLVER_" + kind), 30, 10000)
+    h = nrq.NRQCDField()
+    h.InitSinglePoint(1, 1)
+    with pytest.raises(nrq.NRQError):
+        h.Update(bad, 2.0, c)
+    assert not np.all(np.isfinite(h.download()[0]))
+    h.InitSinglePoint(1, 1)
+    assert h.Update(g, 2.0, c).max_true_relres <= 1e-12
+
+
+@pytest.mark.parametrize("kind", ["GMRES_FP64", "GMRES_MIXED", "CHEBYSHEV_FP64", "CHEBYSHEV_MIXED"])
+def test_a_field_that_is_not_a_number_leaves_the_others_of_a_batch(nrq, cn, kind):
+    """A batch of two fields, one of them not a number at one site: an error, and the
+    other field is stepped as it is alone (both solve to 1e-12, so 1e-10 as above)."""
+    ext = (6, 5, 4)
+    _say(f"CN batch with a NaN field, {kind}")
+    cn(ext, SP)
+    nrq.nrqcd_set_solver(getattr(nrq, "NRQ_SOLVER_" + kind), 30, 10000)
+    rng = np.random.default_rng(2)
+    v = 6 * 5 * 4
+    g = nrq.GaugeConfiguration()
+    g.upload(None, 0.3 * rng.normal(size=(8, 3, v)))
+    g.Update(1.0, 10)
+    Q, A = (rng.normal(size=(6, 6, v)) + 1j * rng.normal(size=(6, 6, v)) for _ in range(2))
+    alone, sound, broken = (nrq.NRQCDField() for _ in range(3))
+    alone.upload(Q, A)
+    alone.Update(g, 2.0, C1)
+    sound.upload(Q, A)
+    Q2 = Q.copy()
+    Q2[:, :, 7] = np.nan
+    broken.upload(Q2, A)
+    with pytest.raises(nrq.NRQError):
+        nrq.update_batch([broken, sound], g, [2.0, 2.0], C1, 1.0)
+    for a, b in zip(alone.download(), sound.download()):
+        assert np.max(np.abs(a - b)) < 1e-10 * np.max(np.abs(a))
+    assert not np.all(np.isfinite(broken.download()[0]))
