@@ -138,8 +138,8 @@ int nrq_gauge_transverse_init(nrq_gauge *h, const double *occupation, int specif
  * leapfrog steps.  charge_density: NULL or 3 x V (colour fastest, the
  * reference's ChargeDensity(colour, index)).  Optional per-iteration outputs
  * (nefieldinit entries, NULL to skip): energy and Gauss deviation after the
- * leapfrog steps, projection sweeps.  The projection is capped at 10^6 sweeps
- * (NRQ_ERR_NOCONV); the reference has no cap. */
+ * leapfrog steps, projection sweeps.  The projection fails after 10^6 sweeps
+ * (the reference has no cap) or on a deviation that is not finite: NRQ_ERR_NOCONV. */
 int nrq_gauge_equilibrium_init(nrq_gauge *h, double beta, int64_t nefieldinit, int64_t nequilibrium, double tolerance,
                                const double *charge_density, double *energies, double *deviations,
                                int64_t *projections);

@@ -231,8 +231,9 @@ __global__ __launch_bounds__(6 * EQ_SITES) void k_eq_sweep(const cplx<R> *__rest
         }
         double tr[8];
         two_re_trace_gen(eq_herm(q), tr);
+        // what is not a number must not pass for a small deviation (a maximum drops it)
 #pragma unroll
-        for (int a = 0; a < 8; ++a) dev = fmax(dev, fabs(tr[a]));
+        for (int a = 0; a < 8; ++a) dev = fabs(tr[a]) < INFINITY ? fmax(dev, fabs(tr[a])) : INFINITY;
     }
     dev = lane_max(dev);
     if (lane == 0) row_raise(row_new, dev);
@@ -330,6 +331,8 @@ static int equilibrium_t(nrq_gauge *h, double beta, int64_t nefieldinit, int64_t
         NRQ_HIP(hipMemcpyAsync(h->e, ehost.data(), ebytes, hipMemcpyHostToDevice, stream()));
         double dev = 0;
         if (int r = start(&dev)) return r;
+        auto not_finite = [&]() { return fail(NRQ_ERR_NOCONV, "EquilibriumInit: the Gauss-law deviation is not finite"); };
+        if (!std::isfinite(dev)) return not_finite();
         const cplx<R> *u = (const cplx<R> *)gauge_links(h); // fixed during the projection
         // batch k: sweeps k EQ_BATCH .. and the deviations after them (rows
         // + 1 ..) to the pinned half k & 1; sweep j reads E and G buffer j & 1
@@ -367,6 +370,7 @@ static int equilibrium_t(nrq_gauge *h, double beta, int64_t nefieldinit, int64_t
                 ++nproj;
                 dev = d[q];
                 done = dev <= tol;
+                if (!std::isfinite(dev)) return not_finite();
             }
             if (!done && !last && k == 0)
                 if (int r = issue()) return r;

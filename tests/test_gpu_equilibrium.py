@@ -67,3 +67,21 @@ def test_equilibrium_init_without_a_sweep(nrq, lattice):
     _, dev, nproj = g.EquilibriumInit(16.0, 1, 0, 1e6)
     assert nproj[0] == 0 and 0 < dev[0] < 1e6
     assert np.isclose(dev[0], g.GetGaussMax(), rtol=1e-12)
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_equilibrium_init_refuses_charges_that_are_not_numbers(nrq, lattice, bad):
+    """A charge density with one entry that is not finite has no Gauss law to project
+    on: an error, where the deviation's maximum once dropped the NaN and the call returned
+    a field without a number in it.  The next call is not affected."""
+    ext = (4, 3, 6)
+    _say(f"EquilibriumInit with a charge of {bad}")
+    lattice(ext, (0.05, 1.0, 1.0, 1.0))
+    rho = np.zeros((3, 72))
+    rho[0, 40] = bad
+    nrq.random_init(5)
+    g = nrq.GaugeConfiguration()
+    with pytest.raises(nrq.NRQError):
+        g.EquilibriumInit(16.0, 1, 2, 1e-2, rho)
+    _, dev, nproj = g.EquilibriumInit(16.0, 1, 2, 1e-2)
+    assert nproj[0] > 0 and np.all(np.isfinite(dev)) and np.all(np.isfinite(g.download()[1]))
