@@ -389,6 +389,8 @@ static int equilibrium_t(nrq_gauge *h, double beta, int64_t nefieldinit, int64_t
         }
         if (projections) projections[it] = nproj;
     }
+    // host values go back with an idle stream (the sweeps and steps of the last round may still run)
+    NRQ_HIP(hipStreamSynchronize(stream()));
     return NRQ_OK;
 }
 

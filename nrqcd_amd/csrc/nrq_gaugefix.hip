@@ -441,7 +441,8 @@ static int gaugefix_t(nrq_gauge *h, double tol, double alpha, int64_t maxit, int
     if (int e = measure(0)) return e;
     int64_t enqueued = 0;
     double dev = 0;
-    for (int64_t done = 0;; ++done) {
+    int64_t done = 0;
+    for (;; ++done) {
         while (enqueued < maxit && enqueued <= done) {
             const int64_t n = enqueued;
             hipfftResult fr = hipfftExecZ2Z(plan, (hipfftDoubleComplex *)fld, (hipfftDoubleComplex *)fld, HIPFFT_FORWARD);
@@ -456,12 +457,12 @@ static int gaugefix_t(nrq_gauge *h, double tol, double alpha, int64_t maxit, int
         }
         NRQ_HIP(hipEventSynchronize(b.ev[done & 1]));
         dev = *(volatile double *)(hmax + (done & 1));
-        if (!std::isfinite(dev)) return fail(NRQ_ERR_NOCONV, "gauge fixing: non-finite divergence");
-        if (dev <= tol || done >= maxit) {
-            if (iterations) *iterations = done;
-            break;
-        }
+        if (!std::isfinite(dev) || dev <= tol || done >= maxit) break;
     }
+    // host values go back with an idle stream: the pair that ran too many ends here
+    NRQ_HIP(hipStreamSynchronize(stream()));
+    if (!std::isfinite(dev)) return fail(NRQ_ERR_NOCONV, "gauge fixing: non-finite divergence");
+    if (iterations) *iterations = done;
     if (final_dev) *final_dev = dev;
     return NRQ_OK;
 }

@@ -5,6 +5,8 @@ Bars: gauge fixing is an iteration whose FP64 trajectories differ only by FFT
 rounding, so the transformation counts agree to +-1 and the links to 1e-8;
 the correlators of the same links agree to 1e-10 relative to their maximum.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -164,3 +166,23 @@ def test_group_log_far_from_identity(nrq, oracle, lattice):
         raa, ree = gf.transverse_correlators(lat, U, E)
         assert np.max(np.abs(aa - raa)) < 1e-10 * np.max(np.abs(raa)), trial
         assert np.max(np.abs(ee - ree)) < 1e-12 * np.max(np.abs(ree)), trial
+
+
+def test_gaugefix_returns_with_an_idle_stream(nrq, lattice):
+    """The call returns host values, so its work is done when it returns: with a tolerance
+    that the first look meets, the iteration that is queued ahead is not left running.
+    At this size it takes a quarter of a millisecond, a wait for an idle stream microseconds."""
+    lattice((96, 96, 96), (0.05, 1.0, 1.0, 1.0))
+    _say("gauge fixing leaves no work behind")
+    g = nrq.GaugeConfiguration()
+    g.CoulombGaugefixing(1e3, 0.08, 2)  # transform plans
+    one, left = [], []
+    for _ in range(5):
+        t0 = time.perf_counter()
+        its, _ = g.CoulombGaugefixing(1e3, 0.08, 20)
+        t1 = time.perf_counter()
+        nrq.synchronize()
+        left.append(time.perf_counter() - t1)
+        one.append(t1 - t0 + left[-1])
+        assert its == 0
+    assert min(left) < 0.2 * min(one), (left, one)
