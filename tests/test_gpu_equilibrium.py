@@ -85,3 +85,14 @@ def test_equilibrium_init_refuses_charges_that_are_not_numbers(nrq, lattice, bad
         g.EquilibriumInit(16.0, 1, 2, 1e-2, rho)
     _, dev, nproj = g.EquilibriumInit(16.0, 1, 2, 1e-2)
     assert nproj[0] > 0 and np.all(np.isfinite(dev)) and np.all(np.isfinite(g.download()[1]))
+
+
+def test_equilibrium_init_that_diverges_is_an_error(nrq, lattice):
+    """At a tenth of the usual spatial spacing the projection's step (kappa = 0.01) is unstable,
+    0.01 * 12 / 0.1^2 > 2: E grows until it is not finite, which is no small deviation."""
+    _say("EquilibriumInit that diverges")
+    lattice((4, 4, 4), (0.05, 0.1, 0.1, 0.1))
+    nrq.random_init(5)
+    g = nrq.GaugeConfiguration()
+    with pytest.raises(nrq.NRQError):
+        g.EquilibriumInit(16.0, 1, 0)
