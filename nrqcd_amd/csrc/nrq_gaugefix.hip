@@ -49,6 +49,7 @@ void *gauge_links_mut(nrq_gauge *h);
 
 constexpr double GF_ZERO_TOL = 1e-12; // tolerances.f90
 constexpr int GF_THREADS = 256;
+constexpr double GF_AHEAD = 1.5; // the next iteration is enqueued ahead above this many tolerances
 constexpr int GF_PLANES = 5;    // complex planes of -i Delta
 constexpr int CORR_PLANES = 12; // complex planes of 24 real fields: pair q of direction i in plane q + 4 i
 
@@ -434,32 +435,36 @@ static int gaugefix_t(nrq_gauge *h, double tol, double alpha, int64_t maxit, int
         NRQ_HIP(hipEventRecord(b.ev[n & 1], stream()));
         return NRQ_OK;
     };
-    // transformation n: made by k_gf_apply if the maximum before it asks for
-    // it.  The next one is enqueued before the host looks at this one's
-    // maximum, so the GPU never waits for the host; one transform pair too many
-    // runs at the end.
+    // transformation n, made by k_gf_apply if the maximum before it asks for it, and
+    // the maximum after it
+    auto transform = [&](int64_t n) -> int {
+        hipfftResult fr = hipfftExecZ2Z(plan, (hipfftDoubleComplex *)fld, (hipfftDoubleComplex *)fld, HIPFFT_FORWARD);
+        if (fr != HIPFFT_SUCCESS) return gf_fft_fail(fr, "exec (forward)");
+        hipLaunchKernelGGL(k_gf_accelerate, dim3(nblk), dim3(GF_THREADS), 0, stream(), fld, g, pmax, fwd * bwd * alpha);
+        fr = hipfftExecZ2Z(plan, (hipfftDoubleComplex *)fld, (hipfftDoubleComplex *)fld, HIPFFT_BACKWARD);
+        if (fr != HIPFFT_SUCCESS) return gf_fft_fail(fr, "exec (backward)");
+        hipLaunchKernelGGL(k_gf_apply<R>, dim3(nblk), dim3(GF_THREADS), 0, stream(), u, fld, g, row(n), tol);
+        // n + 1 uses the event and host slot of n - 1, which the host has read
+        return measure(n + 1);
+    };
     if (int e = measure(0)) return e;
-    int64_t enqueued = 0;
+    int64_t enqueued = 0, done = 0;
     double dev = 0;
-    int64_t done = 0;
     for (;; ++done) {
-        while (enqueued < maxit && enqueued <= done) {
-            const int64_t n = enqueued;
-            hipfftResult fr = hipfftExecZ2Z(plan, (hipfftDoubleComplex *)fld, (hipfftDoubleComplex *)fld, HIPFFT_FORWARD);
-            if (fr != HIPFFT_SUCCESS) return gf_fft_fail(fr, "exec (forward)");
-            hipLaunchKernelGGL(k_gf_accelerate, dim3(nblk), dim3(GF_THREADS), 0, stream(), fld, g, pmax, fwd * bwd * alpha);
-            fr = hipfftExecZ2Z(plan, (hipfftDoubleComplex *)fld, (hipfftDoubleComplex *)fld, HIPFFT_BACKWARD);
-            if (fr != HIPFFT_SUCCESS) return gf_fft_fail(fr, "exec (backward)");
-            hipLaunchKernelGGL(k_gf_apply<R>, dim3(nblk), dim3(GF_THREADS), 0, stream(), u, fld, g, row(n), tol);
-            // n + 1 uses the event and host slot of n - 1, which the host has read
-            if (int e = measure(n + 1)) return e;
-            ++enqueued;
+        // Where the last maximum was far above the tolerance the next transformation is
+        // enqueued before the host looks at this one's, so the GPU does not wait for the host.
+        // Near the tolerance, and before the first look, the host looks first (10 us): a
+        // transformation that is then not made costs more (64^3 130 us, 96^3 440 us).
+        if (enqueued == done && done < maxit && dev > GF_AHEAD * tol) {
+            if (int e = transform(enqueued++)) return e;
         }
         NRQ_HIP(hipEventSynchronize(b.ev[done & 1]));
         dev = *(volatile double *)(hmax + (done & 1));
         if (!std::isfinite(dev) || dev <= tol || done >= maxit) break;
+        if (enqueued == done)
+            if (int e = transform(enqueued++)) return e;
     }
-    // host values go back with an idle stream: the pair that ran too many ends here
+    // host values go back with an idle stream: a transformation that was enqueued too many ends here
     NRQ_HIP(hipStreamSynchronize(stream()));
     if (!std::isfinite(dev)) return fail(NRQ_ERR_NOCONV, "gauge fixing: non-finite divergence");
     if (iterations) *iterations = done;

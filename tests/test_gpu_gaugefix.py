@@ -186,3 +186,26 @@ def test_gaugefix_returns_with_an_idle_stream(nrq, lattice):
         one.append(t1 - t0 + left[-1])
         assert its == 0
     assert min(left) < 0.2 * min(one), (left, one)
+
+
+def test_gaugefix_of_fixed_links_is_a_look(nrq, lattice):
+    """On links that meet the tolerance the call measures the divergence and no more:
+    less than half of an iteration's time."""
+    lattice((96, 96, 96), (0.05, 1.0, 1.0, 1.0))
+    _say("gauge fixing of fixed links")
+    g = nrq.GaugeConfiguration()
+    g.upload(None, 0.1 * np.random.default_rng(7).normal(size=(8, 3, 96 ** 3)))
+    g.Update(1.0, 5)
+    look, ten = [], []
+    for _ in range(5):
+        t0 = time.perf_counter()
+        assert g.CoulombGaugefixing(1e3, 0.08, 20)[0] == 0
+        nrq.synchronize()
+        look.append(time.perf_counter() - t0)
+        c = g.copy()
+        nrq.synchronize()
+        t0 = time.perf_counter()
+        assert c.CoulombGaugefixing(0.0, 0.02, 10)[0] == 10
+        nrq.synchronize()
+        ten.append(time.perf_counter() - t0)
+    assert min(look) < 0.5 * min(ten) / 10, (look, ten)
