@@ -68,8 +68,8 @@ TRAFFIC_FILE = ROOT / "profiles" / "leapfrog_fused_128cubed_traffic.txt"
 # one network apply: 2 flop per multiply-add, 27 taps, 18 -> 32 -> 32 -> 32 -> 18 channels, per site
 CNN_FLOP_PER_SITE = 2 * 27 * (18 * 32 + 32 * 32 + 32 * 32 + 32 * 18)
 BF16_MFMA_PEAK_TFLOPS = 2500.0
-TILINGS = ("consecutive sites", "z-sweep tiles of x-rows", "z-sweep 16-wide tiles", "LDS tiles, 16-plane runs",
-           "LDS tiles, 8-plane runs")
+TILINGS = ("consecutive sites", "z-sweep tiles of x-rows", "z-sweep 16-wide tiles",
+           "LDS tiles, 16-plane or 32-plane runs", "LDS tiles, 8-plane runs")
 
 
 def _shape_key(precision: int, shape: dict) -> str:

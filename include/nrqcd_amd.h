@@ -229,8 +229,9 @@ int nrq_gauge_set_reunitarise_interval(nrq_gauge *h, int64_t interval);
  * tiling (0: consecutive sites, 1: z-sweep tiles of full x-rows, 2: z-sweep
  * tiles 16 sites wide, 3 and 4: LDS-staged tiles, 16 x 8 or where there are
  * enough of them 32 x 8, over runs of 16 (or 32) and 8 z planes, FP32 storage
- * only, extents multiples of 16, 8 and 16 or 8), streaming
- * (1: nontemporal loads/stores of E and the
+ * only, extents multiples of 16, 8 and 16 or 8; 384 threads per block say 16 x 8,
+ * 768 say 32 x 8, which a batch may take where one configuration has too few of them),
+ * streaming (1: nontemporal loads/stores of E and the
  * new links) and two_row (1: neighbour links read as two rows, the third
  * rebuilt as the conjugate cross product, exact for SU(3)).  The first
  * leapfrog call per (precision, size) times every shape on scratch copies;

@@ -756,9 +756,9 @@ struct lf_variant {
     int rec; // neighbour links read as two rows (third rebuilt)
 };
 // Modes 3 and 4 are the LDS-tiled fused pass (k_fused_tile, FP32, 16 x 8 or
-// 32 x 8 tiles, runs of 16 (or 32) and 8 z planes); bs is the narrow tile's
-// thread count.  Their first and last half steps use the consecutive-site
-// map.
+// 32 x 8 tiles, runs of 16 (or 32) and 8 z planes: tile_of); bs is the narrow tile's
+// thread count (block_threads is the launch's).  Their first and last half steps use the
+// consecutive-site map.
 static const lf_variant LF_VARIANTS[] = {
     {256, 8, 1, 1, 1}, {128, 8, 1, 1, 1}, {64, 8, 1, 1, 1}, {256, 8, 0, 1, 1}, {128, 8, 0, 1, 1}, {64, 8, 0, 1, 1},
     {256, 8, 2, 1, 1}, {256, 8, 2, 0, 1}, {256, 8, 0, 0, 1}, {64, 8, 0, 0, 1},  {256, 8, 1, 1, 0}, {256, 8, 0, 0, 0},
@@ -818,40 +818,55 @@ static lf_map make_map(int variant, const geom &g)
     return make_lf_map(g, v.bs, v.xcd, v.mode, 3);
 }
 
-template <typename R, int TX, int ZC, bool NTV>
-static void launch_tile_of(const lf_batch<R> &bt, int nb, const geom &g, R dt, int xcd, int reu)
-{
-    constexpr int TY = 8;
-    const unsigned total = (unsigned)(g.n0 / TX) * (unsigned)(g.n1 / TY) * (unsigned)(g.n2 / ZC);
-    hipLaunchKernelGGL((k_fused_tile<R, TX, TY, ZC, NTV>), dim3(total, (unsigned)nb), dim3(TX * TY * 3), 0, stream(), bt,
-                       g, dt, xcd, reu);
-}
+// Tile of a launch of modes 3 and 4: TX x LF_TY sites and runs of ZC planes.
+struct lf_tile {
+    int tx, zc;
+    bool operator==(const lf_tile &o) const { return tx == o.tx && zc == o.zc; }
+};
+constexpr int LF_TY = 8;
 
+// The tile for nb configurations.
 // 32 x 8 tiles where n0 allows them and they give work to more than half of the
 // CUs (one block of a 32 x 8 tile fills a CU, two of 16 x 8): us per step of the
 // fastest 16 x 8 shape and of the 32 x 8 one, and the latter's blocks: 128^3 415
 // and 323 (512), 160x96x96 303 and 242 (720), 96^3 201 and 147 (216),
 // 64x64x128 93 and 83 (256), 64x96x96 148 and 131 (144), 64^3 46 and 59 (128),
 // 96x64x64 with 16-plane runs 83 and 110 (96).
-template <typename R, int ZC, bool NTV>
-static void launch_tile(const lf_batch<R> &bt, int nb, const geom &g, R dt, int xcd, int reu)
-{
-    if (g.n0 % 32 == 0 && (int64_t)(g.n0 / 32) * (g.n1 / 8) * (g.n2 / ZC) * nb > LF_CUS / 2)
-        launch_tile_of<R, 32, ZC, NTV>(bt, nb, g, dt, xcd, reu);
-    else
-        launch_tile_of<R, 16, ZC, NTV>(bt, nb, g, dt, xcd, reu);
-}
-
 // Mode 3: runs of 32 planes (two extra planes are read per run) where 32 x 8 tiles
 // then still give every CU a block, else of 16: 128^3 311 us per step with 32 and
 // 323 with 16, 128x128x64 (128 blocks) 257 and 162.
-template <typename R, bool NTV>
-static void launch_runs(const lf_batch<R> &bt, int nb, const geom &g, R dt, int xcd, int reu)
+static lf_tile tile_of(int mode, const geom &g, int nb)
 {
-    if (g.n0 % 32 == 0 && g.n2 % 32 == 0 && (int64_t)(g.n0 / 32) * (g.n1 / 8) * (g.n2 / 32) * nb >= LF_CUS)
-        launch_tile_of<R, 32, 32, NTV>(bt, nb, g, dt, xcd, reu);
-    else
-        launch_tile<R, 16, NTV>(bt, nb, g, dt, xcd, reu);
+    const int run = mode == 3 ? 16 : 8;
+    const int64_t columns = g.n0 % 32 == 0 ? (int64_t)(g.n0 / 32) * (g.n1 / LF_TY) * nb : 0;
+    if (mode == 3 && g.n2 % 32 == 0 && columns * (g.n2 / 32) >= LF_CUS) return {32, 32};
+    if (columns * (g.n2 / run) > LF_CUS / 2) return {32, run};
+    return {16, run};
+}
+
+template <typename R, int TX, int ZC, bool NTV>
+static void launch_tile_of(const lf_batch<R> &bt, int nb, const geom &g, R dt, int xcd, int reu)
+{
+    const unsigned total = (unsigned)(g.n0 / TX) * (unsigned)(g.n1 / LF_TY) * (unsigned)(g.n2 / ZC);
+    hipLaunchKernelGGL((k_fused_tile<R, TX, LF_TY, ZC, NTV>), dim3(total, (unsigned)nb), dim3(TX * LF_TY * 3), 0, stream(),
+                       bt, g, dt, xcd, reu);
+}
+
+template <typename R, bool NTV>
+static void launch_tile(lf_tile t, const lf_batch<R> &bt, int nb, const geom &g, R dt, int xcd, int reu)
+{
+    if (t == lf_tile{32, 32}) launch_tile_of<R, 32, 32, NTV>(bt, nb, g, dt, xcd, reu);
+    else if (t == lf_tile{32, 16}) launch_tile_of<R, 32, 16, NTV>(bt, nb, g, dt, xcd, reu);
+    else if (t == lf_tile{32, 8}) launch_tile_of<R, 32, 8, NTV>(bt, nb, g, dt, xcd, reu);
+    else if (t == lf_tile{16, 16}) launch_tile_of<R, 16, 16, NTV>(bt, nb, g, dt, xcd, reu);
+    else launch_tile_of<R, 16, 8, NTV>(bt, nb, g, dt, xcd, reu);
+}
+
+// Threads per block of shape `variant` for nb configurations.
+static int block_threads(int variant, const geom &g, int nb)
+{
+    const lf_variant v = LF_VARIANTS[variant];
+    return v.mode >= 3 && variant_ok(variant, g, 32) ? 3 * LF_TY * tile_of(v.mode, g, nb).tx : v.bs;
 }
 
 template <typename R> static void launch_links(int variant, const lf_batch<R> &bt, int nb, const geom &g, R dt)
@@ -882,10 +897,8 @@ static void launch_fused(int variant, const lf_batch<R> &bt, int nb, const geom 
 {
     const lf_variant tv = LF_VARIANTS[variant];
     if constexpr (sizeof(R) == 4) if (tv.mode >= 3) {
-        if (tv.mode == 3)
-            tv.nt ? launch_runs<R, true>(bt, nb, g, dt, tv.xcd, reu) : launch_runs<R, false>(bt, nb, g, dt, tv.xcd, reu);
-        else
-            tv.nt ? launch_tile<R, 8, true>(bt, nb, g, dt, tv.xcd, reu) : launch_tile<R, 8, false>(bt, nb, g, dt, tv.xcd, reu);
+        const lf_tile t = tile_of(tv.mode, g, nb);
+        tv.nt ? launch_tile<R, true>(t, bt, nb, g, dt, tv.xcd, reu) : launch_tile<R, false>(t, bt, nb, g, dt, tv.xcd, reu);
         return;
     }
     const lf_map m = make_map(variant, g);
@@ -1224,7 +1237,7 @@ int leapfrog_choice(const nrq_gauge *h, int *bs, int *xcd, int *mode, int *nt, i
     int v = 0;
     if (int r = h->precision == 64 ? leapfrog_variant<double>(h, 1.0, &v) : leapfrog_variant<float>(h, 1.0f, &v))
         return r;
-    *bs = LF_VARIANTS[v].bs;
+    *bs = block_threads(v, lat().g, 1);
     *xcd = LF_VARIANTS[v].xcd;
     *mode = LF_VARIANTS[v].mode;
     *nt = LF_VARIANTS[v].nt;
@@ -1715,7 +1728,7 @@ extern "C" int nrq_leapfrog_shape_info(int k, int *block_sites, int *xcd_remap, 
     if (k < 0 || k >= LF_NVARIANTS) return fail(NRQ_ERR_ARG, "launch shape %d out of range", k);
     if (!block_sites || !xcd_remap || !tiling || !streaming || !two_row || !applies) return fail(NRQ_ERR_ARG, "null argument");
     const lf_variant &v = LF_VARIANTS[k];
-    *block_sites = v.bs;
+    *block_sites = lat().initialised ? block_threads(k, lat().g, 1) : v.bs;
     *xcd_remap = v.xcd;
     *tiling = v.mode;
     *streaming = v.nt;

@@ -99,3 +99,17 @@ def test_leapfrog_shape_table(nrq, lattice):
     with pytest.raises(nrq.NRQError):
         nrq.leapfrog_set_shape(len(shapes))
     nrq.leapfrog_set_shape(-1)
+
+
+@pytest.mark.parametrize("ext,wide", [((32, 16, 24), ()), ((64, 64, 64), ()), ((128, 128, 128), (3, 4)), ((48, 48, 48), ()),
+                                      ((64, 96, 96), (3, 4)), ((96, 64, 64), (4,))])
+def test_leapfrog_shape_table_tells_the_threads_of_the_launch(nrq, lattice, ext, wide):
+    """The LDS tiles are 32 x 8 (768 threads, three per site) where more than 128 blocks of
+    them cover the lattice with their runs of planes, else 16 x 8 (384)."""
+    lattice(ext, (0.05, 1, 1, 1))
+    tiles = [s for s in nrq.leapfrog_shapes() if s["tiling"].startswith("LDS") and s["applies_fp32"]]
+    assert tiles
+    for s in tiles:
+        mode = 4 if s["tiling"].endswith(" 8-plane runs") else 3
+        assert mode == 4 or ("16-plane" in s["tiling"] and "32-plane" in s["tiling"])
+        assert s["threads_per_block"] == (768 if mode in wide else 384), s
