@@ -892,12 +892,14 @@ template <typename R> static void launch_efield(int variant, const lf_batch<R> &
 }
 
 // reu: project each link onto SU(3) between the E and the link update.
+// tile: for modes 3 and 4 another one than nb asks for (the tuner's check).
 template <typename R>
-static void launch_fused(int variant, const lf_batch<R> &bt, int nb, const geom &g, R dt, int reu = 0)
+static void launch_fused(int variant, const lf_batch<R> &bt, int nb, const geom &g, R dt, int reu = 0,
+                         const lf_tile *tile = nullptr)
 {
     const lf_variant tv = LF_VARIANTS[variant];
     if constexpr (sizeof(R) == 4) if (tv.mode >= 3) {
-        const lf_tile t = tile_of(tv.mode, g, nb);
+        const lf_tile t = tile ? *tile : tile_of(tv.mode, g, nb);
         tv.nt ? launch_tile<R, true>(t, bt, nb, g, dt, tv.xcd, reu) : launch_tile<R, false>(t, bt, nb, g, dt, tv.xcd, reu);
         return;
     }
@@ -961,7 +963,8 @@ template <typename R> static int max_diff(const R *a, const R *b, int64_t n, dou
 // Times every launch shape on scratch copies of the configuration (the
 // handle's own state is not touched) and returns the fastest of those whose
 // one-pass result agrees with LF_DEFAULT's (shape_tolerance); a shape that
-// does not agree is reported on stderr and never chosen.
+// does not agree, with any of the tiles that it takes for up to LF_MAXB
+// configurations, is reported on stderr and never chosen.
 template <typename R> static int tune_leapfrog(const nrq_gauge *h, R dt, int *best)
 {
     const geom g = lat().g;
@@ -997,20 +1000,39 @@ template <typename R> static int tune_leapfrog(const nrq_gauge *h, R dt, int *be
     if (int r = max_diff<R>(ea, eb_, ne, part, &emax)) return release_all(), r;
     const double tol = shape_tolerance<R>();
     std::vector<char> valid(LF_NVARIANTS, 0);
+    const bool verbose = getenv("NRQ_AUTOTUNE_VERBOSE") != nullptr;
     for (int v = 0; v < LF_NVARIANTS; ++v) {
         if (!variant_ok(v, g, (int)(8 * sizeof(R)))) continue;
-        NRQ_HIP(hipMemcpyAsync(eb_, e0, eb, hipMemcpyDeviceToDevice, stream()));
-        launch_fused<R>(v, one<R>(u0, ub, eb_), 1, g, dt);
-        NRQ_HIP(hipGetLastError());
-        double du = 0, de = 0;
-        if (int r = max_diff<R>((const R *)ua, (const R *)ub, nl, part, &du)) return release_all(), r;
-        if (int r = max_diff<R>(ea, eb_, ne, part, &de)) return release_all(), r;
-        valid[v] = du <= tol && de <= tol * std::max(1.0, emax);
-        if (!valid[v])
+        // every kernel that a call with this shape may launch: modes 3 and 4 take their tile by
+        // the number of configurations, and a batch uses the shape chosen here
+        std::vector<lf_tile> tiles = {{0, 0}};
+        if (LF_VARIANTS[v].mode >= 3) {
+            tiles.clear();
+            for (int nb = 1; nb <= LF_MAXB; ++nb) {
+                const lf_tile t = tile_of(LF_VARIANTS[v].mode, g, nb);
+                if (std::find(tiles.begin(), tiles.end(), t) == tiles.end()) tiles.push_back(t);
+            }
+        }
+        valid[v] = 1;
+        for (const lf_tile &t : tiles) {
+            NRQ_HIP(hipMemcpyAsync(eb_, e0, eb, hipMemcpyDeviceToDevice, stream()));
+            launch_fused<R>(v, one<R>(u0, ub, eb_), 1, g, dt, 0, &t);
+            NRQ_HIP(hipGetLastError());
+            double du = 0, de = 0;
+            if (int r = max_diff<R>((const R *)ua, (const R *)ub, nl, part, &du)) return release_all(), r;
+            if (int r = max_diff<R>(ea, eb_, ne, part, &de)) return release_all(), r;
+            const bool agrees = du <= tol && de <= tol * std::max(1.0, emax);
+            if (verbose && t.tx)
+                fprintf(stderr, "nrqcd_amd autotune: shape %d, %d x %d tiles, runs of %d: differs by %.3e (links), %.3e (E)\n", v,
+                        t.tx, LF_TY, t.zc, du, de);
+            if (agrees) continue;
+            valid[v] = 0;
             fprintf(stderr,
                     "nrqcd_amd autotune: launch shape %d rejected: one pass differs from shape %d by %.3e (links), "
                     "%.3e (E)\n",
                     v, LF_DEFAULT, du, de);
+            break;
+        }
     }
     hipEvent_t t0, t1;
     NRQ_HIP(hipEventCreate(&t0));
@@ -1030,7 +1052,7 @@ template <typename R> static int tune_leapfrog(const nrq_gauge *h, R dt, int *be
             float ms = 0;
             NRQ_HIP(hipEventElapsedTime(&ms, t0, t1));
             best_of[v] = std::min(best_of[v], ms);
-            if (getenv("NRQ_AUTOTUNE_VERBOSE"))
+            if (verbose)
                 fprintf(stderr,
                         "nrqcd_amd autotune: precision %d V=%lld shape %d bs=%d xcd=%d tiling=%d streaming=%d two-row=%d: %.2f us/step\n",
                         (int)(8 * sizeof(R)), (long long)g.vol, v, LF_VARIANTS[v].bs, LF_VARIANTS[v].xcd, LF_VARIANTS[v].mode,

@@ -9,6 +9,8 @@ for SU(3) up to rounding), FP32 storage within 2e-5.  Each CN shape
 (fields per thread, tiling, XCD remap) runs one CN step that must match the
 oracle's within 1e-10 (both solve to true relative residual 1e-12).
 """
+import re
+
 import numpy as np
 import pytest
 
@@ -106,6 +108,31 @@ def test_wide_lds_tiles_of_a_batch_match_single_updates(nrq, lattice, pinned, ex
     for k in (0, 1, nb - 2, nb - 1):
         U, E = ens[k].download()
         assert np.array_equal(U, want[k % 2][0]) and np.array_equal(E, want[k % 2][1]), k
+
+
+@pytest.mark.parametrize("ext,want", [
+    # one configuration has 10, 20 and 40 blocks of 32 x 8 tiles with runs of 32, 16 and 8
+    # planes: batches of 26, 7 and 4 reach the tiles' thresholds of 256, 129 and 129
+    ((64, 40, 32), {(16, 16), (32, 16), (32, 32), (16, 8), (32, 8)}),
+    ((48, 24, 16), {(16, 16), (16, 8)}),
+])
+def test_tuner_checks_every_tile_that_a_batch_may_take(nrq, lattice, pinned, monkeypatch, capfd, ext, want):
+    """A batch runs the shape that was tuned on one configuration, and the number of its
+    members decides the LDS tile: the tuner has compared each of those tiles with the
+    default shape before it chooses."""
+    monkeypatch.setenv("NRQ_AUTOTUNE_VERBOSE", "1")
+    _say(f"tiles checked by the tuner on {ext}")
+    nrq.leapfrog_set_shape(-1)
+    lattice(ext, (0.05, 1.0, 1.0, 1.03))
+    g = nrq.GaugeConfiguration(nrq.NRQ_PRECISION_FP32)
+    g.upload(None, 0.1 * np.random.default_rng(5).normal(size=(8, 3, ext[0] * ext[1] * ext[2])))
+    capfd.readouterr()
+    g.Update(1.0, 2)
+    nrq.synchronize()
+    err = capfd.readouterr().err
+    assert "rejected" not in err
+    got = {(int(t), int(z)) for t, z in re.findall(r"(\d+) x 8 tiles, runs of (\d+): differs", err)}
+    assert got == want
 
 
 def test_pinned_shape_that_does_not_apply_is_an_error(nrq, lattice, pinned):
