@@ -386,12 +386,14 @@ constexpr int PC_COLS = 12;
 template <typename T> struct pc_cols {
     const cplx<T> *v[PC_COLS], *f1[PC_COLS], *f2[PC_COLS];
     cplx<T> *z[PC_COLS];
+    const double *unit[PC_COLS]; // 1 / ||v||
     col_scale sc[PC_COLS];
 };
 
 // BF16 network input of colour field blockIdx.y: v (complex colour-major, 3V)
 // and its features f1 = beta K v, f2 = beta K f1; channel 6 q + 2 c + {re, im}
-// of feature q (v, f1 s1, f2 s2) and colour c, channels >= 18 zero.  A lane
+// of feature q (v, f1 s1, f2 s2) and colour c, channels >= 18 zero.  The network sees
+// the unit vector, so that a field of any size stays within FP32's range.  A lane
 // writes its site's 64 bytes as four vectors.
 template <typename T>
 __global__ __launch_bounds__(256) void k_pack(pc_cols<T> col, bf16 *__restrict__ act, int64_t vol)
@@ -400,7 +402,8 @@ __global__ __launch_bounds__(256) void k_pack(pc_cols<T> col, bf16 *__restrict__
     const int k = blockIdx.y;
     if (s >= vol) return;
     const cplx<T> *f[3] = {col.v[k], col.f1[k], col.f2[k]};
-    const cplx<double> m[3] = {{1.0, 0.0}, col.sc[k].s1, col.sc[k].s2};
+    const double unit = *col.unit[k];
+    const cplx<double> m[3] = {{unit, 0.0}, unit * col.sc[k].s1, unit * col.sc[k].s2};
     u16x8 o[4] = {};
 #pragma unroll
     for (int q = 0; q < 3; ++q)
@@ -430,11 +433,13 @@ __global__ __launch_bounds__(256) void k_unpack(const float *__restrict__ o, pc_
     const f32x4 *p = (const f32x4 *)(o + ((int64_t)k * vol + s) * 8);
     const f32x4 lo = p[0], hi = p[1];
     const float n6[6] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1]};
+    const double unit = *col.unit[k];
+    const cplx<double> back = (unit > 0 ? 1.0 / unit : 0.0) * col.sc[k].c;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
         const int64_t at = (int64_t)c * vol + s;
         const cplx<T> a = col.v[k][at], b = col.f1[k][at], d = col.f2[k][at];
-        const cplx<double> n = cmuld({(double)n6[2 * c], (double)n6[2 * c + 1]}, col.sc[k].c);
+        const cplx<double> n = cmuld({(double)n6[2 * c], (double)n6[2 * c + 1]}, back);
         col.z[k][at] = {(T)((a.re - b.re + d.re) + n.re), (T)((a.im - b.im + d.im) + n.im)};
     }
 }
@@ -685,7 +690,7 @@ static int reserve_columns(nrq_cnn *n, const geom &g, int R)
 
 template <typename T>
 int cnn_precondition(nrq_cnn *net, const cplx<T> *const *v, const cplx<T> *const *f1, const cplx<T> *const *f2,
-                     cplx<T> *const *z, int R, const int *act, const cplx<double> *beta)
+                     cplx<T> *const *z, int R, const int *act, const cplx<double> *beta, const double *unit, int64_t stride)
 {
     const geom g = lat().g;
     if (int e = ensure_geom(net, g)) return e;
@@ -700,6 +705,7 @@ int cnn_precondition(nrq_cnn *net, const cplx<T> *const *v, const cplx<T> *const
             col.f1[n] = f1[r];
             col.f2[n] = f2[r];
             col.z[n] = z[r];
+            col.unit[n] = unit + r * stride;
             col.sc[n] = make_col_scale(beta[r], kmax);
             ++n;
         }
@@ -716,10 +722,10 @@ int cnn_precondition(nrq_cnn *net, const cplx<T> *const *v, const cplx<T> *const
 }
 template int cnn_precondition<double>(nrq_cnn *, const cplx<double> *const *, const cplx<double> *const *,
                                       const cplx<double> *const *, cplx<double> *const *, int, const int *,
-                                      const cplx<double> *);
+                                      const cplx<double> *, const double *, int64_t);
 template int cnn_precondition<float>(nrq_cnn *, const cplx<float> *const *, const cplx<float> *const *,
                                      const cplx<float> *const *, cplx<float> *const *, int, const int *,
-                                     const cplx<double> *);
+                                     const cplx<double> *, const double *, int64_t);
 
 } // namespace nrq
 

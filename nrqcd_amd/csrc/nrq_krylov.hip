@@ -1285,7 +1285,7 @@ static int gmres_core(const cplx<RL> *links, int R, const cplx<T> *b, const slot
                     f2p[r] = res + (size_t)r * n;
                     zp[r] = zj + (size_t)r * n;
                 }
-                if (int e = cnn_precondition<T>(net, vp, f1p, f2p, zp, R, cycle.data(), g_beta_host)) return e;
+                if (int e = cnn_precondition<T>(net, vp, f1p, f2p, zp, R, cycle.data(), g_beta_host, gm.sc + j, gm.m + 1)) return e;
                 launch_stencil<RL, T>(links, ws_slots(zj, R), ws_slots(w, R), R, gm.cyc);
                 hipLaunchKernelGGL(k_mdot<T>, dim3(nb, R), dim3(VTHREADS), 0, stream(), W, nv, (const cplx<T> *)w, n, R,
                                    (const int *)gm.cyc, g_ws.cpart);

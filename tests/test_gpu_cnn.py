@@ -367,3 +367,37 @@ def test_network_apply_timer(nrq, lattice):
     assert np.array_equal(net.weights, w)
     with pytest.raises(nrq.NRQError):
         net.time_forward(0)
+
+
+def test_fgmres_does_not_depend_on_the_fields_scale(nrq, lattice):
+    """The network sees unit vectors: fields larger and smaller than FP32 reaches (powers of
+    two, so that every other number of the solve scales exactly) take the same
+    iterations as fields of order one, with the same fallbacks and result."""
+    ext = (16, 8, 8)
+    v = 16 * 8 * 8
+    lattice(ext, (0.05, 1.0, 1.0, 1.0))
+    _say("FGMRES at three scales")
+    rng = np.random.default_rng(3)
+    g = nrq.GaugeConfiguration()
+    g.upload(None, 0.1 * rng.normal(size=(8, 3, v)))
+    g.Update(1.0, 10)
+    Q, A = (rng.normal(size=(6, 6, v)) + 1j * rng.normal(size=(6, 6, v)) for _ in range(2))
+    nrq.nrqcd_init(2.0, C1, 1.0, 1e-10)
+    try:
+        net = nrq.PreconditionerNet(seed=5)
+        net.harvest(g, 1.0, 1, seed=6)
+        net.train(3, 1e-3, seed=1)
+        nrq.nrqcd_set_preconditioner(net)
+        nrq.nrqcd_set_solver(nrq.NRQ_SOLVER_FGMRES_CNN, 20)
+        got = []
+        for scale in (1.0, 2.0 ** 150, 2.0 ** -170):
+            h = nrq.NRQCDField()
+            h.upload(scale * Q, scale * A)
+            before = nrq.cn_fallbacks()
+            st = h.Update(g, 0.5, C1, 8.0)
+            got.append((st.iterations, st.restarts, nrq.cn_fallbacks() - before, h.download()[0] / scale))
+        for its, cycles, falls, q in got[1:]:
+            assert (its, cycles, falls) == got[0][:3]
+            assert _rel(q, got[0][3]) < 1e-12
+    finally:
+        nrq.nrqcd_finalize()
