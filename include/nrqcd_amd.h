@@ -317,10 +317,10 @@ int nrq_cn_set_solver(int kind, int restart, int64_t maxit);
  * their link loads in the CU's L1; 4: wave items over 64-site blocks of
  * band-planes, runs of up to 8 x-rows at one z, ordered by band and z, so
  * that with the XCD remap each XCD sweeps whole bands through z) and the XCD
- * remap (1 or 8).  With tiling 4 and remap 8 lattices and field counts that fill
- * them go through LDS tiles instead (16 x 4 sites, 12 fields per block; the
- * per-thread counts do not apply to those).  Every shape
- * computes the same per-field sums up to rounding.  NRQ_CN_SHAPE=
+ * remap (1 or 8).  With tiling 4 and remap 8 an operator goes through LDS tiles
+ * instead (16 x 4 sites, 12 fields per block; the per-thread counts do not apply to
+ * those) where these are the faster ones for the lattice and the number of fields.  Every
+ * shape computes the same per-field sums up to rounding.  NRQ_CN_SHAPE=
  * "nc64,nc32,tiling,xcd" in the environment sets the initial value (default
  * 2,4,4,8).  No reference counterpart. */
 int nrq_cn_set_shape(int nc64, int nc32, int tiling, int xcd_remap);

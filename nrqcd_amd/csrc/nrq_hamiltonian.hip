@@ -249,7 +249,8 @@ enum ham_mode {
 // group fastest, and each XCD walks one contiguous range of it, so the groups of a
 // site block share its matrices through that XCD's L2.  33x30x27,
 // 12 columns, FP64: 76 us with one column per thread, 46 us with two; three and four
-// (one wavefront per SIMD for their registers) make a whole step 5 and 17 % slower.
+// (one wavefront per SIMD for their registers) make a whole step 5 and 17 % slower.  The
+// residual form, one launch per cycle, spills 20 (FP32 links 28) bytes per thread at 256 VGPRs.
 template <typename R, int MODE>
 __global__ __launch_bounds__(HAM_SITES, 2) void k_ham_apply(const cplx<R> *__restrict__ u, const double *__restrict__ fld,
                                                          const cplx<double> *__restrict__ blk, geom g, ham_cols cols)

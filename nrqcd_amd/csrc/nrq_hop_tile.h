@@ -39,6 +39,7 @@ constexpr int HT_CELLS = HT_HX * (HT_Y + 2);
 constexpr int HT_HALO = 2 * HT_Y + 2 * HT_X; // halo cells of a plane (no corners)
 constexpr int HT_F = 12;                    // fields (wavefronts) per block
 constexpr int HT_THREADS = 64 * HT_F;
+constexpr int NSLOT_GROUPS = 4; // groups of HT_F slots in a batch
 constexpr int HT_CUS = 256; // one block per CU: LDS and the registers of its 12 wavefronts
 // links of a plane that the tile needs: U_x from x - 1, U_y from y - 1, U_z
 constexpr int HT_LX = (HT_X + 1) * HT_Y, HT_LY = HT_X * (HT_Y + 1), HT_LZ = HT_X * HT_Y;
@@ -391,34 +392,40 @@ inline hop_tiles hop_tiles_for(const geom &g, int nf)
 
 inline unsigned hop_grid(const hop_tiles &t) { return (unsigned)t.ntx * (unsigned)t.nty * (unsigned)t.nzr * (unsigned)t.groups; }
 
-// What a kernel computes: the wave items that cost as much as one z plane of a
-// tile on every CU, from the fit below.
-enum hop_op { HOP_FP32 = 667, HOP_FP64 = 1250, HOP_FP64_CHEB = 1350 };
+enum hop_op { HOP_FP64, HOP_FP64_CHEB, HOP_FP32 }; // what a kernel computes
 
 // Whether the tiles of lattice g are faster than the wave items of nrq_map.h for nf slots.
 // The time of the tiles goes with the planes of a run times the rounds of blocks, one block per CU (half way
 // between whole rounds and their exact number fits best); that of the wave items with their
 // number, whatever part of their lanes is used, so that bands that fill 64 lanes badly favour
-// the tiles and tiles that reach past the lattice the wave items.  Above two groups (more than 24
-// slots) FP64 wave items gain on the tiles, as their chunks share more link lines.
-// Fitted to each operator taken alone both ways in CN steps of four solvers on 230 lattices of 10 to 112
-// a side, 12, 24 and 48 slots, both storages: against wave items everywhere steps are 1.11 times as
-// fast in the mean and no less than 0.95 times.  us per step, wave items / tiles, 12 slots:
+// the tiles and tiles that reach past the lattice the wave items.  plane_items are the wave items
+// that cost as much as one plane of a tile on every CU: by operator, by rows that start on cache
+// lines (n0 a multiple of 16) or do not, and by groups.  A block of wave items holds 16 slots in
+// FP64 and 32 in FP32, so 24 and 36 slots leave part of it idle, and 48 fill it in FP64 only.
+// Fitted to each operator taken alone both ways in CN steps of four solvers on 341 lattices of 10 to 112
+// a side, 12, 24, 36 and 48 slots, both storages: against wave items everywhere steps are 1.12 times as
+// fast in the mean and no less than 0.94 times.  us per step, wave items / tiles, 12 slots:
 // FP64 Chebyshev 64^3 1497 / 1142, 90x62x58 2112 / 2099, 33x30x27 401 / 335, 32^3 238 / 271, 48x25x17
 // 212 / 308; mixed Chebyshev 64^3 1001 / 759, 48^3 462 / 383, 8x81x27 437 / 210, 32^3 185 / 190,
-// 90x62x58 1379 / 1459; GMRES 64^3 2071 / 1689, 40^3 613 / 646, 30x34x22 397 / 393; with 48 slots
-// mixed Chebyshev 48^3 2212 / 1731, FP64 Chebyshev 28^3 596 / 633.
+// 90x62x58 1379 / 1459; GMRES 64^3 2071 / 1689, 40^3 613 / 646, 30x34x22 397 / 393.  With 48 slots
+// mixed Chebyshev 48^3 2212 / 1731; FP64 Chebyshev 28^3 596 / 633, 48^3 2615 / 2489 and 48x25x17
+// 610 / 663 (FP32 links), the line being between the last two.
 // A group with idle wavefronts costs as much as a full one: tiles for at least 4/5 full
 // groups (64^3 with 2 slots, mixed Chebyshev: 311 / 401).
 inline bool hop_tiles_pay(const geom &g, const hop_tiles &t, int nf, hop_op op)
 {
-    if (5 * nf < 4 * HT_F * t.groups) return false;
+    static const double plane_items[3][2][NSLOT_GROUPS] = {
+        {{1175, 1250, 1150, 1370}, {1250, 1165, 1400, 1650}}, // FP64
+        {{1175, 1175, 1150, 1370}, {1360, 1175, 1375, 1650}}, // FP64 Chebyshev step
+        {{675, 625, 350, 350}, {675, 550, 500, 500}},         // FP32
+    };
+    if (5 * nf < 4 * HT_F * t.groups || t.groups > NSLOT_GROUPS) return false;
     const int nc = op == HOP_FP32 ? 4 : 2; // fields per thread of the default wave items
     const lf_map mp = make_lf_map(g, 64, 8, 4, 1);
-    double items = (double)mp.nsb * ((nf + nc - 1) / nc);
-    if (op != HOP_FP32 && t.groups > 2) items *= 0.85;
+    const double items = (double)mp.nsb * ((nf + nc - 1) / nc);
     const double blocks = (double)hop_grid(t) / HT_CUS;
-    return items > 0.5 * (std::ceil(blocks) + blocks) * (t.zc - 0.5) * (double)op;
+    const double per_plane = plane_items[op][g.n0 % HT_X != 0][t.groups - 1];
+    return items > 0.5 * (std::ceil(blocks) + blocks) * (t.zc - 0.5) * per_plane;
 }
 
 } // namespace nrq

@@ -608,7 +608,8 @@ template <typename T, typename TR, bool WRITE_RES> struct tile_resid {
     __device__ __forceinline__ void sum(int r, unsigned i, double v) const { partial[(int64_t)r * nsb + i] = v; }
 };
 
-// k_cheb; FIN: with the FP64 iterate (fin)
+// k_cheb; FIN: with the FP64 iterate (fin, FP32 corrections only).  In FP64 it compiles to
+// 168 VGPRs and 24 B of scratch per thread (k_cheb: 20 B at 128 VGPRs), which its times include.
 template <typename T, bool FIN> struct tile_cheb {
     static constexpr bool NORM = false;
     struct pre {
@@ -908,8 +909,9 @@ static int upload_active(const std::vector<int> &act)
 // Launch shape of the stencil kernels: slots per thread (NC, sharing each
 // link load) for FP64 and for FP32 arithmetic, and the site-block mapping of
 // make_lf_map.  NRQ_CN_SHAPE="nc64,nc32,mode,xcd" in the environment sets
-// the initial value, nrq_cn_set_shape changes it.  Every shape computes the
-// same sums in the same order per slot.
+// the initial value, nrq_cn_set_shape changes it.  The results of the shapes agree
+// up to rounding: partial sums follow the site blocks (and the LDS tiles of the default
+// shape), and the tiled Chebyshev step is an algebraically equal update (tile_cheb).
 struct cn_shape {
     // measured fastest at 128^3 with 12 fields: one work item per wavefront,
     // y-band z-sweep order, each XCD walking whole bands
@@ -952,6 +954,7 @@ static bool use_tiles(int nf, hop_op op, hop_tiles *t)
     *t = hop_tiles_for(lat().g, nf);
     return hop_tiles_pay(lat().g, *t, nf, op);
 }
+static_assert(NSLOT_GROUPS * HT_F == NSLOTS, "hop_tiles_pay has a column for every batch");
 template <typename T> constexpr hop_op op_of() { return sizeof(T) == 8 ? HOP_FP64 : HOP_FP32; }
 static dim3 tile_grid(const hop_tiles &t) { return dim3(hop_grid(t)); }
 
@@ -1637,7 +1640,7 @@ static int gmres_mixed(const cplx<RL> *u, int R, std::vector<double> &bn, const 
         }
         if (!any) break;
         ++cycles;
-        // ||r||^2 of this refinement step at nrm[64..): the inner solve reuses nrm[0..R)
+        // ||r||^2 of this refinement step at nrm[NRM_SAVED ..): the inner solve reuses nrm[0, R)
         double *rnorm2 = g_ws.nrm + workspace::NRM_SAVED;
         NRQ_HIP(hipMemcpyAsync(rnorm2, g_ws.nrm, sizeof(double) * R, hipMemcpyDeviceToDevice, stream()));
         // normalised FP32 correction problem A d = r / ||r||
@@ -1681,7 +1684,7 @@ static int cn_step_t(const cplx<RL> *u, int R, const std::vector<zc> &alpha, con
     int64_t cycles = 0;
     std::vector<int> act(R, 1);
     const bool guess = p.extrapolate && p.kind != KRYLOV_GMRES_FP64;
-    // right-hand sides and guesses; ||y||^2 to nrm[32..)
+    // right-hand sides and guesses; ||y||^2 to nrm[NRM_Y ..)
     const slots<double> tpsi = psi_slots(R), ty = ws_slots(g_ws.y, R), tx = ws_slots(g_ws.x, R);
     // mixed Chebyshev from the guess takes K psi (FP32) for its first correction
     const int wk = guess && p.kind == KRYLOV_CHEB_MIXED ? 1 : 0;
