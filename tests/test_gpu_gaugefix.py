@@ -171,8 +171,8 @@ def test_group_log_far_from_identity(nrq, oracle, lattice):
 def test_gaugefix_returns_with_an_idle_stream(nrq, lattice):
     """The call returns host values, so its work is done when it returns: with a tolerance
     that the first look meets, the iteration that is queued ahead is not left running.
-    At this size it takes a quarter of a millisecond, a wait for an idle stream microseconds."""
-    lattice((96, 96, 96), (0.05, 1.0, 1.0, 1.0))
+    At this size it takes 1.7 ms, a wait for an idle stream microseconds."""
+    lattice((160, 160, 160), (0.05, 1.0, 1.0, 1.0))
     _say("gauge fixing leaves no work behind")
     g = nrq.GaugeConfiguration()
     g.CoulombGaugefixing(1e3, 0.08, 2)  # transform plans
@@ -190,11 +190,12 @@ def test_gaugefix_returns_with_an_idle_stream(nrq, lattice):
 
 def test_gaugefix_of_fixed_links_is_a_look(nrq, lattice):
     """On links that meet the tolerance the call measures the divergence and no more:
-    less than half of an iteration's time."""
-    lattice((96, 96, 96), (0.05, 1.0, 1.0, 1.0))
+    less than half of an iteration's time (0.5 ms and 2.5 ms at this size, so that a slow wait of
+    the host, 0.1 ms, does not count)."""
+    lattice((160, 160, 160), (0.05, 1.0, 1.0, 1.0))
     _say("gauge fixing of fixed links")
     g = nrq.GaugeConfiguration()
-    g.upload(None, 0.1 * np.random.default_rng(7).normal(size=(8, 3, 96 ** 3)))
+    g.upload(None, 0.1 * np.random.default_rng(7).normal(size=(8, 3, 160 ** 3)))
     g.Update(1.0, 5)
     look, ten = [], []
     for _ in range(5):
